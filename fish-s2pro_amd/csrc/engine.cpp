@@ -52,7 +52,7 @@ constexpr uint32_t PREFILL_COLS = 4;     // decode-path columns per pass of the 
 constexpr uint32_t MAX_SEQS = 16;        // requests per batched generate call
 constexpr uint32_t BMM_MAX_K = 10240;    // input width limit of the batched product
 constexpr uint32_t ACT_COLS = 2 * MAX_SEQS;  // activation columns (Fast-AR pass 0 has two per request)
-constexpr uint32_t PREFILL_CHUNK = 512;  // prompt tokens per MFMA prefill pass
+constexpr uint32_t PREFILL_CHUNK = 2048;  // most prompt tokens per MFMA prefill pass
 constexpr uint32_t FRAME_BATCH = 4;
 constexpr uint32_t ATTN_CHECK_MIN_SEQS = 2;  // batched requests: tail attention chunks check first
 constexpr size_t WEIGHT_PAD = 256;  // trailing bytes so block loads never leave a buffer
@@ -300,6 +300,7 @@ class Engine {
   _Float16 *pxh_ = nullptr, *pxl_ = nullptr;
   float* ppart_ = nullptr;  // K-split partial sums of the prefill products
   size_t ppart_cap_ = 0;
+  uint32_t prefill_chunk_ = 0;  // prompt tokens per prefill pass
   float *fh_ = nullptr, *fqkv_ = nullptr, *fq_ = nullptr, *fatt_ = nullptr, *fpart_ = nullptr, *fact_ = nullptr;
   float *flogits_ = nullptr, *fkc_ = nullptr, *fvc_ = nullptr;
   uint32_t fctx_ = 11;
@@ -504,8 +505,9 @@ Engine::Engine(const s2hip_config& cfg) {
   HIPC(hipMemset(counters_, 0, size_t(ACT_COLS) * std::max(s.kv_heads, s.fast_kv_heads) * 4));
   act_ = dalloc<float>(size_t(NC) * s.ffn);
   {
-    const size_t CH = PREFILL_CHUNK, CHP = gemm_rows_pad(PREFILL_CHUNK);
-    const size_t kmax = std::max<size_t>({s.dim, q, s.ffn});
+    prefill_chunk_ = std::min(PREFILL_CHUNK, s.max_seq_len);
+    const size_t CH = prefill_chunk_, CHP = gemm_rows_pad(prefill_chunk_);
+    const size_t kmax = std::max<size_t>({s.dim, q, s.ffn, s.fast_ffn, size_t(s.fast_heads) * s.fast_head_dim});
     ph_ = dalloc<float>(CH * s.dim);
     pqkv_ = dalloc<float>(CH * qkv_w);
     pq_ = dalloc<float>(CH * q);
@@ -1060,7 +1062,7 @@ void Engine::enqueue_frame(const SamplerCfg& cfg, uint32_t nseq, size_t codes_st
 }
 
 // Prompt prefill (forward_slow_ar_block_prefill_layers_cached, slow_ar.rs:1002-1039):
-// chunks of up to PREFILL_CHUNK tokens go through each layer together: every
+// chunks of up to prefill_chunk_ tokens go through each layer together: every
 // linear is one MFMA product over the chunk (weights read once per chunk),
 // QK-norm + RoPE + KV append for all of the chunk's positions, then causal
 // attention of each token over the cache.  One slot (`seq`) at a time;
@@ -1071,6 +1073,10 @@ void Engine::mm(const DevLin& L, const DevLin* L3, int epi, const float* x, uint
   GemmArgs g{};
   g.w = L.w;
   g.w3 = L3 ? L3->w : nullptr;
+  if (L.wt && (!L3 || L3->wt)) {
+    g.wt = L.wt;
+    g.wt3 = L3 ? L3->wt : nullptr;
+  }
   g.row_bytes = L.row_bytes;
   g.M = L.out;
   g.K = L.in;
@@ -1151,7 +1157,7 @@ void Engine::enqueue_prefill(const int32_t* prompt_dev, size_t n_tok, uint32_t s
   size_t t = 0;
   uint32_t nc = 0;
   while (t < n_tok) {
-    nc = uint32_t(std::min<size_t>(PREFILL_CHUNK, n_tok - t));
+    nc = uint32_t(std::min<size_t>(prefill_chunk_, n_tok - t));
     const uint32_t npad = gemm_rows_pad(nc);
     EmbedArgs ea{};
     ea.tokens = prompt_dev + t * cdim;
@@ -1364,6 +1370,7 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
          " max_seq_len=" + std::to_string(s.max_seq_len));
   validate_tokens(flat, n_tok);
   ensure_slots(slot + 1);
+  ensure_tiled();
   ensure_prompt(n_tok * cdim);
   HIPC(hipMemcpyAsync(prompt_dev_, flat, n_tok * cdim * 4, hipMemcpyHostToDevice, stream_));
   // done = 0, err = 0 (eval never runs under a finished frame loop)

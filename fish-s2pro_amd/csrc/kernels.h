@@ -291,8 +291,8 @@ hipError_t launch_add_position(DevState* st, uint32_t n, uint32_t n_seq, hipStre
 hipError_t launch_copy(const void* src, void* dst, size_t bytes, hipStream_t s);
 
 // ---- prompt prefill (prefill.hip) ----
-// Activation rows -> f16 hi / lo planes [Npad][K] and a power-of-two row
-// scale rs[Npad] (optionally RMSNorm first); rows N..Npad-1 are zero.
+// Activation rows -> f16 hi / lo planes of Npad x K elements (tiles of 16 rows
+// x 32 k, see plane_off) and a power-of-two row scale rs[Npad] (optionally RMSNorm first); rows N..Npad-1 are zero.
 // Npad >= N, a multiple of 16 (gemm_rows_pad(N) for launch_gemm_mfma, 16 for
 // launch_skinny_mfma); K must be a multiple of 32.
 uint32_t gemm_rows_pad(uint32_t n);
@@ -303,10 +303,14 @@ hipError_t launch_split_rows(const float* x, uint32_t ldx, const float* norm, fl
 // MFMA product y[n][m] (op)= rs[n] * sum_k W[m][k] * x[n][k] for n < N, m < M,
 // x given as the split planes; epilogues as for launch_gemv (SwiGLU uses w3).
 // part (nullable): workspace of part_cap floats for K-split partial sums
-// (gemm_part_floats(Npad, M) floats lets every short-M product split).
+// (gemm_part_floats(Npad, M) floats lets every short-M product split as it would).
+// F16 weights: wt (and wt3) in the fragment order of launch_tile_f16, or null
+// and the rows themselves.
 struct GemmArgs {
   const uint8_t* w;
   const uint8_t* w3;
+  const _Float16* wt;
+  const _Float16* wt3;
   size_t row_bytes;
   uint32_t M, K;
   const _Float16* xh;

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "expf_glibc.h"
@@ -34,6 +35,29 @@ __device__ __forceinline__ float half_bits_to_float_p(uint16_t b) {
   return static_cast<float>(__builtin_bit_cast(_Float16, b));
 }
 __device__ __forceinline__ float wave_max_f(float v) { return wave_max(v); }
+
+constexpr int TM = 128, TN = 128, KS = 32;
+
+// Tile rows are KS halfs (four 16-byte chunks) with no padding; chunk j of
+// row r sits at chunk position j ^ swz(r).  Both access patterns to such a
+// tile in LDS then hit distinct banks with 32 or 64 banks of 4 bytes: the
+// staging stores (4 lanes per row, consecutive rows) and the fragment reads
+// (one row per lane, 32 consecutive rows, one chunk).
+__device__ __forceinline__ uint32_t swz(uint32_t r) { return ((r >> 1) ^ (r >> 3)) & 3u; }
+__device__ __forceinline__ uint32_t tile_off(uint32_t r, uint32_t k) {  // k: a multiple of 8
+  return r * KS + (((k >> 3) ^ swz(r)) << 3);
+}
+
+// Layout of the split activation planes ([Npad][K] elements): 16 rows x 32 k
+// are one contiguous KiB whose rows are laid out as tile_off, so a wave load
+// is one contiguous KiB and lands in LDS as the fragment reads want it.  With
+// row-major planes a wave load touches 64 bytes of each of 16 rows, half a
+// cache line each, and the products were bound by that: w1/w3 of 256 tokens
+// took 98-107 us at every tile and pipeline depth.  Offset in halfs of the 8
+// elements from k (a multiple of 8) of row n:
+__device__ __forceinline__ size_t plane_off(uint32_t n, uint32_t k, uint32_t K) {
+  return (size_t(n >> 4) * (K / KS) + (k / KS)) * (16 * KS) + (n & 15u) * KS + ((((k >> 3) & 3u) ^ swz(n)) << 3);
+}
 
 // ---------------------------------------------------------------------------
 // Activation split: one block per row n < Npad.
@@ -81,12 +105,10 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* x, uint32_
                                                          float* rs, uint32_t* err) {
   __shared__ float red[4];
   const uint32_t n = blockIdx.x, tid = threadIdx.x;
-  _Float16* hr = xh + size_t(n) * K;
-  _Float16* lr = xl + size_t(n) * K;
   if (n >= N) {
-    for (uint32_t i = tid; i < K; i += 256) {
-      hr[i] = _Float16(0.0f);
-      lr[i] = _Float16(0.0f);
+    for (uint32_t k = tid * 8u; k < K; k += 2048u) {
+      *reinterpret_cast<uint4*>(xh + plane_off(n, k, K)) = make_uint4(0u, 0u, 0u, 0u);
+      *reinterpret_cast<uint4*>(xl + plane_off(n, k, K)) = make_uint4(0u, 0u, 0u, 0u);
     }
     if (tid == 0) rs[n] = 1.0f;
     return;
@@ -138,8 +160,9 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* x, uint32_
         h[c] = _Float16(e[c]);
         l[c] = _Float16(e[c] - float(h[c]));
       }
-      *reinterpret_cast<uint2*>(hr + 4 * j) = *reinterpret_cast<const uint2*>(h);
-      *reinterpret_cast<uint2*>(lr + 4 * j) = *reinterpret_cast<const uint2*>(l);
+      const size_t o = plane_off(n, 4 * j, K) + (j & 1u) * 4u;
+      *reinterpret_cast<uint2*>(xh + o) = *reinterpret_cast<const uint2*>(h);
+      *reinterpret_cast<uint2*>(xl + o) = *reinterpret_cast<const uint2*>(l);
     }
     if (tid == 0) rs[n] = r;
     return;
@@ -167,8 +190,9 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* x, uint32_
     if (norm) v = __fmul_rn(__fmul_rn(v, scale), norm[i]);
     v *= inv;
     const _Float16 h = _Float16(v);
-    hr[i] = h;
-    lr[i] = _Float16(v - float(h));
+    const size_t o = plane_off(n, i, K) + (i & 7u);
+    xh[o] = h;
+    xl[o] = _Float16(v - float(h));
   }
   if (tid == 0) rs[n] = r;
 }
@@ -225,18 +249,7 @@ __device__ __forceinline__ void weight8(const uint8_t* row, uint32_t e, half8& h
 //   to part[split][n][m]; gemm_split_reduce_kernel adds the splits in order
 //   and applies rs and the epilogue.
 // ---------------------------------------------------------------------------
-constexpr int TM = 128, TN = 128, KS = 32;
-
-// LDS tile rows are KS halfs (four 16-byte chunks) with no padding; chunk j of
-// row r sits at chunk position j ^ swz(r).  Both access patterns then hit
-// distinct banks with 32 or 64 banks of 4 bytes: the staging stores (4 lanes
-// per row, consecutive rows) and the fragment reads (one row per lane, 32
-// consecutive rows, one chunk).
-__device__ __forceinline__ uint32_t swz(uint32_t r) { return ((r >> 1) ^ (r >> 3)) & 3u; }
-__device__ __forceinline__ uint32_t tile_off(uint32_t r, uint32_t k) {  // k: a multiple of 8
-  return r * KS + (((k >> 3) ^ swz(r)) << 3);
-}
-constexpr uint32_t GEMM_MAX_SPLITS = 4;
+constexpr uint32_t GEMM_MAX_SPLITS = 8;
 
 // Epilogue of the MFMA GEMM: acc[tn][tm][v] = D[token 8 (v/4) + 4 (lane/32) +
 // v%4][weight slot lane%32] of the wave's 2 x 2 tiles.
@@ -330,7 +343,7 @@ __global__ __launch_bounds__(256, 3) void gemm_mfma_kernel(GemmArgs a, uint32_t 
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const uint32_t c = tid + 256u * j;
-    xrow[j] = ((c >> 9) ? a.xl : a.xh) + size_t(n_base + ((c >> 2) & 127u)) * a.K + part8;
+    xrow[j] = ((c >> 9) ? a.xl : a.xh) + plane_off(n_base + ((c >> 2) & 127u), part8, a.K);
   }
 
   // a ring of D register sets: the loads of stage st + D go out while stage
@@ -345,7 +358,7 @@ __global__ __launch_bounds__(256, 3) void gemm_mfma_kernel(GemmArgs a, uint32_t 
       if constexpr (WSPLIT) rw[r][j][WP - 1] = lo;
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) rx[r][j] = *reinterpret_cast<const half8*>(xrow[j] + k0);
+    for (int j = 0; j < 4; ++j) rx[r][j] = *reinterpret_cast<const half8*>(xrow[j] + k0 * 16u);
   };
   auto store_stage = [&](int r, uint32_t buf) {
 #pragma unroll
@@ -423,178 +436,204 @@ __global__ __launch_bounds__(256, 3) void gemm_mfma_kernel(GemmArgs a, uint32_t 
   gemm_epilogue<WT, EPI>(a, acc, accl, mt, n_base, sp, splits, wm, wn, lane);
 }
 
-// F16 weights: the same tiles, staged by LDS-DMA loads (global_load_lds_dwordx4:
-// a wave's 64 lanes fill 1 KiB of LDS, lane i at byte 16 i of the wave's
-// destination), so staging takes no registers and no LDS store instructions.
-// A wave's 1 KiB is 16 consecutive tile rows of 64 bytes; lane i takes row
-// i / 4 and physical chunk i % 4 and loads the logical chunk (i % 4) ^ swz(row),
-// which puts the tile in the swizzled layout of tile_off.  Three LDS stages
-// rotate: while stage st computes, stage st + 1 is in flight and stage st + 2
-// is issued into the buffer that stage st - 1 has left.
-constexpr uint32_t GEMM_DMA_PER_STAGE = 6;  // 16-byte loads per thread per stage (4 token + 2 weight)
-
+// ---------------------------------------------------------------------------
+// F16 weights: block tile 64 TMW weight rows x 64 TNW tokens, 4 waves in 2 x 2,
+// each 32 TMW rows x 32 TNW tokens (a 128 x 64 wave reads 8 KiB of fragments
+// from LDS per 16 MFMAs; a 64 x 64 wave 6 KiB per 8, which leaves the LDS
+// port, not the matrix cores, as the bound).
+// Weights come from the fragment-ordered copy (tiles of 16 rows x 32 k, one
+// contiguous KiB each), tokens from the split planes (plane_off).
+// Staged by LDS-DMA loads (global_load_lds_dwordx4: a wave's 64 lanes fill
+// 1 KiB of LDS, lane i at byte 16 i of the wave's destination), so staging
+// takes no registers and no LDS store instructions.
+// Each stage (32 k) is computed in two halves of 16 k with the fragments of
+// the next half read from LDS while the current half's MFMAs run.  The barrier
+// sits between the halves: by then the wave has read all of stage st and its
+// own loads of stage st + 1 have landed, so past it stage st + 1 may be read
+// and the buffer of stage st takes the loads of stage st + NB.
+// ---------------------------------------------------------------------------
 constexpr bool DUAL_EPI(int epi) { return epi == EPI_SWIGLU_SLOW || epi == EPI_SWIGLU_FAST; }
 
-// One LDS-DMA load: 16 bytes per lane from `src` into the wave's 1 KiB at
-// `lds` (lane i at byte 16 i).  Written as inline assembly so that the
-// compiler does not treat every later LDS read as dependent on it (it would
-// wait for all loads in flight first); the kernel waits for these loads
-// itself (vmcnt) before the barrier that publishes a stage.
-__device__ __forceinline__ void dma16(const void* src, const _Float16* lds) {
-  const uint32_t m0 = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(reinterpret_cast<uintptr_t>(lds)))));
-  asm volatile("s_nop 1\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(m0), "v"(src)
+// One LDS-DMA load: 16 bytes per lane from `base` (wave-uniform) + `off` into
+// the wave's 1 KiB at LDS byte `lds` (lane i at byte 16 i).  Written as inline
+// assembly so that the compiler does not treat every later LDS read as
+// dependent on it (it would wait for all loads in flight first); the kernel
+// waits for these loads itself (vmcnt) before the barrier that publishes a
+// stage.
+__device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_nop 1\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds), "v"(off), "s"(base)
                : "memory", "m0");
 }
 
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef const __attribute__((address_space(1))) void glob_void_t;
+// s_waitcnt immediate: at most `v` vector memory loads in flight, LDS reads
+// drained if `lgkm0`
+constexpr int wait_imm(int v, bool lgkm0) { return (v & 15) | ((v >> 4) << 14) | 0x70 | (lgkm0 ? 0 : 0xF00); }
 
-template <int B>
-struct StageTag {
-  static constexpr int value = B;
-};
-
-template <int EPI>
+template <int EPI, int TMW, int TNW, int NB>
 __global__ __launch_bounds__(256, 2) void gemm_f16_dma_kernel(GemmArgs a, uint32_t m_tiles, uint32_t n_tiles,
                                                               uint32_t splits) {
-  // one LDS object per stage buffer, always addressed with a compile-time
-  // stage index: the compiler then knows which buffer a DMA writes and a
-  // fragment read reads, and waits only where they meet
-  __shared__ _Float16 xs0[2 * TN * KS], xs1[2 * TN * KS], xs2[2 * TN * KS];
-  __shared__ _Float16 ws0[TM * KS], ws1[TM * KS], ws2[TM * KS];
-  auto xbuf = [&](auto tag) -> _Float16* {
-    if constexpr (decltype(tag)::value == 0) return xs0;
-    else if constexpr (decltype(tag)::value == 1) return xs1;
-    else return xs2;
-  };
-  auto wbuf = [&](auto tag) -> _Float16* {
-    if constexpr (decltype(tag)::value == 0) return ws0;
-    else if constexpr (decltype(tag)::value == 1) return ws1;
-    else return ws2;
-  };
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  constexpr bool DUAL = DUAL_EPI(EPI);
+  constexpr uint32_t WR = 64 * TMW, XR = 64 * TNW;            // tile rows
+  constexpr uint32_t STAGE = (WR + 2 * XR) * KS * 2;          // bytes: weights, then the hi and lo token planes
+  constexpr int PER = TMW + 2 * TNW;                          // 1 KiB loads per wave and stage
+  extern __shared__ __align__(16) uint8_t gemm_lds[];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
   const uint32_t wm = wave & 1u, wn = wave >> 1;
-  const uint32_t L = blockIdx.x, inner = n_tiles * splits;
-  const uint32_t sidx = L >> 3, mt = (sidx / inner) * 8u + (L & 7u);
-  if (mt >= m_tiles) return;
-  const uint32_t rr = sidx % inner, nt = rr % n_tiles, sp = rr / n_tiles;
-  const uint32_t n_base = nt * TN;
+  // Workgroup b runs on XCD b % 8; tiles go to the XCDs in contiguous ranges
+  // of t = (m tile, split, n tile), n fastest, so the blocks that read one m
+  // tile's weight rows share an L2.
+  const uint32_t nb = gridDim.x, xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7u;
+  const uint32_t t = xcd < r8 ? xcd * (q8 + 1u) + slot : r8 * (q8 + 1u) + (xcd - r8) * q8 + slot;
+  const uint32_t nt = uint32_t(__builtin_amdgcn_readfirstlane(int(t % n_tiles))), tr = t / n_tiles;
+  const uint32_t sp = uint32_t(__builtin_amdgcn_readfirstlane(int(tr % splits)));
+  const uint32_t mt = uint32_t(__builtin_amdgcn_readfirstlane(int(tr / splits)));
+  const uint32_t n_base = nt * XR, m_base = mt * (DUAL ? WR / 2 : WR);
   const uint32_t nst = a.K / KS, st0 = sp * nst / splits, st1 = (sp + 1) * nst / splits;
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(gemm_lds));
 
-  // this lane's rows and logical chunks: token chunk c = tid + 256 j (j < 4):
-  // plane c / 512, row (c / 4) % 128; weight chunk c = tid + 256 j (j < 2):
-  // slot c / 4.  The LDS destination of the wave's load j is the 1 KiB at the
-  // tile row of its lane 0.
-  // Source addresses are a wave-uniform base (scalar registers, advanced by
-  // the stage's k offset) plus a loop-invariant 32-bit lane offset, so the
-  // loads take the scalar-base form and no address register is rebuilt.
-  const uint32_t pc = lane & 3u;  // physical chunk
-  const uint8_t* xbase[4];
-  uint32_t xoff[4], xdst[4];
+  // This wave's loads of a stage, each one contiguous KiB: weight tiles TMW
+  // wave + j of 16 rows, token tiles g of plane p with 2 TNW wave + j =
+  // 4 TNW p + g.
+  const uint32_t kt = a.K / KS, wt_last = (a.M + 15u) / 16u - 1u, off = lane * 16u;
+  const uint8_t* src[PER];
+  uint32_t dst[PER];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t c = tid + 256u * j, plane = c >> 9, row = (c >> 2) & 127u;
-    xbase[j] = reinterpret_cast<const uint8_t*>((plane ? a.xl : a.xh) + size_t(n_base) * a.K);
-    xoff[j] = (row * a.K + ((pc ^ swz(row)) << 3)) * 2u;
-    xdst[j] = plane * (TN * KS) + (((c & ~63u) >> 2) & 127u) * KS;  // halfs, wave-uniform
+  for (int j = 0; j < TMW; ++j) {
+    const uint32_t g = TMW * wave + j;
+    // SwiGLU: w1 and w3 rows alternate every 32 slots
+    const uint32_t tile = m_base / 16u + (DUAL ? (g >> 2) * 2u + (g & 1u) : g);
+    const _Float16* base = (DUAL && ((g >> 1) & 1u)) ? a.wt3 : a.wt;
+    src[j] = reinterpret_cast<const uint8_t*>(base) + size_t(min(tile, wt_last)) * kt * 1024u;
+    dst[j] = lds0 + g * 1024u;
   }
-  const uint8_t* wbase[2];
-  uint32_t woff[2], wdst[2];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const uint32_t c = tid + 256u * j, slot = c >> 2;
-    uint32_t row;
-    const uint8_t* base = a.w;
-    if constexpr (DUAL_EPI(EPI)) {
-      const uint32_t grp = slot >> 5;  // w1 / w3 alternate every 32 slots: uniform over a wave
-      row = mt * 64u + (grp >> 1) * 32u + (slot & 31u);
-      base = (grp & 1u) ? a.w3 : a.w;
-      const uint64_t bu = reinterpret_cast<uint64_t>(base);
-      base = reinterpret_cast<const uint8_t*>(
-          uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(bu))))) |
-          (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(bu >> 32))))) << 32));
-    } else {
-      row = mt * TM + slot;
-    }
-    wbase[j] = base;
-    woff[j] = uint32_t(min(row, a.M - 1) * a.row_bytes) + ((pc ^ swz(slot)) << 4);
-    wdst[j] = ((c & ~63u) >> 2) * KS;
+  for (int j = 0; j < 2 * TNW; ++j) {
+    const uint32_t g = 2u * TNW * wave + j, plane = g / (4u * TNW), tile = n_base / 16u + g % (4u * TNW);
+    src[TMW + j] = reinterpret_cast<const uint8_t*>(plane ? a.xl : a.xh) + size_t(tile) * kt * 1024u;
+    dst[TMW + j] = lds0 + WR * 64u + g * 1024u;
   }
-  // The address registers of a stage's loads are kept live until the end of
-  // the step that issued them (`hold`): were they reused for a fragment
-  // read's result, the compiler would first wait for every load in flight.
-  const uint8_t* src[6];
-  auto issue = [&](uint32_t st, auto tag) {
-    const uint32_t kb = min(st, st1 - 1u) * (KS * 2u);  // bytes; past the range: a valid, unused stage
-    _Float16* xb = xbuf(tag);
-    _Float16* wb = wbuf(tag);
+  auto issue = [&](uint32_t st, uint32_t buf) {
+    const uint32_t kb = min(st, st1 - 1u) * 1024u;  // past the range: a valid, unused stage
 #pragma unroll
-    for (int j = 0; j < 4; ++j) src[j] = xbase[j] + kb + xoff[j];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) src[4 + j] = wbase[j] + kb + woff[j];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) dma16(src[j], xb + xdst[j]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) dma16(src[4 + j], wb + wdst[j]);
-  };
-  auto hold = [&]() {
-    asm volatile("" : : "v"(src[0]), "v"(src[1]), "v"(src[2]), "v"(src[3]), "v"(src[4]), "v"(src[5]));
+    for (int j = 0; j < PER; ++j) dma16(src[j] + kb, off, dst[j] + buf);
   };
 
-  floatx16 acc[2][2], accl[1][1];
+  // fragments of 16 k (half h of a stage): rows fr + 32 i, chunk 2 h + lane / 32;
+  // token rows are swizzled (the swizzle repeats every 32 rows), weight tiles
+  // hold chunk c of row r at 16 (r % 16 + 16 c)
+  const uint32_t fr = lane & 31u;
+  const uint32_t wrd = wm * TMW * 2048u + (fr >> 4) * 1024u + (fr & 15u) * 16u + (lane >> 5) * 256u;
+  const uint32_t xrd = WR * 64u + (wn * 32u * TNW + fr) * 64u + (((lane >> 5) ^ swz(fr)) << 4);
+  struct Frags {
+    half8 w[TMW], x[TNW][2];
+  };
+  auto read = [&](Frags& f, uint32_t buf, uint32_t h) {
+    const uint8_t* pw = gemm_lds + buf + wrd + h * 512u;
+    const uint8_t* px = gemm_lds + buf + (xrd ^ (h << 5));
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TNW; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
-  const uint32_t fr = lane & 31u, fk = 8u * (lane >> 5);
-  // stage st in buffer B: wait until it has landed in every thread (only the
-  // next stage's loads may still be in flight), then the buffer of stage st - 1
-  // is free for stage st + 2
-  auto step = [&](uint32_t st, auto tag) {
-    constexpr int B = decltype(tag)::value;
-    __builtin_amdgcn_s_waitcnt(0x0F70 | GEMM_DMA_PER_STAGE);  // vmcnt(6); lgkmcnt / expcnt unconstrained
+      for (int p = 0; p < 2; ++p) f.x[i][p] = *reinterpret_cast<const half8*>(px + (p * XR + 32 * i) * 64);
+#pragma unroll
+    for (int i = 0; i < TMW; ++i) f.w[i] = *reinterpret_cast<const half8*>(pw + 32 * i * 64);
+  };
+  // The lo products have their own sums where the registers allow it: half as
+  // many roundings at the size of the hi sums
+  constexpr int LP = TNW == 1 ? 2 : 1;
+  floatx16 accp[LP][TNW][TMW];
+#pragma unroll
+  for (int p = 0; p < LP; ++p)
+#pragma unroll
+    for (int i = 0; i < TNW; ++i)
+#pragma unroll
+      for (int j = 0; j < TMW; ++j) accp[p][i][j] = floatx16{};
+  auto mma = [&](const Frags& f) {  // the hi products of every accumulator first, then the lo products
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int j = 0; j < TMW; ++j)
+#pragma unroll
+        for (int i = 0; i < TNW; ++i)
+          accp[p % LP][i][j] =
+              __builtin_amdgcn_mfma_f32_32x32x16_f16(f.x[i][p], f.w[j], accp[p % LP][i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int b = 0; b < NB; ++b) issue(st0 + b, b * STAGE);
+  __builtin_amdgcn_s_waitcnt(wait_imm((NB - 1) * PER, false));  // vmcnt: stage st0 has landed
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  Frags f0, f1;
+  uint32_t buf = 0;
+  read(f0, 0, 0);
+  for (uint32_t st = st0; st < st1; ++st) {
+    read(f1, buf, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(f0);
+    __builtin_amdgcn_sched_barrier(0);
+    // vmcnt: stage st + 1 has landed; lgkmcnt(0): stage st is read
+    __builtin_amdgcn_s_waitcnt(wait_imm((NB - 2) * PER, true));
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    // every fragment of the stage is read before the next loads are issued
-    // (an LDS read behind an LDS-DMA load makes the compiler wait for it)
-    const _Float16* xb = xbuf(tag);
-    const _Float16* wb = wbuf(tag);
-    half8 xa[2][2][2], wf[2][2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const uint32_t kk = 16u * q;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-          xa[q][t][p] = *reinterpret_cast<const half8*>(xb + p * (TN * KS) + tile_off(64 * wn + 32 * t + fr, kk + fk));
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-        wf[q][t] = *reinterpret_cast<const half8*>(wb + tile_off(64 * wm + 32 * t + fr, kk + fk));
-    }
-    issue(st + 2, StageTag<(B + 2) % 3>{});
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-      // the four accumulators' hi products first, then their lo products
-#pragma unroll
-      for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int tn = 0; tn < 2; ++tn)
-#pragma unroll
-          for (int tm = 0; tm < 2; ++tm)
-            acc[tn][tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[q][tn][p], wf[q][tm], acc[tn][tm], 0, 0, 0);
-    hold();
-  };
-  issue(st0, StageTag<0>{});
-  issue(st0 + 1, StageTag<1>{});
-  for (uint32_t st = st0; st < st1; st += 3) {
-    step(st, StageTag<0>{});
-    if (st + 1 < st1) step(st + 1, StageTag<1>{});
-    if (st + 2 < st1) step(st + 2, StageTag<2>{});
+    issue(st + NB, buf);
+    buf = buf + STAGE == NB * STAGE ? 0u : buf + STAGE;
+    read(f0, buf, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(f1);
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // the unused tail loads have landed before the block ends
-  gemm_epilogue<W_F16, EPI>(a, acc, accl, mt, n_base, sp, splits, wm, wn, lane);
+  __builtin_amdgcn_s_waitcnt(wait_imm(0, false));  // the unused tail loads have landed before the block ends
+
+  auto& acc = accp[0];
+  if constexpr (LP == 2) {
+#pragma unroll
+    for (int i = 0; i < TNW; ++i)
+#pragma unroll
+      for (int j = 0; j < TMW; ++j) acc[i][j] += accp[LP - 1][i][j];
+  }
+  // acc[i][j][v] = D[token 8 (v / 4) + 4 (lane / 32) + v % 4][weight slot lane % 32]
+#pragma unroll
+  for (int i = 0; i < TNW; ++i) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const uint32_t n = n_base + 32u * (TNW * wn + i) + 8u * (v / 4) + 4u * (lane >> 5) + (v % 4);
+      if (n >= a.N) continue;
+      const float r = splits > 1 ? 1.0f : a.rs[n];
+      if constexpr (DUAL) {
+#pragma unroll
+        for (int j = 0; j < TMW; j += 2) {
+          const uint32_t m = m_base + 16u * (TMW * wm + j) + fr;
+          if (m >= a.M) continue;
+          const float g = acc[i][j][v] * r, u = acc[i][j + 1][v] * r;
+          float* dst = a.y + size_t(n) * a.ldy + m;
+          if constexpr (EPI == EPI_SWIGLU_SLOW) {
+            const float sig = __fdiv_rn(1.0f, __fadd_rn(1.0f, expf_glibc(-g)));
+            *dst = __fmul_rn(__fmul_rn(g, sig), u);
+          } else {
+            *dst = __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, expf_glibc(-g))), u);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < TMW; ++j) {
+          const uint32_t m = m_base + 32u * (TMW * wm + j) + fr;
+          if (m >= a.M) continue;
+          if (splits > 1) {
+            a.part[(size_t(sp) * a.N + n) * a.M + m] = acc[i][j][v];
+          } else {
+            const float g = acc[i][j][v] * r;
+            float* dst = a.y + size_t(n) * a.ldy + m;
+            if constexpr (EPI == EPI_STORE) *dst = g;
+            else *dst = __fadd_rn(*dst, g);
+          }
+        }
+      }
+    }
+  }
 }
 
 // y[n][m] (op)= rs[n] * (part[0][n][m] + part[1][n][m] + ...), splits added in
@@ -653,8 +692,8 @@ __global__ __launch_bounds__(SK_WAVES * 64) void skinny_mfma_kernel(SkinnyArgs a
   if constexpr (DUAL) wp[NW - 1] = a.w3 + size_t(wr) * a.row_bytes;
   const uint32_t koff = 8u * (lane >> 4);
   const uint32_t tok = lane & 15u;
-  const _Float16* xhp = a.xh + size_t(tok) * a.K + koff;
-  const _Float16* xlp = a.xl + size_t(tok) * a.K + koff;
+  const _Float16* xhp = a.xh + plane_off(tok, koff, a.K);
+  const _Float16* xlp = a.xl + plane_off(tok, koff, a.K);
   const uint32_t kq = a.K / SK_WAVES, kbeg = wave * kq, steps = kq / 32;
   const uint32_t done = a.done ? *a.done : 0u;
 
@@ -665,8 +704,8 @@ __global__ __launch_bounds__(SK_WAVES * 64) void skinny_mfma_kernel(SkinnyArgs a
     const uint32_t k = kbeg + 32u * min(s, steps - 1);  // clamped: past-the-end steps reload the last one
 #pragma unroll
     for (int m = 0; m < NW; ++m) weight8<WT>(wp[m], k + koff, st.wh[m], st.wl[m]);
-    st.bh = *reinterpret_cast<const half8*>(xhp + k);
-    st.bl = *reinterpret_cast<const half8*>(xlp + k);
+    st.bh = *reinterpret_cast<const half8*>(xhp + k * 16u);
+    st.bl = *reinterpret_cast<const half8*>(xlp + k * 16u);
   };
   floatx4 acc[NW], accl[NW];
 #pragma unroll
@@ -1052,24 +1091,89 @@ hipError_t launch_split_rows(const float* x, uint32_t ldx, const float* norm, fl
 // 4 sets measured the same for 1536-token prefill (92.3 / 94.3 / 93.1 ms).
 constexpr int GEMM_DEPTH = 2;
 
-static hipError_t gemm_f16(int epi, const GemmArgs& a, uint32_t m_tiles, uint32_t n_tiles, uint32_t splits,
-                           hipStream_t s) {
-  const dim3 grid((m_tiles + 7u) / 8u * 8u * n_tiles * splits), block(256);
+// Tile of the F16 product and its K split.  Three tiles (weight rows x tokens,
+// LDS stages): 128 x 64 x 4, 256 x 64 x 3, 256 x 128 x 2, all two blocks per CU.
+// Up to GEMM_WIDE_N tokens a product has few tiles and each stage's loads bound
+// it, so the smaller tiles with deeper pipelines win, spread over whole rounds
+// of the 256 CUs; beyond, 256 x 128 (fewest LDS reads per MFMA) over whole
+// rounds of 512 resident blocks.  Among the candidates the fill of the last
+// round decides, a split costing its partial sums' traffic.  Measured (us, 40 /
+// 256 / 512 / 1500 tokens, 128x64x4 : 256x64x3 : 256x128x2): w1/w3 28.8 : 41.7 :
+// -, 67.5 : 70.3 : 78.8, 110 : 110 : 119, - : 286 : 263; w2 (K 9728) in its best
+// split 14.4 : 18.4 : -, 33.0 : 31.0 : 36, 54.3 : 52.9 : 54.0, - : 144 : 133.
+// (The 128 x 128 tile of 64 x 64 waves with row-major operands took 95 us for
+// w1/w3 at 256 tokens and 153 at 512.)
+// Long rows are split at least so often that no running sum gets longer than
+// it was before these tiles: 2560 wide with the lo products apart (64-token
+// tiles), 1280 where they share the accumulator, at most four.
+constexpr uint32_t GEMM_WIDE_N = 768;
+struct GemmPlan {
+  uint32_t tile;  // 0: 128 x 64, 1: 256 x 64, 2: 256 x 128
+  uint32_t m_tiles, n_tiles, splits;
+};
+static GemmPlan gemm_plan(const GemmArgs& a, bool dual) {
+  GemmPlan best{};
+  float best_score = -1.0f;
+  const bool wide = a.N > GEMM_WIDE_N;
+  const uint32_t slots = wide ? 512u : 256u;
+  for (uint32_t tile = wide ? 1u : 0u; tile < (wide ? 3u : 2u); ++tile) {
+    const uint32_t wr = (tile ? 256u : 128u) / (dual ? 2u : 1u), xr = tile == 2u ? 128u : 64u;
+    GemmPlan p{tile, (a.M + wr - 1) / wr, (a.N + xr - 1) / xr, 1u};
+    const uint32_t most = dual || !a.part || a.M % 4u ? 1u : GEMM_MAX_SPLITS;
+    const uint32_t least = std::min(std::min(most, 4u), tile == 2u ? (a.K + 1279u) / 1280u : (a.K + 2559u) / 2560u);
+    for (p.splits = 1; p.splits <= most; ++p.splits) {
+      if (p.splits > 1 && (a.K / KS < 8u * p.splits || size_t(p.splits) * a.N * a.M > a.part_cap)) break;
+      const uint32_t blocks = p.m_tiles * p.n_tiles * p.splits, rounds = (blocks + slots - 1) / slots;
+      float score = float(blocks) / float(rounds * slots);
+      if (p.splits > 1) score /= 1.0f + float(p.splits) * 480.0f / float(a.K);
+      // near ties: 256 x 64 over 128 x 64; 256 x 128 where it fills a round
+      if (tile == 1u && !wide) score *= 1.03f;
+      if (tile == 2u) score *= blocks >= slots ? 1.03f : 0.97f;
+      if (p.splits < least) score *= 0.1f * float(p.splits);
+      if (score > best_score) {
+        best_score = score;
+        best = p;
+      }
+    }
+  }
+  return best;
+}
+
+template <int EPI, int TMW, int TNW, int NB>
+static hipError_t gemm_f16_launch(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
+  constexpr uint32_t lds = NB * (64 * TMW + 2 * 64 * TNW) * KS * 2;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f16_dma_kernel<EPI, TMW, TNW, NB>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((gemm_f16_dma_kernel<EPI, TMW, TNW, NB>), dim3(p.m_tiles * p.n_tiles * p.splits), dim3(256), lds, s,
+                     a, p.m_tiles, p.n_tiles, p.splits);
+  return hipGetLastError();
+}
+template <int EPI>
+static hipError_t gemm_f16_tile(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
+  switch (p.tile) {
+    case 0: return gemm_f16_launch<EPI, 2, 1, 4>(a, p, s);
+    case 1: return gemm_f16_launch<EPI, 4, 1, 3>(a, p, s);
+    default: return gemm_f16_launch<EPI, 4, 2, 2>(a, p, s);
+  }
+}
+static hipError_t gemm_f16(int epi, const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
   switch (epi) {
-    case EPI_STORE:
-      hipLaunchKernelGGL((gemm_f16_dma_kernel<EPI_STORE>), grid, block, 0, s, a, m_tiles, n_tiles, splits);
-      break;
-    case EPI_RESID:
-      hipLaunchKernelGGL((gemm_f16_dma_kernel<EPI_RESID>), grid, block, 0, s, a, m_tiles, n_tiles, splits);
-      break;
-    case EPI_SWIGLU_SLOW:
-      hipLaunchKernelGGL((gemm_f16_dma_kernel<EPI_SWIGLU_SLOW>), grid, block, 0, s, a, m_tiles, n_tiles, splits);
-      break;
-    case EPI_SWIGLU_FAST:
-      hipLaunchKernelGGL((gemm_f16_dma_kernel<EPI_SWIGLU_FAST>), grid, block, 0, s, a, m_tiles, n_tiles, splits);
-      break;
+    case EPI_STORE: return gemm_f16_tile<EPI_STORE>(a, p, s);
+    case EPI_RESID: return gemm_f16_tile<EPI_RESID>(a, p, s);
+    case EPI_SWIGLU_SLOW: return gemm_f16_tile<EPI_SWIGLU_SLOW>(a, p, s);
+    case EPI_SWIGLU_FAST: return gemm_f16_tile<EPI_SWIGLU_FAST>(a, p, s);
     default: return hipErrorInvalidValue;
   }
+}
+
+static hipError_t gemm_reduce(int epi, const GemmArgs& a, uint32_t splits, hipStream_t s) {
+  const dim3 rgrid(uint32_t((size_t(a.N) * (a.M / 4u) + 255u) / 256u)), block(256);
+  if (epi == EPI_STORE)
+    hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI_STORE>), rgrid, block, 0, s, a, splits);
+  else
+    hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI_RESID>), rgrid, block, 0, s, a, splits);
   return hipGetLastError();
 }
 
@@ -1077,10 +1181,6 @@ template <uint32_t WT>
 static hipError_t gemm_epi(int epi, const GemmArgs& a, uint32_t m_tiles, uint32_t n_tiles, uint32_t splits,
                            hipStream_t s) {
   const dim3 grid((m_tiles + 7u) / 8u * 8u * n_tiles * splits), block(256);
-  if (WT == W_F16) {
-    const hipError_t e = gemm_f16(epi, a, m_tiles, n_tiles, splits, s);
-    if (e != hipSuccess) return e;
-  } else {
   switch (epi) {
     case EPI_STORE:
       hipLaunchKernelGGL((gemm_mfma_kernel<WT, EPI_STORE, GEMM_DEPTH>), grid, block, 0, s, a, m_tiles, n_tiles,
@@ -1100,25 +1200,27 @@ static hipError_t gemm_epi(int epi, const GemmArgs& a, uint32_t m_tiles, uint32_
       break;
     default: return hipErrorInvalidValue;
   }
-  }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || splits == 1) return e;
-  const dim3 rgrid(uint32_t((size_t(a.N) * (a.M / 4u) + 255u) / 256u));
-  if (epi == EPI_STORE)
-    hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI_STORE>), rgrid, block, 0, s, a, splits);
-  else
-    hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI_RESID>), rgrid, block, 0, s, a, splits);
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess || splits == 1 ? e : gemm_reduce(epi, a, splits, s);
 }
 
 uint32_t gemm_rows_pad(uint32_t n) { return (n + TN - 1) / TN * TN; }
 
-size_t gemm_part_floats(uint32_t n_pad, uint32_t m) { return size_t(GEMM_MAX_SPLITS) * n_pad * m; }
+// (more than four splits only pay below GEMM_WIDE_N tokens)
+size_t gemm_part_floats(uint32_t n_pad, uint32_t m) {
+  return std::max(size_t(GEMM_MAX_SPLITS) * std::min(n_pad, GEMM_WIDE_N), size_t(4) * n_pad) * m;
+}
 
 hipError_t launch_gemm_mfma(uint32_t wtype, int epi, const GemmArgs& a, hipStream_t s) {
   if (a.K % KS || a.M == 0 || a.N == 0) return hipErrorInvalidValue;
   const bool dual = epi == EPI_SWIGLU_SLOW || epi == EPI_SWIGLU_FAST;
   if (dual && !a.w3) return hipErrorInvalidValue;
+  if (wtype == W_F16 && a.wt) {
+    if (dual && !a.wt3) return hipErrorInvalidValue;
+    const GemmPlan p = gemm_plan(a, dual);
+    const hipError_t e = gemm_f16(epi, a, p, s);
+    return e != hipSuccess || p.splits == 1 ? e : gemm_reduce(epi, a, p.splits, s);
+  }
   const uint32_t m_tiles = dual ? (a.M + 63u) / 64u : (a.M + TM - 1u) / TM;
   const uint32_t n_tiles = gemm_rows_pad(a.N) / TN;
   // short-M products: split K so that the grid covers the 256 CUs (each split
@@ -1126,7 +1228,7 @@ hipError_t launch_gemm_mfma(uint32_t wtype, int epi, const GemmArgs& a, hipStrea
   uint32_t splits = 1;
   if (!dual && a.part && a.M % 4u == 0) {
     const uint32_t tiles = m_tiles * n_tiles;
-    while (splits < GEMM_MAX_SPLITS && tiles * splits < 256u && a.K / KS >= 8u * (splits + 1u) &&
+    while (splits < 4u && tiles * splits < 256u && a.K / KS >= 8u * (splits + 1u) &&
            size_t(splits + 1u) * a.N * a.M <= a.part_cap)
       ++splits;
   }

@@ -1,0 +1,42 @@
+"""Prompt lengths around the tile edges of the prefill products, on every weight
+type: one token past and short of a 64- and 128-token tile, past the length
+where the wide tile takes over, and past one prefill pass (2048 tokens).  The
+second shape's FFN width is no multiple of a weight tile (and, as the input
+width of w2, has no fragment-ordered copy).  f32-level products: hidden
+states and logits agree with the oracle to 1e-4 relative."""
+
+import numpy as np
+import pytest
+
+from conftest import make_prompt
+from oracle import oracle as O
+from s2hip import synth
+
+pytestmark = pytest.mark.gpu
+
+BASE = synth.TINY.with_(name="tiles", slow_layers=2, fast_layers=1, vocab=2304, semantic_begin=1024, semantic_end=2047,
+                        im_end_id=1000)
+TYPES = {"f16": synth.GGML_F16, "q8_0": synth.GGML_Q8_0, "q4_0": synth.GGML_Q4_0}
+
+
+def _rel(a, b):
+    return float(np.max(np.abs(a - b)) / max(1e-30, float(np.max(np.abs(b)))))
+
+
+@pytest.mark.parametrize("weights", sorted(TYPES))
+@pytest.mark.parametrize("ffn,lengths", [(1536, (3, 16, 17, 63, 65, 129, 257, 770, 2100)), (1504, (5, 33, 300))])
+def test_prefill_lengths_match_oracle(model_dir, weights, ffn, lengths):
+    from s2hip import Engine
+
+    shape = BASE.with_(name=f"tiles{ffn}", linear_type=TYPES[weights], ffn=ffn)
+    path = synth.ensure_gguf(shape, model_dir)
+    o = O.OracleModel(path, 2200, shape.im_end_id)
+    with Engine(path, 2200, shape.im_end_id) as e:
+        for n in lengths:
+            prompt = make_prompt(shape, n, seed=n)
+            e.reset()
+            o.reset()
+            hg, lg = e.eval(prompt)
+            ho, lo = o.eval(prompt)
+            assert e.n_past == n
+            assert _rel(hg, ho) < 1e-4 and _rel(lg, lo) < 1e-4, (n, _rel(hg, ho), _rel(lg, lo))
