@@ -39,6 +39,7 @@
 
 #include "expf_glibc.h"
 #include "kernels.h"
+#include "qfrag.h"
 #include "wave.h"
 
 namespace s2 {
@@ -69,6 +70,70 @@ __global__ __launch_bounds__(256) void tile_f16_kernel(const uint16_t* src, uint
     *reinterpret_cast<uint4*>(dst + q * 8) = v;
   }
 }
+
+// ---------------------------------------------------------------------------
+// Q8_0 / Q4_0 rows -> the same tiles, a block of 32 k per row: lane l's 8
+// values as 8 bytes (Q8_0: q + 128) or 4 bytes (Q4_0: the stored nibbles,
+// value 2 j at nibble j and value 2 j + 1 at nibble j + 4), and the 16 row
+// scales of a tile as f16 at [tile][16].  Rows M..Mpad-1 have scale 0.
+// ---------------------------------------------------------------------------
+template <uint32_t WT>
+__global__ __launch_bounds__(256) void tile_q_kernel(const uint8_t* src, size_t row_bytes, uint32_t K, uint32_t M,
+                                                     uint32_t Mpad, uint8_t* dst, uint16_t* scales) {
+  constexpr uint32_t BB = WT == W_Q8_0 ? 34u : 18u;
+  const uint32_t kt = K / 32;
+  const size_t chunks = size_t(Mpad / 16) * kt * 64;
+  for (size_t q = size_t(blockIdx.x) * 256 + threadIdx.x; q < chunks; q += size_t(gridDim.x) * 256) {
+    const size_t tile = q / 64;
+    const uint32_t lane = uint32_t(q % 64), grp = lane / 16;
+    const uint32_t tm = uint32_t(tile / kt), tk = uint32_t(tile % kt), r = 16 * tm + lane % 16;
+    const uint8_t* blk = src + size_t(r) * row_bytes + size_t(tk) * BB;
+    uint32_t u[8] = {};  // unsigned values; a padded row's are zero (its scale is too)
+    if (r < M) {
+#pragma unroll
+      for (uint32_t e = 0; e < 8; ++e)
+        u[e] = WT == W_Q8_0 ? blk[2 + 8 * grp + e] ^ 0x80u : (blk[2 + 8 * (grp & 1u) + e] >> (grp >= 2 ? 4 : 0)) & 15u;
+    }
+    if constexpr (WT == W_Q8_0) {
+      uint2 o = make_uint2(0u, 0u);
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) {
+        o.x |= u[e] << (8 * e);
+        o.y |= u[4 + e] << (8 * e);
+      }
+      *reinterpret_cast<uint2*>(dst + q * 8) = o;
+    } else {
+      uint32_t o = 0;
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) o |= (u[2 * j] << (4 * j)) | (u[2 * j + 1] << (4 * j + 16));
+      *reinterpret_cast<uint32_t*>(dst + q * 4) = o;
+    }
+    if (lane < 16) scales[tile * 16 + lane] = r < M ? uint16_t(blk[0] | (uint32_t(blk[1]) << 8)) : uint16_t(0);
+  }
+}
+
+// A lane's weights of one step as loaded, and as f16 (Q8_0 / Q4_0: the
+// integers, exact; the block's scale goes to the 32-k partial sum, so a
+// quantized product costs the MFMAs of an F16 one and one FMA per result).
+// Q4_0 at 5 columns, us per launch (before: row-major blocks dequantised and
+// split per fragment, plus a launch of ~5 us to split the activations):
+// w1/w3 79 -> 21, w2 and wo 31 -> 12.7, wqkv 32 -> 11.2.
+template <uint32_t WT>
+struct WRaw {
+  half8 v;
+};
+template <>
+struct WRaw<W_Q8_0> {
+  uint2 v;
+  uint2 d;  // f16 scales of the lane's 4 result rows
+};
+template <>
+struct WRaw<W_Q4_0> {
+  uint32_t v;
+  uint2 d;
+};
+template <uint32_t WT>
+constexpr uint32_t TILE_BYTES = WT == W_F16 ? 1024u : WT == W_Q8_0 ? 512u : 256u;
 
 // ---------------------------------------------------------------------------
 // Batched product.  Block = WAVES waves on one 16-row tile; wave w takes the
@@ -103,9 +168,45 @@ __device__ __forceinline__ void split8(const floatx4& a, const floatx4& b, half8
 // Weight fragments are read once per launch: non-temporal loads stream them
 // past L2 without evicting the staged activations (8 columns: w13 24.4 ->
 // 23.2 us).
-__device__ __forceinline__ half8 bmm_wload(const half8* p) { return __builtin_nontemporal_load(p); }
+template <uint32_t WT>
+__device__ __forceinline__ WRaw<WT> bmm_wload(const uint8_t* w, const uint8_t* scales, uint32_t tile) {
+  WRaw<WT> r;
+  if constexpr (WT == W_F16) {
+    r.v = __builtin_nontemporal_load(reinterpret_cast<const half8*>(w + size_t(tile) * 1024u));
+  } else {
+    if constexpr (WT == W_Q8_0) {
+      typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
+      const uint2v t = __builtin_nontemporal_load(reinterpret_cast<const uint2v*>(w + size_t(tile) * 512u));
+      r.v = make_uint2(t.x, t.y);
+    } else {
+      r.v = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(w + size_t(tile) * 256u));
+    }
+    r.d = *reinterpret_cast<const uint2*>(scales + size_t(tile) * 32u);
+  }
+  return r;
+}
+// acc += the product of one step (F16), or its scaled 32-k partial sum
+template <uint32_t WT>
+__device__ __forceinline__ half8 bmm_frag(const WRaw<WT>& r) {
+  if constexpr (WT == W_F16) return r.v;
+  else if constexpr (WT == W_Q8_0) return q8_frag(r.v.x, r.v.y);
+  else return q4_frag(r.v);
+}
+template <uint32_t WT>
+__device__ __forceinline__ void bmm_mma(const WRaw<WT>& r, const half8& w, const half8& x, floatx4& acc) {
+  if constexpr (WT == W_F16) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, acc, 0, 0, 0);
+  } else {
+    const floatx4 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, floatx4{}, 0, 0, 0);
+    const half2v d0 = __builtin_bit_cast(half2v, r.d.x), d1 = __builtin_bit_cast(half2v, r.d.y);
+    acc[0] = fmaf(float(d0.x), t[0], acc[0]);
+    acc[1] = fmaf(float(d0.y), t[1], acc[1]);
+    acc[2] = fmaf(float(d1.x), t[2], acc[2]);
+    acc[3] = fmaf(float(d1.y), t[3], acc[3]);
+  }
+}
 
-template <int EPI, bool NORM, int WAVES, int NB>
+template <uint32_t WT, int EPI, bool NORM, int WAVES, int NB>
 __global__ __launch_bounds__(WAVES * 64) void bmm_kernel(BmmArgs a) {
   constexpr bool DUAL = (EPI == EPI_SWIGLU_SLOW || EPI == EPI_SWIGLU_FAST);
   constexpr int NW = DUAL ? 2 : 1;
@@ -121,9 +222,12 @@ __global__ __launch_bounds__(WAVES * 64) void bmm_kernel(BmmArgs a) {
   const uint32_t tm = blockIdx.x, m0 = tm * 16;
   const uint32_t kt = a.K / 32, KS = kt / WAVES;
   const uint32_t n = lane & 15u, grp = lane >> 4;
-  const size_t tile0 = (size_t(tm) * kt + size_t(wave) * KS) * 512 + size_t(lane) * 8;
-  const _Float16* wp0 = a.wt + tile0;
-  const _Float16* wp1 = DUAL ? a.wt3 + tile0 : wp0;
+  constexpr uint32_t TB = TILE_BYTES<WT>;
+  const size_t tile0 = size_t(tm) * kt + size_t(wave) * KS;
+  const uint8_t* wp0 = static_cast<const uint8_t*>(a.wt) + tile0 * TB + lane * (TB / 64);
+  const uint8_t* wp1 = DUAL ? static_cast<const uint8_t*>(a.wt3) + tile0 * TB + lane * (TB / 64) : wp0;
+  const uint8_t* sp0 = WT == W_F16 ? nullptr : reinterpret_cast<const uint8_t*>(a.ws + tile0 * 16) + 8 * grp;
+  const uint8_t* sp1 = WT == W_F16 || !DUAL ? sp0 : reinterpret_cast<const uint8_t*>(a.ws3 + tile0 * 16) + 8 * grp;
   const uint32_t last = KS - 1;
   const uint32_t nsc = (KS + WIN - 1) / WIN;  // pairs of chunks
   const uint32_t kbase = wave * KS * 32;
@@ -157,7 +261,7 @@ __global__ __launch_bounds__(WAVES * 64) void bmm_kernel(BmmArgs a) {
     if constexpr (NORM) *reinterpret_cast<floatx4*>(gsw + buf * (XC * 32) + 4 * sq) = gr;
   };
 
-  half8 wb[WIN][NW];
+  WRaw<WT> wb[WIN][NW];
   floatx4 sxa[LDX], sxb[LDX], sga, sgb;  // staged chunks in flight (even, odd)
   // chunk 0 and 1 activations, then the first WIN weight steps
   stage_load(sxa, sga, 0);
@@ -165,8 +269,8 @@ __global__ __launch_bounds__(WAVES * 64) void bmm_kernel(BmmArgs a) {
 #pragma unroll
   for (int i = 0; i < WIN; ++i) {
     const uint32_t t = min(uint32_t(i), last);
-    wb[i][0] = bmm_wload(reinterpret_cast<const half8*>(wp0 + 512 * t));
-    if constexpr (DUAL) wb[i][1] = bmm_wload(reinterpret_cast<const half8*>(wp1 + 512 * t));
+    wb[i][0] = bmm_wload<WT>(wp0, sp0, t);
+    if constexpr (DUAL) wb[i][1] = bmm_wload<WT>(wp1, sp1, t);
   }
   stage_store(sxa, sga, 0);
   // Per-(wave, column) power-of-two scale: the largest |x g| of the first two
@@ -251,13 +355,14 @@ __global__ __launch_bounds__(WAVES * 64) void bmm_kernel(BmmArgs a) {
       split8(x0, x1, bh, bl);
 #pragma unroll
       for (int m = 0; m < NW; ++m) {
-        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb[wi][m], bh, acc[m], 0, 0, 0);
-        accl[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb[wi][m], bl, accl[m], 0, 0, 0);
+        const half8 wf = bmm_frag<WT>(wb[wi][m]);
+        bmm_mma<WT>(wb[wi][m], wf, bh, acc[m]);
+        bmm_mma<WT>(wb[wi][m], wf, bl, accl[m]);
       }
       __builtin_amdgcn_sched_barrier(0);
       const uint32_t tw = min(s + WIN, last);
-      wb[wi][0] = bmm_wload(reinterpret_cast<const half8*>(wp0 + 512 * tw));
-      if constexpr (DUAL) wb[wi][1] = bmm_wload(reinterpret_cast<const half8*>(wp1 + 512 * tw));
+      wb[wi][0] = bmm_wload<WT>(wp0, sp0, tw);
+      if constexpr (DUAL) wb[wi][1] = bmm_wload<WT>(wp1, sp1, tw);
       __builtin_amdgcn_sched_barrier(0);
       cx0 = nx0;
       cx1 = nx1;
@@ -363,7 +468,7 @@ constexpr int PK_ROW = 40;                 // halfs per fragment row: 32 + 8 (co
 constexpr int PK_STEP = 16 * PK_ROW + 32;  // halfs per step: +64 B puts the 4 steps' staging writes on other banks
 constexpr int PK_QSTEP = 72;               // sum-of-squares floats per step: 8 columns x 4 groups x 2, +8
 
-template <int EPI, bool NORM, int WAVES>
+template <uint32_t WT, int EPI, bool NORM, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void bmm_pk_kernel(BmmArgs a) {
   constexpr bool DUAL = (EPI == EPI_SWIGLU_SLOW || EPI == EPI_SWIGLU_FAST);
   constexpr int NW = DUAL ? 2 : 1;
@@ -379,9 +484,12 @@ __global__ __launch_bounds__(WAVES * 64) void bmm_pk_kernel(BmmArgs a) {
   const uint32_t tm = blockIdx.x, m0 = tm * 16;
   const uint32_t kt = a.K / 32, KS = kt / WAVES;
   const uint32_t n = lane & 15u, grp = lane >> 4, col = n & 7u;
-  const size_t tile0 = (size_t(tm) * kt + size_t(wave) * KS) * 512 + size_t(lane) * 8;
-  const _Float16* wp0 = a.wt + tile0;
-  const _Float16* wp1 = DUAL ? a.wt3 + tile0 : wp0;
+  constexpr uint32_t TB = TILE_BYTES<WT>;
+  const size_t tile0 = size_t(tm) * kt + size_t(wave) * KS;
+  const uint8_t* wp0 = static_cast<const uint8_t*>(a.wt) + tile0 * TB + lane * (TB / 64);
+  const uint8_t* wp1 = DUAL ? static_cast<const uint8_t*>(a.wt3) + tile0 * TB + lane * (TB / 64) : wp0;
+  const uint8_t* sp0 = WT == W_F16 ? nullptr : reinterpret_cast<const uint8_t*>(a.ws + tile0 * 16) + 8 * grp;
+  const uint8_t* sp1 = WT == W_F16 || !DUAL ? sp0 : reinterpret_cast<const uint8_t*>(a.ws3 + tile0 * 16) + 8 * grp;
   const uint32_t last = KS - 1;
   const uint32_t nsc = (KS + WIN - 1) / WIN;  // pairs of chunks
   const uint32_t kbase = wave * KS * 32;
@@ -404,15 +512,15 @@ __global__ __launch_bounds__(WAVES * 64) void bmm_pk_kernel(BmmArgs a) {
     }
   };
 
-  half8 wb[WIN][NW];
+  WRaw<WT> wb[WIN][NW];
   floatx4 sxa[LDX], sxb[LDX], sga, sgb;  // staged chunks in flight (even, odd)
   stage_load(sxa, sga, 0);
   stage_load(sxb, sgb, 1);
 #pragma unroll
   for (int i = 0; i < WIN; ++i) {
     const uint32_t t = min(uint32_t(i), last);
-    wb[i][0] = bmm_wload(reinterpret_cast<const half8*>(wp0 + 512 * t));
-    if constexpr (DUAL) wb[i][1] = bmm_wload(reinterpret_cast<const half8*>(wp1 + 512 * t));
+    wb[i][0] = bmm_wload<WT>(wp0, sp0, t);
+    if constexpr (DUAL) wb[i][1] = bmm_wload<WT>(wp1, sp1, t);
   }
   // Per-(wave, column) power-of-two scale from the largest |x g| of the first
   // two chunks of this wave's range, as in bmm_kernel.  Staging lanes need it
@@ -499,11 +607,11 @@ __global__ __launch_bounds__(WAVES * 64) void bmm_pk_kernel(BmmArgs a) {
         ss += cq.y;
       }
 #pragma unroll
-      for (int m = 0; m < NW; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wb[wi][m], cf, acc[m], 0, 0, 0);
+      for (int m = 0; m < NW; ++m) bmm_mma<WT>(wb[wi][m], bmm_frag<WT>(wb[wi][m]), cf, acc[m]);
       __builtin_amdgcn_sched_barrier(0);
       const uint32_t tw = min(s + WIN, last);
-      wb[wi][0] = bmm_wload(reinterpret_cast<const half8*>(wp0 + 512 * tw));
-      if constexpr (DUAL) wb[wi][1] = bmm_wload(reinterpret_cast<const half8*>(wp1 + 512 * tw));
+      wb[wi][0] = bmm_wload<WT>(wp0, sp0, tw);
+      if constexpr (DUAL) wb[wi][1] = bmm_wload<WT>(wp1, sp1, tw);
       __builtin_amdgcn_sched_barrier(0);
       cf = nf;
       cq = nq;
@@ -585,36 +693,46 @@ __global__ __launch_bounds__(WAVES * 64) void bmm_pk_kernel(BmmArgs a) {
   }
 }
 
-template <int EPI, bool NORM>
+template <uint32_t WT, int EPI, bool NORM>
 hipError_t launch_bmm_pk(const BmmArgs& a, uint32_t waves, hipStream_t s) {
   const dim3 grid((a.M + 15) / 16);
   switch (waves) {
-    case 1: hipLaunchKernelGGL((bmm_pk_kernel<EPI, NORM, 1>), grid, dim3(64), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((bmm_pk_kernel<EPI, NORM, 2>), grid, dim3(128), 0, s, a); break;
-    case 4: hipLaunchKernelGGL((bmm_pk_kernel<EPI, NORM, 4>), grid, dim3(256), 0, s, a); break;
-    case 8: hipLaunchKernelGGL((bmm_pk_kernel<EPI, NORM, 8>), grid, dim3(512), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((bmm_pk_kernel<WT, EPI, NORM, 1>), grid, dim3(64), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((bmm_pk_kernel<WT, EPI, NORM, 2>), grid, dim3(128), 0, s, a); break;
+    case 4: hipLaunchKernelGGL((bmm_pk_kernel<WT, EPI, NORM, 4>), grid, dim3(256), 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
-template <int EPI, bool NORM, int NB>
+template <uint32_t WT, int EPI, bool NORM, int NB>
 hipError_t launch_bmm_waves(const BmmArgs& a, uint32_t waves, hipStream_t s) {
   const dim3 grid((a.M + 15) / 16);
   switch (waves) {
-    case 1: hipLaunchKernelGGL((bmm_kernel<EPI, NORM, 1, NB>), grid, dim3(64), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((bmm_kernel<EPI, NORM, 2, NB>), grid, dim3(128), 0, s, a); break;
-    case 4: hipLaunchKernelGGL((bmm_kernel<EPI, NORM, 4, NB>), grid, dim3(256), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((bmm_kernel<WT, EPI, NORM, 1, NB>), grid, dim3(64), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((bmm_kernel<WT, EPI, NORM, 2, NB>), grid, dim3(128), 0, s, a); break;
+    case 4: hipLaunchKernelGGL((bmm_kernel<WT, EPI, NORM, 4, NB>), grid, dim3(256), 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
-template <int EPI>
+template <uint32_t WT, int EPI>
 hipError_t launch_bmm_epi(const BmmArgs& a, uint32_t waves, hipStream_t s) {
   const bool norm = a.norm != nullptr;
-  if (a.N <= 8) return norm ? launch_bmm_pk<EPI, true>(a, waves, s) : launch_bmm_pk<EPI, false>(a, waves, s);
-  return norm ? launch_bmm_waves<EPI, true, 16>(a, waves, s) : launch_bmm_waves<EPI, false, 16>(a, waves, s);
+  if (a.N <= 8) return norm ? launch_bmm_pk<WT, EPI, true>(a, waves, s) : launch_bmm_pk<WT, EPI, false>(a, waves, s);
+  return norm ? launch_bmm_waves<WT, EPI, true, 16>(a, waves, s) : launch_bmm_waves<WT, EPI, false, 16>(a, waves, s);
+}
+
+template <uint32_t WT>
+hipError_t launch_bmm_type(int epi, const BmmArgs& a, uint32_t waves, hipStream_t s) {
+  switch (epi) {
+    case EPI_STORE: return launch_bmm_epi<WT, EPI_STORE>(a, waves, s);
+    case EPI_RESID: return launch_bmm_epi<WT, EPI_RESID>(a, waves, s);
+    case EPI_SWIGLU_SLOW: return launch_bmm_epi<WT, EPI_SWIGLU_SLOW>(a, waves, s);
+    case EPI_SWIGLU_FAST: return launch_bmm_epi<WT, EPI_SWIGLU_FAST>(a, waves, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace
@@ -628,6 +746,21 @@ hipError_t launch_tile_f16(const uint16_t* src, uint32_t K, uint32_t M, uint32_t
   const size_t chunks = size_t(Mpad / 16) * (K / 32) * 64;
   const uint32_t blocks = uint32_t(std::min<size_t>((chunks + 255) / 256, 8192));
   hipLaunchKernelGGL(tile_f16_kernel, dim3(blocks), dim3(256), 0, s, src, K, M, Mpad, row_base, extra_row, dst);
+  return hipGetLastError();
+}
+
+uint32_t tile_q_bytes(uint32_t wtype) { return wtype == W_Q8_0 ? TILE_BYTES<W_Q8_0> : wtype == W_Q4_0 ? TILE_BYTES<W_Q4_0> : 0u; }
+
+hipError_t launch_tile_q(const uint8_t* src, size_t row_bytes, uint32_t wtype, uint32_t K, uint32_t M, uint8_t* dst,
+                         uint16_t* scales, hipStream_t s) {
+  if (K % 32 || M == 0 || !tile_q_bytes(wtype)) return hipErrorInvalidValue;
+  const uint32_t Mpad = bmm_rows_pad(M);
+  const size_t chunks = size_t(Mpad / 16) * (K / 32) * 64;
+  const uint32_t blocks = uint32_t(std::min<size_t>((chunks + 255) / 256, 8192));
+  if (wtype == W_Q8_0)
+    hipLaunchKernelGGL(tile_q_kernel<W_Q8_0>, dim3(blocks), dim3(256), 0, s, src, row_bytes, K, M, Mpad, dst, scales);
+  else
+    hipLaunchKernelGGL(tile_q_kernel<W_Q4_0>, dim3(blocks), dim3(256), 0, s, src, row_bytes, K, M, Mpad, dst, scales);
   return hipGetLastError();
 }
 
@@ -649,11 +782,11 @@ hipError_t launch_bmm(int epi, const BmmArgs& a, hipStream_t s) {
   if (dual && !a.wt3) return hipErrorInvalidValue;
   const uint32_t waves = a.waves ? a.waves : bmm_waves(a.M, a.K);
   if ((a.K / 32) % waves) return hipErrorInvalidValue;
-  switch (epi) {
-    case EPI_STORE: return launch_bmm_epi<EPI_STORE>(a, waves, s);
-    case EPI_RESID: return launch_bmm_epi<EPI_RESID>(a, waves, s);
-    case EPI_SWIGLU_SLOW: return launch_bmm_epi<EPI_SWIGLU_SLOW>(a, waves, s);
-    case EPI_SWIGLU_FAST: return launch_bmm_epi<EPI_SWIGLU_FAST>(a, waves, s);
+  if (a.wtype != W_F16 && (!a.ws || (dual && !a.ws3))) return hipErrorInvalidValue;
+  switch (a.wtype) {
+    case W_F16: return launch_bmm_type<W_F16>(epi, a, waves, s);
+    case W_Q8_0: return launch_bmm_type<W_Q8_0>(epi, a, waves, s);
+    case W_Q4_0: return launch_bmm_type<W_Q4_0>(epi, a, waves, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -93,9 +93,11 @@ struct DevLin {
   uint32_t in = 0, out = 0;
   size_t row_bytes = 0;
   uint64_t bytes = 0;
-  // F16 weights in MFMA fragment order for the batched product (built on
-  // first use); its rows are the logical rows (any row mapping baked in)
-  _Float16* wt = nullptr;
+  // the weights in MFMA fragment order for the batched and prefill products
+  // (built on first use; Q8_0 / Q4_0: integer tiles and their scales ws); its
+  // rows are the logical rows (any row mapping baked in)
+  uint8_t* wt = nullptr;
+  uint16_t* ws = nullptr;
   // Q8_0 / Q4_0 rows repacked for the one-column decode GEMV (built on
   // first use): 16-byte-aligned block values and an f16 scale plane
   uint8_t* qp = nullptr;
@@ -197,8 +199,10 @@ class Engine {
   void enqueue_prefill_gemv(const int32_t* prompt_dev, size_t n_tok, uint32_t seq);
   void ensure_slots(uint32_t n);
   void ensure_tiled();
+  void ensure_repacked();
   void repack(DevLin& L);
   void tile(DevLin& L, uint32_t rows, uint32_t row_base, uint32_t extra_row);
+  uint8_t* try_dalloc(size_t bytes);
   void bmm(const DevLin& L, const DevLin* L3, int epi, uint32_t ncol, const float* x, uint32_t ldx, const float* norm,
            float eps, float* y, uint32_t ldy, const uint32_t* done, uint32_t* err, uint32_t waves = 0);
   void validate_prompt(const int32_t* prompt, size_t cols);
@@ -243,7 +247,7 @@ class Engine {
   float *norm_ = nullptr, *fast_norm_ = nullptr;
   DevLin head_full_, fast_out_;
   DevLin head_cand_;  // the candidate rows of the head (tiled copy only)
-  bool tiled_ = false;
+  bool tiled_ = false, repacked_ = false;
   uint32_t bmm_min_cols_ = 2;  // columns from which F16 linears use the batched product
   // Set while a call is re-run after ERR_F16_RANGE: every multi-column linear
   // then takes the per-column paths (two-column GEMV, or the skinny product
@@ -688,6 +692,9 @@ void Engine::bmm(const DevLin& L, const DevLin* L3, int epi, uint32_t ncol, cons
     BmmArgs b{};
     b.wt = L.wt;
     b.wt3 = L3 ? L3->wt : nullptr;
+    b.ws = L.ws;
+    b.ws3 = L3 ? L3->ws : nullptr;
+    b.wtype = L.type;
     b.M = L.out;
     b.K = L.in;
     b.x = x + size_t(c) * ldx;
@@ -711,6 +718,7 @@ void Engine::bmm(const DevLin& L, const DevLin* L3, int epi, uint32_t ncol, cons
 // frames/s against 304.1-304.3 with w1/w3 and w2 on the product).
 bool Engine::uses_bmm(const DevLin& L, const DevLin* L3, uint32_t ncol) const {
   if (bmm_off_ || !L.wt || !bmm_min_cols_ || ncol < bmm_min_cols_ || (L3 && !L3->wt)) return false;
+  if (L.in % 256 || L.in > BMM_MAX_K) return false;
   return !(ncol == 2 && gemv_rows_per_block(L.type, L.in, L.out, false, L3 != nullptr, ncol) != 0);
 }
 
@@ -1076,6 +1084,8 @@ void Engine::mm(const DevLin& L, const DevLin* L3, int epi, const float* x, uint
   if (L.wt && (!L3 || L3->wt)) {
     g.wt = L.wt;
     g.wt3 = L3 ? L3->wt : nullptr;
+    g.ws = L.ws;
+    g.ws3 = L3 ? L3->ws : nullptr;
   }
   g.row_bytes = L.row_bytes;
   g.M = L.out;
@@ -1290,35 +1300,64 @@ void Engine::repack(DevLin& L) {
 }
 
 void Engine::tile(DevLin& L, uint32_t rows, uint32_t row_base, uint32_t extra_row) {
-  if (L.type != W_F16 || L.in % 256 || L.in > BMM_MAX_K || L.wt) return;
-  L.wt = dalloc<_Float16>(size_t(bmm_rows_pad(rows)) * L.in);
-  HIPC(launch_tile_f16(reinterpret_cast<const uint16_t*>(L.w), L.in, rows, row_base, extra_row,
-                       reinterpret_cast<uint16_t*>(L.wt), stream_));
+  if (L.in % 32 || L.wt) return;
+  const size_t elems = size_t(bmm_rows_pad(rows)) * L.in;
+  if (L.type == W_F16) {
+    L.wt = try_dalloc(elems * 2);
+    if (L.wt)
+      HIPC(launch_tile_f16(reinterpret_cast<const uint16_t*>(L.w), L.in, rows, row_base, extra_row,
+                           reinterpret_cast<uint16_t*>(L.wt), stream_));
+    return;
+  }
+  if (!tile_q_bytes(L.type) || row_base || extra_row != NO_ROW) return;
+  // the values and, 16-byte aligned behind them, the scales
+  const size_t vals = elems / 512 * tile_q_bytes(L.type);
+  uint8_t* w = try_dalloc(vals + elems / 32 * 2);
+  if (!w) return;
+  L.ws = reinterpret_cast<uint16_t*>(w + vals);
+  HIPC(launch_tile_q(L.w, L.row_bytes, L.type, L.in, rows, w, L.ws, stream_));
+  L.wt = w;
 }
 
-// The batched product's copies of the F16 linears and the repacked Q8_0 /
-// Q4_0 linears of the one-column GEMV (one more HBM copy of the weights),
-// built once, the first time a decode needs them.
+// Device memory for a copy that only speeds later calls up: null when there is
+// none left (the products then read the rows themselves).
+uint8_t* Engine::try_dalloc(size_t bytes) {
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  count_device_alloc();
+  allocs_.push_back(p);
+  return static_cast<uint8_t*>(p);
+}
+
+// The batched and prefill products' copies of the linears (one more HBM copy
+// of the weights), built once, the first time a call needs them.
 void Engine::ensure_tiled() {
   if (tiled_) return;
+  if (bmm_min_cols_) {
+    for (auto& L : slow_)
+      for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) tile(*d, d->out, 0, NO_ROW);
+    for (auto& L : fast_)
+      for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) tile(*d, d->out, 0, NO_ROW);
+    tile(fast_out_, fast_out_.out, 0, NO_ROW);
+    tile(head_cand_, n_cand_, spec.semantic_begin, head_extra_);
+    HIPC(hipStreamSynchronize(stream_));
+  }
+  tiled_ = true;
+}
+
+// The Q8_0 / Q4_0 linears repacked for the one-column decode GEMV, likewise.
+void Engine::ensure_repacked() {
+  if (repacked_) return;
   for (auto& L : slow_)
     for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) repack(*d);
   for (auto& L : fast_)
     for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) repack(*d);
   repack(fast_out_);
-  if (!bmm_min_cols_) {
-    HIPC(hipStreamSynchronize(stream_));
-    tiled_ = true;
-    return;
-  }
-  for (auto& L : slow_)
-    for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) tile(*d, d->out, 0, NO_ROW);
-  for (auto& L : fast_)
-    for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) tile(*d, d->out, 0, NO_ROW);
-  tile(fast_out_, fast_out_.out, 0, NO_ROW);
-  tile(head_cand_, n_cand_, spec.semantic_begin, head_extra_);
   HIPC(hipStreamSynchronize(stream_));
-  tiled_ = true;
+  repacked_ = true;
 }
 
 void Engine::check_state_err(uint32_t nseq) {
@@ -1489,6 +1528,7 @@ void Engine::generate(uint32_t nseq, const int32_t* const* prompts, const size_t
   const size_t ncodes = size_t(s.num_codebooks) * p.max_new_tokens;
   ensure_slots(nseq);
   ensure_tiled();
+  ensure_repacked();
   ensure_fast_table();
   ensure_codes(ncodes * nseq);
   ensure_prompt(total_cols * cdim);
@@ -1705,7 +1745,7 @@ struct TmpBuf {
 void Engine::ensure_fast_table() {
   const s2hip_spec& s = spec;
   if (fast_table_ || fast_table_off_ || s.fast_layers == 0) return;
-  ensure_tiled();  // the repacked rows decide which one-column kernel the linear takes
+  ensure_repacked();  // the repacked rows decide which one-column kernel the linear takes
   const DevLin& L = fast_[0].wqkv;
   const uint32_t w = (s.fast_heads + 2 * s.fast_kv_heads) * s.fast_head_dim;
   float* tab = dalloc<float>(size_t(s.codebook_size) * w);
@@ -1736,11 +1776,17 @@ void Engine::op_linear(const void* w, uint32_t type, size_t in, size_t out, cons
   L.out = uint32_t(out);
   L.row_bytes = rb;
   const bool batched = bmm_min_cols_ && ncol >= bmm_min_cols_ && in % 256 == 0 && in <= BMM_MAX_K;
-  if (batched && type == W_F16) {  // batched-decode product on a tiled copy
-    TmpBuf dt(size_t(bmm_rows_pad(uint32_t(out))) * in * 2), derr(4);
-    L.wt = dt.as<_Float16>();
-    HIPC(launch_tile_f16(reinterpret_cast<const uint16_t*>(L.w), uint32_t(in), uint32_t(out), 0, NO_ROW,
-                         reinterpret_cast<uint16_t*>(L.wt), stream_));
+  if (batched && (type == W_F16 || ncol >= 3)) {  // batched-decode product on a tiled copy
+    const size_t elems = size_t(bmm_rows_pad(uint32_t(out))) * in;
+    const size_t vals = type == W_F16 ? elems * 2 : elems / 512 * tile_q_bytes(type);
+    TmpBuf dt(vals + elems / 32 * 2), derr(4);
+    L.wt = dt.as<uint8_t>();
+    L.ws = reinterpret_cast<uint16_t*>(L.wt + vals);
+    if (type == W_F16)
+      HIPC(launch_tile_f16(reinterpret_cast<const uint16_t*>(L.w), uint32_t(in), uint32_t(out), 0, NO_ROW,
+                           reinterpret_cast<uint16_t*>(L.wt), stream_));
+    else
+      HIPC(launch_tile_q(L.w, rb, type, uint32_t(in), uint32_t(out), L.wt, L.ws, stream_));
     HIPC(hipMemsetAsync(derr.p, 0, 4, stream_));
     bmm(L, nullptr, EPI_STORE, uint32_t(ncol), dx.as<float>(), uint32_t(in), nullptr, 0.0f, dy.as<float>(),
         uint32_t(out), nullptr, derr.as<uint32_t>());
@@ -1764,7 +1810,7 @@ void Engine::op_linear(const void* w, uint32_t type, size_t in, size_t out, cons
     L.qs = dsc->as<uint16_t>();
     HIPC(launch_repack_q(L.w, rb, type, uint32_t(in), uint32_t(out), L.qp, L.qs, stream_));
   }
-  if (ncol >= 3 && ncol <= 16 && in % 256 == 0)  // batched-decode product (quantized rows)
+  if (ncol >= 3 && ncol <= 16 && in % 256 == 0)  // the whole-row-scale product
     mm_skinny(L, nullptr, EPI_STORE, dx.as<float>(), uint32_t(in), nullptr, 0.0f, uint32_t(ncol), dy.as<float>(),
               uint32_t(out), 0, NO_ROW, uint32_t(out), nullptr);
   else
@@ -2074,7 +2120,7 @@ void Engine::time_kernel(const std::string& full_name, uint32_t reps, double* av
     } else if (force == 'g') {
       gemv(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, 0, NO_ROW, L.out, nullptr);
     } else if (force == 't') {
-      if (!L.wt) fail("no batched-product copy of this matrix (F16 with in % 256 == 0 only)");
+      if (!L.wt || L.in % 256) fail("no batched-product copy of this matrix (in % 256 == 0 only)");
       bmm(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, nullptr, &st_->err, waves);
     } else {
       lin(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, 0, NO_ROW, L.out, nullptr);

@@ -304,13 +304,15 @@ hipError_t launch_split_rows(const float* x, uint32_t ldx, const float* norm, fl
 // x given as the split planes; epilogues as for launch_gemv (SwiGLU uses w3).
 // part (nullable): workspace of part_cap floats for K-split partial sums
 // (gemm_part_floats(Npad, M) floats lets every short-M product split as it would).
-// F16 weights: wt (and wt3) in the fragment order of launch_tile_f16, or null
-// and the rows themselves.
+// wt (and wt3): the weights in the fragment order of launch_tile_f16 /
+// launch_tile_q (then with the scales ws, ws3), or null and the rows themselves.
 struct GemmArgs {
   const uint8_t* w;
   const uint8_t* w3;
-  const _Float16* wt;
-  const _Float16* wt3;
+  const uint8_t* wt;
+  const uint8_t* wt3;
+  const uint16_t* ws;
+  const uint16_t* ws3;
   size_t row_bytes;
   uint32_t M, K;
   const _Float16* xh;
@@ -352,14 +354,22 @@ hipError_t launch_skinny_mfma(uint32_t wtype, int epi, const SkinnyArgs& a, hipS
 uint32_t bmm_rows_pad(uint32_t m);
 hipError_t launch_tile_f16(const uint16_t* src, uint32_t K, uint32_t M, uint32_t row_base, uint32_t extra_row,
                            uint16_t* dst, hipStream_t s);
+// Q8_0 / Q4_0 rows in the same order: tiles of tile_q_bytes(wtype) bytes of
+// integer values and [tile][16] f16 row scales (K % 32 == 0).
+uint32_t tile_q_bytes(uint32_t wtype);
+hipError_t launch_tile_q(const uint8_t* src, size_t row_bytes, uint32_t wtype, uint32_t K, uint32_t M, uint8_t* dst,
+                         uint16_t* scales, hipStream_t s);
 // y[n][m] (op)= sum_k W[m][k] xn[n][k] for n < N <= 16, m < M; xn = x, or
 // RMSNorm(x) with gain `norm`; epilogues as for launch_gemv.  K % 256 == 0.
 // Each wave scales each column by a power of two from its first activations
 // (any magnitude keeps ~2^-22 relative accuracy); a non-finite activation,
 // or one 2^15 times larger than those, sets ERR_F16_RANGE in *err.
 struct BmmArgs {
-  const _Float16* wt;
-  const _Float16* wt3;   // second matrix for SwiGLU epilogues
+  const void* wt;        // fragment-ordered tiles of type wtype
+  const void* wt3;       // second matrix for SwiGLU epilogues
+  const uint16_t* ws;    // Q8_0 / Q4_0: the tiles' scales
+  const uint16_t* ws3;
+  uint32_t wtype;
   uint32_t M, K;
   const float* x;        // [N][ldx]
   uint32_t ldx, N;

@@ -21,6 +21,7 @@
 
 #include "expf_glibc.h"
 #include "kernels.h"
+#include "qfrag.h"
 #include "wave.h"
 
 namespace s2 {
@@ -231,7 +232,9 @@ __device__ __forceinline__ void weight8(const uint8_t* row, uint32_t e, half8& h
 }
 
 // ---------------------------------------------------------------------------
-// MFMA GEMM  Y[n][m] (op)= rs[n] * sum_k W[m][k] * X[n][k]
+// MFMA GEMM  Y[n][m] (op)= rs[n] * sum_k W[m][k] * X[n][k]  over weight rows as
+// they are in the file (products without a fragment-ordered copy: no memory
+// left for it; those with one take the DMA kernels below)
 //   Block tile: 128 weight rows x 128 tokens, 4 waves in 2 x 2, each wave
 //   64 rows x 64 tokens = 2 x 2 tiles of v_mfma_f32_32x32x16_f16 with the
 //   token fragment as A and the weight fragment as B, so a lane's results
@@ -471,6 +474,54 @@ __device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint32_
 // drained if `lgkm0`
 constexpr int wait_imm(int v, bool lgkm0) { return (v & 15) | ((v >> 4) << 14) | 0x70 | (lgkm0 ? 0 : 0xF00); }
 
+// Stores of a wave's 32 TMW weight slots x 32 TNW tokens from slot m_base
+// (SwiGLU: output m_base) and token n_base on:
+//   acc[i][j][v] = D[token 8 (v / 4) + 4 (lane / 32) + v % 4][weight slot lane % 32]
+template <int EPI, int TMW, int TNW>
+__device__ __forceinline__ void gemm_store(const GemmArgs& a, const floatx16 (&acc)[TNW][TMW], uint32_t n_base,
+                                           uint32_t m_base, uint32_t sp, uint32_t splits, uint32_t lane) {
+  constexpr bool DUAL = DUAL_EPI(EPI);
+  const uint32_t fr = lane & 31u;
+#pragma unroll
+  for (int i = 0; i < TNW; ++i) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const uint32_t n = n_base + 32u * i + 8u * (v / 4) + 4u * (lane >> 5) + (v % 4);
+      if (n >= a.N) continue;
+      const float r = splits > 1 ? 1.0f : a.rs[n];
+      if constexpr (DUAL) {
+#pragma unroll
+        for (int j = 0; j < TMW; j += 2) {
+          const uint32_t m = m_base + 16u * j + fr;
+          if (m >= a.M) continue;
+          const float g = acc[i][j][v] * r, u = acc[i][j + 1][v] * r;
+          float* dst = a.y + size_t(n) * a.ldy + m;
+          if constexpr (EPI == EPI_SWIGLU_SLOW) {
+            const float sig = __fdiv_rn(1.0f, __fadd_rn(1.0f, expf_glibc(-g)));
+            *dst = __fmul_rn(__fmul_rn(g, sig), u);
+          } else {
+            *dst = __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, expf_glibc(-g))), u);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < TMW; ++j) {
+          const uint32_t m = m_base + 32u * j + fr;
+          if (m >= a.M) continue;
+          if (splits > 1) {
+            a.part[(size_t(sp) * a.N + n) * a.M + m] = acc[i][j][v];
+          } else {
+            const float g = acc[i][j][v] * r;
+            float* dst = a.y + size_t(n) * a.ldy + m;
+            if constexpr (EPI == EPI_STORE) *dst = g;
+            else *dst = __fadd_rn(*dst, g);
+          }
+        }
+      }
+    }
+  }
+}
+
 template <int EPI, int TMW, int TNW, int NB>
 __global__ __launch_bounds__(256, 2) void gemm_f16_dma_kernel(GemmArgs a, uint32_t m_tiles, uint32_t n_tiles,
                                                               uint32_t splits) {
@@ -505,8 +556,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_dma_kernel(GemmArgs a, uint32
     const uint32_t g = TMW * wave + j;
     // SwiGLU: w1 and w3 rows alternate every 32 slots
     const uint32_t tile = m_base / 16u + (DUAL ? (g >> 2) * 2u + (g & 1u) : g);
-    const _Float16* base = (DUAL && ((g >> 1) & 1u)) ? a.wt3 : a.wt;
-    src[j] = reinterpret_cast<const uint8_t*>(base) + size_t(min(tile, wt_last)) * kt * 1024u;
+    const uint8_t* base = (DUAL && ((g >> 1) & 1u)) ? a.wt3 : a.wt;
+    src[j] = base + size_t(min(tile, wt_last)) * kt * 1024u;
     dst[j] = lds0 + g * 1024u;
   }
 #pragma unroll
@@ -595,45 +646,149 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_dma_kernel(GemmArgs a, uint32
 #pragma unroll
       for (int j = 0; j < TMW; ++j) acc[i][j] += accp[LP - 1][i][j];
   }
-  // acc[i][j][v] = D[token 8 (v / 4) + 4 (lane / 32) + v % 4][weight slot lane % 32]
+  gemm_store<EPI, TMW, TNW>(a, acc, n_base + 32u * TNW * wn, m_base + (DUAL ? 16u : 32u) * TMW * wm, sp, splits, lane);
+}
+
+// ---------------------------------------------------------------------------
+// Q8_0 / Q4_0 weights in fragment order: the tiles and the pipeline of the F16
+// product, the weights staged as the integers they are.  A wave turns its
+// fragments into f16 (exact) as it reads them; the 4 MFMAs of a block of 32 k
+// (two halves, hi and lo) start from zero and their sum, times the block's
+// scale, is added to the accumulator: one FMA per result and block in place of
+// the third product that a hi + lo split of the dequantised weights needs, and
+// a quarter or an eighth of its weight bytes.  Q8_0 w1/w3 of 389 tokens 264 ->
+// 129 us, w2 117 -> 52 (the row-major kernel dequantised and split each weight
+// while staging it), and the sums are nearer to 64-bit ones (4.8e-6 -> 2.6e-6
+// over a whole prompt): one rounding per block instead of six.  One barrier per stage; the other
+// block of the CU multiplies while this one reads.
+// ---------------------------------------------------------------------------
+// One LDS-DMA load with an address per lane (W bytes: 16 or 4 per lane).
+template <int W>
+__device__ __forceinline__ void dma_lane(const uint8_t* src, uint32_t lds) {
+  if constexpr (W == 16)
+    asm volatile("s_nop 1\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
+  else
+    asm volatile("s_nop 1\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
+}
+
+template <uint32_t WT, int EPI, int TMW, int TNW, int NB>
+__global__ __launch_bounds__(256, 2) void gemm_q_dma_kernel(GemmArgs a, uint32_t m_tiles, uint32_t n_tiles,
+                                                            uint32_t splits) {
+  constexpr bool DUAL = DUAL_EPI(EPI);
+  constexpr uint32_t WR = 64 * TMW, XR = 64 * TNW;  // tile rows
+  constexpr uint32_t TB = WT == W_Q8_0 ? 512 : 256;  // bytes of a 16-row weight tile
+  constexpr uint32_t WB = WR / 16 * TB, SB = 512, STAGE = WB + SB + 2 * XR * KS * 2;  // weights, scales, token planes
+  constexpr int PW = WB >= 4096 ? int(WB / 4096) : 1;  // weight loads per wave (2 KiB stages: waves 2, 3 repeat 0, 1)
+  constexpr int PER = PW + 1 + 2 * TNW;
+  extern __shared__ __align__(16) uint8_t gemm_lds[];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
+  const uint32_t wm = wave & 1u, wn = wave >> 1;
+  // tiles to XCDs as in gemm_f16_dma_kernel
+  const uint32_t nb = gridDim.x, xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3, q8 = nb >> 3, r8 = nb & 7u;
+  const uint32_t t = xcd < r8 ? xcd * (q8 + 1u) + slot : r8 * (q8 + 1u) + (xcd - r8) * q8 + slot;
+  const uint32_t nt = uint32_t(__builtin_amdgcn_readfirstlane(int(t % n_tiles))), tr = t / n_tiles;
+  const uint32_t sp = uint32_t(__builtin_amdgcn_readfirstlane(int(tr % splits)));
+  const uint32_t mt = uint32_t(__builtin_amdgcn_readfirstlane(int(tr / splits)));
+  const uint32_t n_base = nt * XR, m_base = mt * (DUAL ? WR / 2 : WR);
+  const uint32_t nst = a.K / KS, st0 = sp * nst / splits, st1 = (sp + 1) * nst / splits;
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(gemm_lds));
+  const uint32_t kt = a.K / KS, wt_last = (a.M + 15u) / 16u - 1u, off = lane * 16u;
+
+  // 16-row tile g of the block: its index and matrix (SwiGLU: w1 and w3 alternate every 32 slots)
+  auto tile_of = [&](uint32_t g) { return min(m_base / 16u + (DUAL ? (g >> 2) * 2u + (g & 1u) : g), wt_last); };
+  // weight load j: the KiB at (PW wave + j) of the stage's WB bytes, each lane's 16 bytes in tile g
+  const uint8_t* wsrc[PW];
+  uint32_t wdst[PW];
 #pragma unroll
-  for (int i = 0; i < TNW; ++i) {
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const uint32_t n = n_base + 32u * (TNW * wn + i) + 8u * (v / 4) + 4u * (lane >> 5) + (v % 4);
-      if (n >= a.N) continue;
-      const float r = splits > 1 ? 1.0f : a.rs[n];
-      if constexpr (DUAL) {
-#pragma unroll
-        for (int j = 0; j < TMW; j += 2) {
-          const uint32_t m = m_base + 16u * (TMW * wm + j) + fr;
-          if (m >= a.M) continue;
-          const float g = acc[i][j][v] * r, u = acc[i][j + 1][v] * r;
-          float* dst = a.y + size_t(n) * a.ldy + m;
-          if constexpr (EPI == EPI_SWIGLU_SLOW) {
-            const float sig = __fdiv_rn(1.0f, __fadd_rn(1.0f, expf_glibc(-g)));
-            *dst = __fmul_rn(__fmul_rn(g, sig), u);
-          } else {
-            *dst = __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, expf_glibc(-g))), u);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < TMW; ++j) {
-          const uint32_t m = m_base + 32u * (TMW * wm + j) + fr;
-          if (m >= a.M) continue;
-          if (splits > 1) {
-            a.part[(size_t(sp) * a.N + n) * a.M + m] = acc[i][j][v];
-          } else {
-            const float g = acc[i][j][v] * r;
-            float* dst = a.y + size_t(n) * a.ldy + m;
-            if constexpr (EPI == EPI_STORE) *dst = g;
-            else *dst = __fadd_rn(*dst, g);
-          }
-        }
-      }
-    }
+  for (int j = 0; j < PW; ++j) {
+    const uint32_t kib = (PW * wave + j) % (WB / 1024u), byte = kib * 1024u + lane * 16u, g = byte / TB;
+    const uint8_t* base = DUAL && ((g >> 1) & 1u) ? a.wt3 : a.wt;
+    wsrc[j] = base + size_t(tile_of(g)) * kt * TB + byte % TB;
+    wdst[j] = lds0 + kib * 1024u;
   }
+  // scales: 8 tiles of 32 bytes per load; with 8 tiles in the stage every wave repeats the same load
+  const uint32_t sg = (wave * 8u) % (WR / 16u) + lane / 8u;
+  const uint8_t* ssrc = reinterpret_cast<const uint8_t*>(DUAL && ((sg >> 1) & 1u) ? a.ws3 : a.ws) +
+                        size_t(tile_of(sg)) * kt * 32u + (lane & 7u) * 4u;
+  const uint32_t sdst = lds0 + WB + (wave * 8u) % (WR / 16u) * 32u;
+  const uint8_t* xsrc[2 * TNW];
+  uint32_t xdst[2 * TNW];
+#pragma unroll
+  for (int j = 0; j < 2 * TNW; ++j) {
+    const uint32_t g = 2u * TNW * wave + j, plane = g / (4u * TNW), tile = n_base / 16u + g % (4u * TNW);
+    xsrc[j] = reinterpret_cast<const uint8_t*>(plane ? a.xl : a.xh) + size_t(tile) * kt * 1024u;
+    xdst[j] = lds0 + WB + SB + g * 1024u;
+  }
+  auto issue = [&](uint32_t st, uint32_t buf) {
+    const uint32_t k = min(st, st1 - 1u);  // past the range: a valid, unused stage
+#pragma unroll
+    for (int j = 0; j < PW; ++j) dma_lane<16>(wsrc[j] + k * TB, wdst[j] + buf);
+    dma_lane<4>(ssrc + k * 32u, sdst + buf);
+#pragma unroll
+    for (int j = 0; j < 2 * TNW; ++j) dma16(xsrc[j] + k * 1024u, off, xdst[j] + buf);
+  };
+
+  const uint32_t fr = lane & 31u;
+  // weight fragment i, half h: 8 values of row fr + 32 i from k 16 h + 8 (lane / 32)
+  const uint32_t wrd = wm * TMW * 2u * TB + (fr >> 4) * TB + ((fr & 15u) + 16u * (lane >> 5)) * (TB / 64u);
+  const uint32_t srd = WB + (wm * 32u * TMW + fr) * 2u;
+  const uint32_t xrd = WB + SB + (wn * 32u * TNW + fr) * 64u + (((lane >> 5) ^ swz(fr)) << 4);
+  floatx16 acc[TNW][TMW];
+#pragma unroll
+  for (int i = 0; i < TNW; ++i)
+#pragma unroll
+    for (int j = 0; j < TMW; ++j) acc[i][j] = floatx16{};
+#pragma unroll
+  for (int b = 0; b < NB - 1; ++b) issue(st0 + b, b * STAGE);
+  uint32_t buf = 0, fill = (NB - 1) * STAGE;
+  for (uint32_t st = st0; st < st1; ++st) {
+    // stage st has landed in every wave, and every wave is done with stage st - 1
+    __builtin_amdgcn_s_waitcnt(wait_imm((NB - 2) * PER, true));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue(st + NB - 1, fill);
+    const uint8_t* B = gemm_lds + buf;
+    half8 x[2][TNW][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < TNW; ++i)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          x[h][i][p] = *reinterpret_cast<const half8*>(B + (xrd ^ (h << 5)) + (p * XR + 32 * i) * 64);
+#pragma unroll
+    for (int j = 0; j < TMW; ++j) {
+      const float d = float(*reinterpret_cast<const _Float16*>(B + srd + 64 * j));
+      floatx16 s[TNW];
+#pragma unroll
+      for (int i = 0; i < TNW; ++i) s[i] = floatx16{};
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        half8 w;
+        const uint8_t* pw = B + wrd + j * 2 * TB + h * (TB / 2);
+        if constexpr (WT == W_Q8_0) {
+          const uint2 r = *reinterpret_cast<const uint2*>(pw);
+          w = q8_frag(r.x, r.y);
+        } else {
+          w = q4_frag(*reinterpret_cast<const uint32_t*>(pw));
+        }
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int i = 0; i < TNW; ++i) s[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[h][i][p], w, s[i], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < TNW; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = fmaf(d, s[i][v], acc[i][j][v]);
+    }
+    buf = buf + STAGE == NB * STAGE ? 0u : buf + STAGE;
+    fill = fill + STAGE == NB * STAGE ? 0u : fill + STAGE;
+  }
+  __builtin_amdgcn_s_waitcnt(wait_imm(0, false));  // the unused tail loads have landed before the block ends
+  gemm_store<EPI, TMW, TNW>(a, acc, n_base + 32u * TNW * wn, m_base + (DUAL ? 16u : 32u) * TMW * wm, sp, splits, lane);
 }
 
 // y[n][m] (op)= rs[n] * (part[0][n][m] + part[1][n][m] + ...), splits added in
@@ -1150,20 +1305,40 @@ static hipError_t gemm_f16_launch(const GemmArgs& a, const GemmPlan& p, hipStrea
                      a, p.m_tiles, p.n_tiles, p.splits);
   return hipGetLastError();
 }
-template <int EPI>
-static hipError_t gemm_f16_tile(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
-  switch (p.tile) {
-    case 0: return gemm_f16_launch<EPI, 2, 1, 4>(a, p, s);
-    case 1: return gemm_f16_launch<EPI, 4, 1, 3>(a, p, s);
-    default: return gemm_f16_launch<EPI, 4, 2, 2>(a, p, s);
+template <uint32_t WT, int EPI, int TMW, int TNW, int NB>
+static hipError_t gemm_q_launch(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
+  constexpr uint32_t lds = NB * (64 * TMW * (WT == W_Q8_0 ? 32 : 16) + 512 + 2 * 64 * TNW * KS * 2);
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_q_dma_kernel<WT, EPI, TMW, TNW, NB>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((gemm_q_dma_kernel<WT, EPI, TMW, TNW, NB>), dim3(p.m_tiles * p.n_tiles * p.splits), dim3(256), lds,
+                     s, a, p.m_tiles, p.n_tiles, p.splits);
+  return hipGetLastError();
+}
+template <uint32_t WT, int EPI>
+static hipError_t gemm_tile(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
+  if constexpr (WT == W_F16) {
+    switch (p.tile) {
+      case 0: return gemm_f16_launch<EPI, 2, 1, 4>(a, p, s);
+      case 1: return gemm_f16_launch<EPI, 4, 1, 3>(a, p, s);
+      default: return gemm_f16_launch<EPI, 4, 2, 2>(a, p, s);
+    }
+  } else {
+    switch (p.tile) {
+      case 0: return gemm_q_launch<WT, EPI, 2, 1, 4>(a, p, s);
+      case 1: return gemm_q_launch<WT, EPI, 4, 1, 4>(a, p, s);
+      default: return gemm_q_launch<WT, EPI, 4, 2, 3>(a, p, s);
+    }
   }
 }
-static hipError_t gemm_f16(int epi, const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
+template <uint32_t WT>
+static hipError_t gemm_dma(int epi, const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
   switch (epi) {
-    case EPI_STORE: return gemm_f16_tile<EPI_STORE>(a, p, s);
-    case EPI_RESID: return gemm_f16_tile<EPI_RESID>(a, p, s);
-    case EPI_SWIGLU_SLOW: return gemm_f16_tile<EPI_SWIGLU_SLOW>(a, p, s);
-    case EPI_SWIGLU_FAST: return gemm_f16_tile<EPI_SWIGLU_FAST>(a, p, s);
+    case EPI_STORE: return gemm_tile<WT, EPI_STORE>(a, p, s);
+    case EPI_RESID: return gemm_tile<WT, EPI_RESID>(a, p, s);
+    case EPI_SWIGLU_SLOW: return gemm_tile<WT, EPI_SWIGLU_SLOW>(a, p, s);
+    case EPI_SWIGLU_FAST: return gemm_tile<WT, EPI_SWIGLU_FAST>(a, p, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1215,10 +1390,13 @@ hipError_t launch_gemm_mfma(uint32_t wtype, int epi, const GemmArgs& a, hipStrea
   if (a.K % KS || a.M == 0 || a.N == 0) return hipErrorInvalidValue;
   const bool dual = epi == EPI_SWIGLU_SLOW || epi == EPI_SWIGLU_FAST;
   if (dual && !a.w3) return hipErrorInvalidValue;
-  if (wtype == W_F16 && a.wt) {
-    if (dual && !a.wt3) return hipErrorInvalidValue;
+  if (a.wt) {
+    if ((dual && !a.wt3) || (wtype != W_F16 && (!a.ws || (dual && !a.ws3)))) return hipErrorInvalidValue;
     const GemmPlan p = gemm_plan(a, dual);
-    const hipError_t e = gemm_f16(epi, a, p, s);
+    const hipError_t e = wtype == W_F16    ? gemm_dma<W_F16>(epi, a, p, s)
+                         : wtype == W_Q8_0 ? gemm_dma<W_Q8_0>(epi, a, p, s)
+                         : wtype == W_Q4_0 ? gemm_dma<W_Q4_0>(epi, a, p, s)
+                                           : hipErrorInvalidValue;
     return e != hipSuccess || p.splits == 1 ? e : gemm_reduce(epi, a, p.splits, s);
   }
   const uint32_t m_tiles = dual ? (a.M + 63u) / 64u : (a.M + TM - 1u) / TM;
