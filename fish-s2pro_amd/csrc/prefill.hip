@@ -1258,6 +1258,10 @@ constexpr int GEMM_DEPTH = 2;
 // split 14.4 : 18.4 : -, 33.0 : 31.0 : 36, 54.3 : 52.9 : 54.0, - : 144 : 133.
 // (The 128 x 128 tile of 64 x 64 waves with row-major operands took 95 us for
 // w1/w3 at 256 tokens and 153 at 512.)
+// Quantized weights leave the small tile three blocks per CU, which hide each
+// other's unpacking: rounds of 768 blocks of 128 x 64 (Q8_0, 389 tokens: wqkv
+// 76 -> 45 us against both tiles over rounds of 256, w2 and wo together 105 ->
+// 96; Q4_0, 150 tokens: w1/w3 82 -> 59, wqkv 43 -> 24).
 // Long rows are split at least so often that no running sum gets longer than
 // it was before these tiles: 2560 wide with the lo products apart (64-token
 // tiles), 1280 where they share the accumulator, at most four.
@@ -1266,12 +1270,12 @@ struct GemmPlan {
   uint32_t tile;  // 0: 128 x 64, 1: 256 x 64, 2: 256 x 128
   uint32_t m_tiles, n_tiles, splits;
 };
-static GemmPlan gemm_plan(const GemmArgs& a, bool dual) {
+static GemmPlan gemm_plan(const GemmArgs& a, bool dual, bool quant) {
   GemmPlan best{};
   float best_score = -1.0f;
   const bool wide = a.N > GEMM_WIDE_N;
-  const uint32_t slots = wide ? 512u : 256u;
-  for (uint32_t tile = wide ? 1u : 0u; tile < (wide ? 3u : 2u); ++tile) {
+  const uint32_t slots = wide ? 512u : quant ? 768u : 256u;
+  for (uint32_t tile = wide ? 1u : 0u; tile < (wide ? 3u : quant ? 1u : 2u); ++tile) {
     const uint32_t wr = (tile ? 256u : 128u) / (dual ? 2u : 1u), xr = tile == 2u ? 128u : 64u;
     GemmPlan p{tile, (a.M + wr - 1) / wr, (a.N + xr - 1) / xr, 1u};
     const uint32_t most = dual || !a.part || a.M % 4u ? 1u : GEMM_MAX_SPLITS;
@@ -1392,7 +1396,7 @@ hipError_t launch_gemm_mfma(uint32_t wtype, int epi, const GemmArgs& a, hipStrea
   if (dual && !a.w3) return hipErrorInvalidValue;
   if (a.wt) {
     if ((dual && !a.wt3) || (wtype != W_F16 && (!a.ws || (dual && !a.ws3)))) return hipErrorInvalidValue;
-    const GemmPlan p = gemm_plan(a, dual);
+    const GemmPlan p = gemm_plan(a, dual, wtype != W_F16);
     const hipError_t e = wtype == W_F16    ? gemm_dma<W_F16>(epi, a, p, s)
                          : wtype == W_Q8_0 ? gemm_dma<W_Q8_0>(epi, a, p, s)
                          : wtype == W_Q4_0 ? gemm_dma<W_Q4_0>(epi, a, p, s)
