@@ -48,7 +48,7 @@ void count_device_alloc() { g_device_allocs.fetch_add(1, std::memory_order_relax
 
 [[noreturn]] void fail(const std::string& m) { throw std::runtime_error(m); }
 
-constexpr uint32_t PREFILL_COLS = 4;     // decode-path columns per pass of the GEMV prefill
+constexpr uint32_t PREFILL_COLS = 4;     // most columns of one sequence per pass of the decode kernels
 constexpr uint32_t MAX_SEQS = 16;        // requests per batched generate call
 constexpr uint32_t BMM_MAX_K = 10240;    // input width limit of the batched product
 constexpr uint32_t ACT_COLS = 2 * MAX_SEQS;  // activation columns (Fast-AR pass 0 has two per request)
@@ -248,6 +248,7 @@ class Engine {
   DevLin head_full_, fast_out_;
   DevLin head_cand_;  // the candidate rows of the head (tiled copy only)
   bool tiled_ = false, repacked_ = false;
+  uint32_t* lin_err_ = nullptr;  // error word of the linears (null: slot 0's)
   uint32_t bmm_min_cols_ = 2;  // columns from which F16 linears use the batched product
   // Set while a call is re-run after ERR_F16_RANGE: every multi-column linear
   // then takes the per-column paths (two-column GEMV, or the skinny product
@@ -730,7 +731,7 @@ void Engine::lin(const DevLin& L, const DevLin* L3, int epi, uint32_t ncol, cons
     return;
   }
   if (uses_bmm(L, L3, ncol)) {
-    bmm(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, done, &st_->err, bmm_waves);
+    bmm(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, done, lin_err_ ? lin_err_ : &st_->err, bmm_waves);
     return;
   }
   if (ncol <= 2 || L.in % 256) {
@@ -1106,7 +1107,8 @@ void Engine::mm(const DevLin& L, const DevLin* L3, int epi, const float* x, uint
 void Engine::mm_skinny(const DevLin& L, const DevLin* L3, int epi, const float* x, uint32_t ldx, const float* norm,
                        float eps, uint32_t n, float* y, uint32_t ldy, uint32_t row_base, uint32_t extra_row,
                        uint32_t out_rows, const uint32_t* done) {
-  HIPC(launch_split_rows(x, ldx, norm, eps, n, 16, L.in, pxh_, pxl_, prs_, &st_->err, stream_));
+  HIPC(launch_split_rows(x, ldx, norm, eps, n, 16, L.in, pxh_, pxl_, prs_,
+                         lin_err_ ? lin_err_ : &st_->err, stream_));
   SkinnyArgs g{};
   g.w = L.w;
   g.w3 = L3 ? L3->w : nullptr;
@@ -1409,19 +1411,42 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
          " max_seq_len=" + std::to_string(s.max_seq_len));
   validate_tokens(flat, n_tok);
   ensure_slots(slot + 1);
-  ensure_tiled();
+  // a few tokens: the decode kernels (a product's 64-token tile would stand
+  // nearly empty).  Beyond the batched product's range (three and four
+  // tokens), the call runs again on the prefill products.
+  bool few = n_tok <= PREFILL_COLS;
+  if (few && n_tok <= 2) ensure_repacked();
+  else ensure_tiled();
   ensure_prompt(n_tok * cdim);
   HIPC(hipMemcpyAsync(prompt_dev_, flat, n_tok * cdim * 4, hipMemcpyHostToDevice, stream_));
-  // done = 0, err = 0 (eval never runs under a finished frame loop)
-  HIPC(hipMemsetAsync(&st_[slot].done, 0, sizeof(uint32_t), stream_));
-  HIPC(hipMemsetAsync(&st_[slot].err, 0, sizeof(uint32_t), stream_));
-  enqueue_prefill(prompt_dev_, n_tok, slot);
-  enqueue_head(1, hn_, logits_c_, logits_out != nullptr, nullptr);
-  HIPC(hipMemcpyAsync(hidden_out, hn_, s.dim * 4, hipMemcpyDeviceToHost, stream_));
-  if (logits_out) HIPC(hipMemcpyAsync(logits_out, logits_full_, size_t(s.vocab) * 4, hipMemcpyDeviceToHost, stream_));
-  HIPC(hipMemcpyAsync(st_host_ + slot, st_ + slot, sizeof(DevState), hipMemcpyDeviceToHost, stream_));
-  HIPC(hipStreamSynchronize(stream_));
-  const uint32_t e = st_host_[slot].err;
+  uint32_t e = 0;
+  for (;;) {
+    // done = 0, err = 0 (eval never runs under a finished frame loop)
+    HIPC(hipMemsetAsync(&st_[slot].done, 0, sizeof(uint32_t), stream_));
+    HIPC(hipMemsetAsync(&st_[slot].err, 0, sizeof(uint32_t), stream_));
+    if (few || prefill_gemv_) {
+      lin_err_ = &st_[slot].err;
+      enqueue_prefill_gemv(prompt_dev_, n_tok, slot);
+      lin_err_ = nullptr;
+    } else {
+      enqueue_prefill(prompt_dev_, n_tok, slot);
+    }
+    enqueue_head(1, hn_, logits_c_, logits_out != nullptr, nullptr);
+    HIPC(hipMemcpyAsync(hidden_out, hn_, s.dim * 4, hipMemcpyDeviceToHost, stream_));
+    if (logits_out) HIPC(hipMemcpyAsync(logits_out, logits_full_, size_t(s.vocab) * 4, hipMemcpyDeviceToHost, stream_));
+    HIPC(hipMemcpyAsync(st_host_ + slot, st_ + slot, sizeof(DevState), hipMemcpyDeviceToHost, stream_));
+    HIPC(hipStreamSynchronize(stream_));
+    e = st_host_[slot].err;
+    if (!few) break;
+    if (!(e & ERR_F16_RANGE)) {
+      for (uint32_t i = 0; i < s.dim; ++i)
+        if (!std::isfinite(hidden_out[i])) e |= ERR_F16_RANGE;
+      break;
+    }
+    few = false;
+    ensure_tiled();
+    HIPC(hipMemcpyAsync(&st_[slot].n_past, &n_past_host[slot], sizeof(uint32_t), hipMemcpyHostToDevice, stream_));
+  }
   if (e & ERR_TOKEN_RANGE) fail("token id out of range");
   if (e & ERR_KV_OVERFLOW) fail("KV cache overflow");
   if (e & ERR_F16_RANGE) fail("activation not finite or beyond the range of the batched product");

@@ -24,7 +24,7 @@ def _rel(a, b):
 
 
 @pytest.mark.parametrize("weights", sorted(TYPES))
-@pytest.mark.parametrize("ffn,lengths", [(1536, (3, 16, 17, 63, 65, 129, 257, 770, 2100)), (1504, (5, 33, 300))])
+@pytest.mark.parametrize("ffn,lengths", [(1536, (1, 2, 3, 4, 5, 17, 63, 65, 129, 257, 770, 2100)), (1504, (5, 33, 300))])
 def test_prefill_lengths_match_oracle(model_dir, weights, ffn, lengths):
     from s2hip import Engine
 
@@ -40,3 +40,27 @@ def test_prefill_lengths_match_oracle(model_dir, weights, ffn, lengths):
             ho, lo = o.eval(prompt)
             assert e.n_past == n
             assert _rel(hg, ho) < 1e-4 and _rel(lg, lo) < 1e-4, (n, _rel(hg, ho), _rel(lg, lo))
+
+
+def test_short_eval_beyond_the_batched_range(model_dir, tmp_path):
+    """Three tokens take the batched decode product; an FFN channel far above the
+    first 256 of its row (past the product's per-wave headroom) makes the call
+    run again on the prefill products, in KV slot 1 and at a later position."""
+    import shutil
+
+    import gguf_util
+    from s2hip import Engine
+
+    path = str(tmp_path / "outlier.gguf")
+    shutil.copyfile(synth.ensure_gguf(synth.TINY, model_dir), path)
+    for l in range(synth.TINY.slow_layers):
+        for w in ("w1", "w3"):
+            gguf_util.scale_rows(path, f"layers.{l}.feed_forward.{w}.weight", [300], 300.0)
+    o = O.OracleModel(path, 64, synth.TINY.im_end_id)
+    with Engine(path, 64, synth.TINY.im_end_id) as e:
+        for n, seed in ((2, 1), (3, 2), (1, 3), (4, 4)):
+            prompt = make_prompt(synth.TINY, n, seed=seed)
+            hg, lg = e.eval_slot(1, prompt)
+            ho, lo = o.eval(prompt)
+            assert _rel(hg, ho) < 1e-4 and _rel(lg, lo) < 1e-4, n
+        assert e.n_past_slot(1) == o.n_past == 10 and e.n_past == 0
