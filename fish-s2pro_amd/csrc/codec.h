@@ -9,10 +9,18 @@
 
 namespace s2 {
 
+// f16 activation planes [frame][channel] are stored in tiles of 16 frames x 32
+// channels (1 KiB; act_off in codec.hip): frame tile by frame tile, and in it
+// channel tile by channel tile.  Before frame 0 a plane holds ACT_GUARD zero
+// frames (the causal padding; tile-aligned), behind its last frame at least
+// ACT_TAIL frames of 4096 channels of any content (read and written for the
+// last frame tile's missing frames, never used); so do the f32 outputs.
+constexpr int32_t ACT_GUARD = 64, ACT_TAIL = 256;
+
 // Implicit-GEMM convolution on MFMA (v_mfma_f32_32x32x16_f16):
 //   y[f * ostride + phase][m] = epilogue( sum_g sum_c A[f + off0 + g * ostep][c] * W[phase][m][g][c] )
-// for frames f < F and output channels m < M.  A rows outside [0, F) are
-// zero (causal left padding).  A is one f16 plane (conv inputs, which the
+// for frames f < F and output channels m < M; taps reach back only, at most
+// ACT_GUARD frames.  A is one f16 plane (conv inputs, which the
 // reference rounds to f16) or two planes hi + lo with hi = f16(x),
 // lo = f16(x - hi), whose products sum to the f32 input's product within
 // ~2^-22 relative (transposed-conv and pointwise inputs, f32 in the
@@ -23,8 +31,7 @@ namespace s2 {
 struct ConvGemmArgs {
   const _Float16* xh;
   const _Float16* xl;  // null: one plane
-  uint32_t ldx;        // elements per input row
-  uint32_t C;          // input channels (a multiple of the stage width, 16 or 32)
+  uint32_t C;          // input channels (a multiple of 32)
   uint32_t F;          // frames per phase (input frames)
   uint32_t G;          // taps
   int32_t off0, ostep; // tap g reads input frame f + off0 + g * ostep
@@ -41,14 +48,13 @@ struct ConvGemmArgs {
   const float* alpha;
   _Float16* yh;
   _Float16* yl;
-  uint32_t ldh;
   // K split (nullable): when a launch would leave CUs idle, splits of the
   // input-channel stages write partial sums to part ([split][row][M] f32,
   // part_cap floats) and a reduce kernel adds them in split order and
   // applies the epilogue
   float* part;
   size_t part_cap;
-  // Fused residual unit (M <= 128, one m tile): the product above is the unit's
+  // Fused residual unit (one m tile): the product above is the unit's
   // k7 conv; Y = f16(snake(acc + bias_mid, alpha_mid)) goes to LDS and acc =
   // Y . W1 (the unit's k1 conv, w1 packed like any k1 conv of M channels)
   // before the epilogue, which then uses bias (the k1 conv's) onwards.
@@ -57,34 +63,34 @@ struct ConvGemmArgs {
   const float* alpha_mid;
 };
 
-// Tile geometry of a packed weight: TM = 32 * mc output channels per tile,
-// kc input channels per stage.
-struct ConvTile {
-  uint32_t mc, kc;
-};
-ConvTile conv_tile(uint32_t M, uint32_t G, bool split);
+// Output channels per weight tile.
+uint32_t conv_tile_rows(uint32_t M);
 // Packs W(phase, m, g, c) = src(phase, m, g, c) into the layout the kernel
-// streams: [phase][m_tile][c / kc][g][TM][kc], zero rows for m >= M.
-// Host side; returns halfs written (phases * m_tiles * TM * G * C).
-size_t conv_packed_halfs(uint32_t phases, uint32_t M, uint32_t G, uint32_t C, ConvTile t);
+// streams: [phase][m tile][c / 32][g][rows / 16] tiles of 16 rows x 32
+// channels in MFMA fragment order (lane l's 8 halfs: row l % 16, channels 8
+// (l / 16) ..), zero rows for m >= M.
+// Host side; returns halfs written (phases * m_tiles * tile rows * G * C).
+size_t conv_packed_halfs(uint32_t phases, uint32_t M, uint32_t G, uint32_t C);
 template <class Src>
-void pack_conv_weights(uint16_t* dst, uint32_t phases, uint32_t M, uint32_t G, uint32_t C, ConvTile t, Src src) {
-  const uint32_t TM = 32 * t.mc, mt = (M + TM - 1) / TM, nch = C / t.kc;
+void pack_conv_weights(uint16_t* dst, uint32_t phases, uint32_t M, uint32_t G, uint32_t C, Src src) {
+  const uint32_t MT = conv_tile_rows(M), mt = (M + MT - 1) / MT, nch = C / 32;
   size_t o = 0;
   for (uint32_t p = 0; p < phases; ++p)
     for (uint32_t ti = 0; ti < mt; ++ti)
       for (uint32_t ch = 0; ch < nch; ++ch)
         for (uint32_t g = 0; g < G; ++g)
-          for (uint32_t r = 0; r < TM; ++r)
-            for (uint32_t k = 0; k < t.kc; ++k) {
-              const uint32_t m = ti * TM + r;
-              dst[o++] = m < M ? src(p, m, g, ch * t.kc + k) : uint16_t(0);
-            }
+          for (uint32_t r = 0; r < MT; r += 16)
+            for (uint32_t l = 0; l < 64; ++l)
+              for (uint32_t k = 0; k < 8; ++k) {
+                const uint32_t m = ti * MT + r + l % 16;
+                dst[o++] = m < M ? src(p, m, g, ch * 32 + 8 * (l / 16) + k) : uint16_t(0);
+              }
 }
-hipError_t launch_conv_gemm(const ConvGemmArgs& a, uint32_t phases, ConvTile t, hipStream_t s);
-// The residual unit's k7 conv + snake + k1 conv in one launch (a.w1 set; M a
-// multiple of 32, at most 128; tile t of the k7 conv).
-hipError_t launch_residual_unit(const ConvGemmArgs& a, ConvTile t, hipStream_t s);
+hipError_t launch_conv_gemm(const ConvGemmArgs& a, uint32_t phases, hipStream_t s);
+// The residual unit's k7 conv + snake + k1 conv in one launch (a.w1 set), for
+// channel counts that one block holds.
+bool residual_unit_fits(uint32_t M);
+hipError_t launch_residual_unit(const ConvGemmArgs& a, hipStream_t s);
 
 // rvq_lookup_codes: latents[f][o] = sum over codebooks q (in order) of
 // (codebook_q[code] . proj_w_q[o] + proj_b_q[o]); codes codebook-major
@@ -113,8 +119,8 @@ hipError_t launch_codec_attention(const float* qkv, uint32_t T, float* out, hipS
 hipError_t launch_codec_scaled_residual(float* x, const float* p, const float* scale, uint32_t T, uint32_t D,
                                         hipStream_t s);
 
-// hi = f16(x), lo = f16(x - hi) over n elements
-hipError_t launch_codec_split16(const float* x, _Float16* hi, _Float16* lo, size_t n, hipStream_t s);
+// x [frames][C] -> planes hi = f16(x) and, unless null, lo = f16(x - hi)
+hipError_t launch_codec_split16(const float* x, _Float16* hi, _Float16* lo, size_t frames, uint32_t C, hipStream_t s);
 
 // ConvNeXt front: depthwise causal conv (k 7) + LayerNorm (eps) per frame of
 // 1024 channels, output as hi / lo planes.  w: [1024][7] f32.

@@ -2,19 +2,30 @@
 //
 // The decoder's convolutions (causal conv1d, transposed conv1d, pointwise
 // linears) all run on one implicit-GEMM MFMA kernel, conv_gemm_kernel:
-//   * block tile: 256 frames x TM = 32 * MC output channels, 4 waves each
-//     holding 64 frames x TM channels (2 x MC tiles of v_mfma_f32_32x32x16_f16,
-//     frames as the A operand, weights as B, so the 32 lanes of a row group
-//     store 32 consecutive channels of one frame);
-//   * K runs over input-channel stages of KC (16 or 32) channels; a stage
-//     holds the stage's A window -- the tile's 256 frames plus the halo the
-//     taps reach back, loaded once and read by every tap at its own row
-//     offset -- and the weights of all G taps for those channels;
-//   * two LDS buffers: the next stage's global loads are in registers while a
-//     stage computes, written to the other buffer after it, one barrier per
-//     stage;
+//   * block tile: 128 frames x 192 or 256 output channels (4 waves in 2 x 2) or
+//     256 frames x 96 (4 x 1), each wave 64 frames x 96 or 128 channels of
+//     v_mfma_f32_32x32x16_f16 (frames as the A operand, weights as B, so the 32
+//     lanes of a row group store 32 consecutive channels of one frame);
+//   * K runs over stages of 32 input channels and, in a stage, over the taps:
+//     a stage holds the window of the tile's frames plus the halo the taps
+//     reach back, read by every tap at its own row offset; a step holds one
+//     tap's weights for those channels;
+//   * activations and weights lie in memory as contiguous KiB tiles of 16 rows
+//     x 32 channels, staged by LDS-DMA loads of one KiB per wave: weights NB
+//     steps ahead, windows NA stages ahead.  (Frame-major rows were read 32
+//     bytes at a time into registers, one stage ahead.)  The causal padding is
+//     a zeroed guard before each plane, so no load is predicated;
+//   * a step is computed in two halves of 16 channels; the next half's
+//     fragments are read from LDS while the current one multiplies, and the
+//     barrier between the halves frees the step's buffers;
 //   * tiles of one weight tile (m tile) are dealt to the same XCD, so that
 //     XCD's L2 serves its weights to all of its frame tiles.
+// Measured at 2048 latent frames (512 code frames; before: 256-frame tiles of
+// 16-channel stages through registers), us: entry 78 -> 64, transposed convs of
+// blocks 1-4 238 / 448 / 621 / 441 -> 145 / 325 / 385 / 309, k7 convs of blocks
+// 1 and 2 184 / 346 -> 131 / 264, their k1 convs 91 / 232 -> 43 / 150, a residual
+// unit of block 3 (k7 and k1 in one launch now) 856 -> 472, of block 4 548 -> 360;
+// whole decode 10.34 -> 7.20 ms.
 // Small per-frame kernels handle the rest: RVQ lookup, RoPE, the windowed
 // attention of the post-module transformer, depthwise conv + LayerNorm, the
 // output conv + tanh.
@@ -32,21 +43,16 @@ namespace {
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-constexpr uint32_t CG_TF = 256;    // frames per block tile
-constexpr uint32_t CG_MAXLD = 10;  // 16-byte staging loads per thread per stage
 constexpr size_t CG_FMAJOR_WEIGHT_BYTES = size_t(3) << 19;  // 1.5 MiB of a 4 MiB XCD L2
 
-// LDS rows are KC halfs (CH = KC / 8 chunks of 16 bytes), chunk c of row r
-// stored at c ^ swz(r).  Weight rows are read 32 at a time from a multiple
-// of 32; A window rows from any offset (the tap's shift), so their swizzle
-// only needs 8 consecutive rows on distinct banks.
-template <uint32_t CH>
-__device__ __forceinline__ uint32_t swz_a(uint32_t r) {
-  return CH == 2 ? ((r >> 2) & 1u) : (((r >> 1) ^ (r >> 3)) & 3u);
-}
-template <uint32_t CH>
-__device__ __forceinline__ uint32_t swz_w(uint32_t r) {
-  return CH == 2 ? (((r >> 2) ^ (r >> 3)) & 1u) : (((r >> 1) ^ (r >> 3)) & 3u);
+// swizzle of a 16-row activation tile (act_off): the 16-byte chunk c of row r
+// sits at c ^ act_swz(r), so 16 consecutive rows from any start put one chunk
+// each on distinct LDS banks
+__device__ __forceinline__ uint32_t act_swz(uint32_t r) { return ((r >> 1) & 3u) ^ ((r >> 3) & 1u); }
+// offset in halfs of channel c of frame f in a plane of C channels
+__device__ __forceinline__ size_t act_off(uint32_t f, uint32_t c, uint32_t C) {
+  return (size_t(f >> 4) * (C >> 5) + (c >> 5)) * 512 + (f & 15u) * 32u + ((((c >> 3) & 3u) ^ act_swz(f)) << 3) +
+         (c & 7u);
 }
 
 // erf_approx and gelu_erf (codec.rs:3886-3899), the reference's operation order.
@@ -64,16 +70,36 @@ __device__ __forceinline__ float erf_as(float value) {
 __device__ __forceinline__ float gelu_as(float v) {
   return __fmul_rn(__fmul_rn(0.5f, v), __fadd_rn(1.0f, erf_as(__fmul_rn(v, 0.70710677f))));
 }
-// snake_activation_frame_major (codec.rs:2162-2186), sin^2 from sin_cw.h
-__device__ __forceinline__ float snake(float x, float alpha) { return snake_cw(x, alpha); }
+// snake_activation_frame_major (codec.rs:2162-2186), sin^2 from sin_cw.h;
+// inv = 1 / (guarded alpha), once per channel
+__device__ __forceinline__ float snake(float x, float alpha, float inv) { return snake_cw(x, alpha, inv); }
 
-template <int MC, int KC, int PL, bool FU = false>
+// s_waitcnt immediate: at most `v` vector memory loads in flight, LDS reads
+// drained if `lgkm0`
+constexpr int wait_imm(int v, bool lgkm0) { return (v & 15) | ((v >> 4) << 14) | 0x70 | (lgkm0 ? 0 : 0xF00); }
+
+// One LDS-DMA load: the KiB at `base` (wave-uniform; lane i its 16 bytes at
+// 16 i) into LDS byte `lds`.  Inline assembly, so that the compiler does not
+// hold every later LDS read for it; the kernel waits itself.
+__device__ __forceinline__ void dma_kib(const uint8_t* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_nop 1\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds), "v"(off), "s"(base)
+               : "memory");
+}
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); }
+
+template <int G, int PL, int MC, int FC, int WMG, int NB, int NA, bool FU, int OS>
 __global__ __launch_bounds__(256, 2) void conv_gemm_kernel(ConvGemmArgs a, uint32_t m_tiles, uint32_t f_tiles,
-                                                           uint32_t halo, int32_t wbase, int32_t toff0,
-                                                           int32_t tstep, uint32_t fmajor) {
-  constexpr uint32_t TM = 32 * MC, CH = KC / 8;
-  extern __shared__ __align__(16) _Float16 cg_lds[];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+                                                           int32_t tile0, uint32_t a_tiles, int32_t t0, int32_t tstep,
+                                                           uint32_t fmajor) {
+  constexpr uint32_t MT = 32 * MC * WMG, FT = 32 * FC * (4 / WMG);
+  constexpr uint32_t AT = FT / 16 + (G == 7 ? 4 : G == 1 ? 0 : 1);  // most 16-frame tiles of a window
+  constexpr uint32_t WSTEP = MT * 64, APL = AT * 1024, ABUF = PL * APL;
+  constexpr int PW = (int(MT / 16) + 3) / 4, PA = (PL * int(AT) + 3) / 4;  // KiB loads per wave
+  extern __shared__ __align__(16) uint8_t cg_lds[];
+  const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
+  const uint32_t wm = wave % WMG, wf = wave / WMG;
   // Workgroup b runs on XCD b % 8; tiles are dealt to XCDs in contiguous
   // ranges (XCD-major), in one of two orders.
   //   fmajor: over all phases, t = (ft * phases + phase) * m_tiles + mt, so
@@ -105,169 +131,189 @@ __global__ __launch_bounds__(256, 2) void conv_gemm_kernel(ConvGemmArgs a, uint3
   }
   // (the divisions above are expanded on the vector unit: move the results
   // to scalar registers, where they cost no vector registers in the loop)
-  mt = uint32_t(__builtin_amdgcn_readfirstlane(int(mt)));
-  ft = uint32_t(__builtin_amdgcn_readfirstlane(int(ft)));
-  phase = uint32_t(__builtin_amdgcn_readfirstlane(int(phase)));
-  const uint32_t f0 = ft * CG_TF;
-  const uint32_t AR = CG_TF + halo;
-  const uint32_t a_chunks = PL * AR * CH, w_chunks = a.G * TM * CH, tot = a_chunks + w_chunks;
-  const uint32_t buf_halfs = (PL * AR + a.G * TM) * KC;
-  const uint32_t nst_all = a.C / KC, splits = gridDim.z, sp = blockIdx.z;
-  const uint32_t st_begin = nst_all * sp / splits, nst = nst_all * (sp + 1) / splits - st_begin;
-  const _Float16* wsrc = a.w + (size_t(phase) * m_tiles + mt) * (size_t(a.G) * TM * a.C);
-  const int32_t row0 = int32_t(f0) + wbase;
+  mt = uniform(mt);
+  ft = uniform(ft);
+  phase = uniform(phase);
+  const uint32_t f0 = ft * FT, kt = a.C / 32, splits = gridDim.z, sp = blockIdx.z;
+  const int32_t c0 = int32_t(kt * sp / splits), c1 = int32_t(kt * (sp + 1) / splits);
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>(cg_lds)), off = lane * 16u;
 
-  // Per staging slot i (chunk tid + 256 i of a stage): the element offset of
-  // its 16 bytes at stage 0 and its LDS offset, with the source in bits
-  // 30..31 (0: A hi plane, 1: A lo plane, 2: weights, 3: zero / no chunk).
-  // Stage st adds st * KC (A) or st * G * TM * KC (weights) to the offset.
-  uint32_t goff[CG_MAXLD], loff[CG_MAXLD];
+  // this wave's loads: weight tiles PW wave + j of a step, activation tiles
+  // PA wave + j of a window (plane-major); a load past the last tile repeats it
+  const uint8_t* wsrc = reinterpret_cast<const uint8_t*>(a.w) + (size_t(phase) * m_tiles + mt) * (size_t(G) * WSTEP * kt);
+  const uint8_t* asrc[PA];
+  uint32_t adst[PA];
 #pragma unroll
-  for (uint32_t i = 0; i < CG_MAXLD; ++i) {
-    const uint32_t qd = tid + 256u * i;
-    uint32_t kind = 3u, g = 0u, l = 0u;
-    if (qd < a_chunks) {
-      const uint32_t pl = PL == 2 ? qd / (AR * CH) : 0u, rem = qd - pl * (AR * CH);
-      const uint32_t row = rem / CH, c = rem - row * CH;
-      const int32_t src = row0 + int32_t(row);
-      l = (pl * AR + row) * KC + ((c ^ swz_a<CH>(row)) << 3);
-      if (src >= 0 && src < int32_t(a.F)) {
-        kind = pl;
-        g = uint32_t(src) * a.ldx + c * 8u;
-      }
-    } else if (qd < tot) {
-      const uint32_t wq = qd - a_chunks, row = wq / CH, c = wq - row * CH;
-      l = PL * AR * KC + row * KC + ((c ^ swz_w<CH>(row)) << 3);
-      kind = 2u;
-      g = wq * 8u;
-    } else {
-      l = 0xffffffffu >> 2;  // no chunk: nothing stored
-    }
-    goff[i] = g;
-    loff[i] = l | (kind << 30);
+  for (int j = 0; j < PA; ++j) {
+    const uint32_t q = min(PA * wave + j, uint32_t(PL) * AT - 1u), plane = q / AT, tile = min(q % AT, a_tiles - 1u);
+    asrc[j] = reinterpret_cast<const uint8_t*>(plane ? a.xl : a.xh) +
+              (int64_t(f0 / 16u) + tile0 + int32_t(tile)) * int64_t(kt) * 1024;
+    adst[j] = lds0 + NB * WSTEP + plane * APL + tile * 1024u;
   }
-  const uint32_t wstage = a.G * TM * KC;
-
-  uint4 stg[CG_MAXLD];
-  auto load = [&](uint32_t st) {
+  auto issue_w = [&](int32_t idx, uint32_t buf) {  // step idx = stage * G + tap, from this split's first
+    const uint8_t* src = wsrc + size_t(min(idx, (c1 - c0) * G - 1) + c0 * G) * WSTEP;
 #pragma unroll
-    for (uint32_t i = 0; i < CG_MAXLD; ++i) {
-      const uint32_t kind = loff[i] >> 30;
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (kind == 2u) {
-        v = *reinterpret_cast<const uint4*>(wsrc + size_t(st_begin + st) * wstage + goff[i]);
-      } else if (kind < 2u) {
-        const _Float16* base = kind ? a.xl : a.xh;
-        v = *reinterpret_cast<const uint4*>(base + size_t(goff[i]) + (st_begin + st) * KC);
-      }
-      stg[i] = v;
+    for (int j = 0; j < PW; ++j) {
+      const uint32_t q = min(PW * wave + j, MT / 16u - 1u) * 1024u;
+      dma_kib(src + q, off, lds0 + buf + q);
     }
   };
-  auto store = [&](uint32_t bsel) {
-    _Float16* B = cg_lds + bsel * buf_halfs;
+  auto issue_a = [&](int32_t st, uint32_t buf) {
+    const uint32_t k = uint32_t(min(c0 + st, c1 - 1)) * 1024u;
 #pragma unroll
-    for (uint32_t i = 0; i < CG_MAXLD; ++i) {
-      const uint32_t l = loff[i] & 0x3fffffffu;
-      if (l != (0xffffffffu >> 2)) *reinterpret_cast<uint4*>(B + l) = stg[i];
-    }
+    for (int j = 0; j < PA; ++j) dma_kib(asrc[j] + k, off, adst[j] + buf);
   };
 
-  floatx16 acc[2][MC];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < MC; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-  auto compute = [&](uint32_t bsel) {
-    const _Float16* A = cg_lds + bsel * buf_halfs;
-    const _Float16* W = A + PL * AR * KC;
-    for (uint32_t g = 0; g < a.G; ++g) {
-      const uint32_t toff = uint32_t(toff0 + int32_t(g) * tstep);
-#pragma unroll
-      for (uint32_t kk = 0; kk < uint32_t(KC / 16); ++kk) {
-        const uint32_t c = kk * 2u + (lane >> 5);
-        half8 bf[MC];
-#pragma unroll
-        for (int j = 0; j < MC; ++j) {
-          const uint32_t row = g * TM + uint32_t(j) * 32u + (lane & 31u);
-          bf[j] = *reinterpret_cast<const half8*>(W + row * KC + ((c ^ swz_w<CH>(row)) << 3));
-        }
-#pragma unroll
-        for (int p = 0; p < PL; ++p) {
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const uint32_t row = wave * 64u + uint32_t(i) * 32u + (lane & 31u) + toff;
-            const half8 af =
-                *reinterpret_cast<const half8*>(A + (uint32_t(p) * AR + row) * KC + ((c ^ swz_a<CH>(row)) << 3));
-#pragma unroll
-            for (int j = 0; j < MC; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[j], acc[i][j], 0, 0, 0);
-          }
-        }
-      }
-    }
+  const uint32_t fr = lane & 31u;
+  const uint32_t wrd = wm * MC * 2048u + (fr >> 4) * 1024u + (fr & 15u) * 16u + (lane >> 5) * 256u;
+  const uint32_t arow = wf * 32u * FC + fr;
+  struct Frags {
+    half8 w[MC], x[FC][PL];
   };
-
-  load(0);
-  store(0);
-  __syncthreads();
-  if (nst > 1) load(1);
-  for (uint32_t st = 0; st < nst; ++st) {
-    compute(st & 1u);
-    if (st + 1 < nst) store((st + 1) & 1u);
-    __syncthreads();
-    if (st + 2 < nst) load(st + 2);
+  auto read = [&](Frags& f, uint32_t wbuf, uint32_t abuf, int g, uint32_t h) {
+    const uint32_t row = arow + uint32_t(t0 + g * tstep);
+    const uint8_t* pa = cg_lds + abuf + row * 64u + (((2u * h + (lane >> 5)) ^ act_swz(row)) << 4);
+#pragma unroll
+    for (int i = 0; i < FC; ++i)
+#pragma unroll
+      for (int p = 0; p < PL; ++p) f.x[i][p] = *reinterpret_cast<const half8*>(pa + p * APL + i * 2048);
+    const uint8_t* pw = cg_lds + wbuf + wrd + h * 512u;
+#pragma unroll
+    for (int j = 0; j < MC; ++j) f.w[j] = *reinterpret_cast<const half8*>(pw + j * 2048);
+  };
+  floatx16 acc[FC][MC];
+#pragma unroll
+  for (int i = 0; i < FC; ++i)
+#pragma unroll
+    for (int j = 0; j < MC; ++j) acc[i][j] = floatx16{};
+  auto mma = [&](const Frags& f) {
+#pragma unroll
+    for (int p = 0; p < PL; ++p)
+#pragma unroll
+      for (int j = 0; j < MC; ++j)
+#pragma unroll
+        for (int i = 0; i < FC; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.x[i][p], f.w[j], acc[i][j], 0, 0, 0);
+  };
+  constexpr uint32_t A0 = NB * WSTEP;  // LDS byte of the first window
+  // The loads go out in the order of the steps that issue them (below), from
+  // as many steps before the first as the buffers reach ahead.
+  constexpr int PRE = NB > NA * G ? NB : NA * G;
+#pragma unroll
+  for (int v = -PRE; v < 0; ++v) {
+    if ((v + PRE * G) % G == G - 1 && (v - (G - 1)) / G + NA >= 0) {
+      const int st = (v - (G - 1)) / G + NA;
+      issue_a(st, (st % NA) * ABUF);
+    }
+    if (v + NB >= 0) issue_w(v + NB, ((v + NB) % NB) * WSTEP);
   }
+  __builtin_amdgcn_s_waitcnt(wait_imm(0, false));
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  Frags fa, fb;
+  uint32_t wbuf = 0, abuf = A0;
+  int32_t idx = 0;
+  read(fa, wbuf, abuf, 0, 0);
+  for (int32_t st = 0; st < c1 - c0; ++st) {
+#pragma unroll
+    for (int g = 0; g < G; ++g, ++idx) {
+      read(fb, wbuf, abuf, g, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(fa);
+      __builtin_amdgcn_sched_barrier(0);
+      // Wait for the weights of step idx + 1 (and, at the last tap, the next
+      // window): NB - 2 later weight steps may be in flight and the windows
+      // issued among them; lgkmcnt(0): this step's buffers are read.
+      constexpr auto later = [](int gg) {
+        int n = (NB - 2) * PW;
+        for (int k = 0; k <= NB - 3; ++k) n += k % G == gg % G ? PA : 0;
+        const int na = (NA - 1) * G * PW + (NA - 2) * PA;
+        return gg == G - 1 && na < n ? na : n;
+      };
+      switch (g) {  // (a constant after unrolling; the immediate must be one)
+        case 0: __builtin_amdgcn_s_waitcnt(wait_imm(later(0), true)); break;
+        case 1: __builtin_amdgcn_s_waitcnt(wait_imm(later(1), true)); break;
+        case 2: __builtin_amdgcn_s_waitcnt(wait_imm(later(2), true)); break;
+        case 3: __builtin_amdgcn_s_waitcnt(wait_imm(later(3), true)); break;
+        case 4: __builtin_amdgcn_s_waitcnt(wait_imm(later(4), true)); break;
+        case 5: __builtin_amdgcn_s_waitcnt(wait_imm(later(5), true)); break;
+        default: __builtin_amdgcn_s_waitcnt(wait_imm(later(6), true)); break;
+      }
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (g == G - 1) {
+        issue_a(st + NA, abuf - A0);
+        abuf = abuf + ABUF == A0 + NA * ABUF ? A0 : abuf + ABUF;
+      }
+      issue_w(idx + NB, wbuf);
+      wbuf = wbuf + WSTEP == NB * WSTEP ? 0u : wbuf + WSTEP;
+      read(fa, wbuf, abuf, g == G - 1 ? 0 : g + 1, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(fb);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // the unused tail loads have landed before LDS is used again or the block ends
+  __builtin_amdgcn_s_waitcnt(wait_imm(0, true));
 
   if constexpr (FU) {
     // The residual unit's k1 conv on the tile just computed (all M channels):
-    // Y = f16(snake(acc + bias_mid, alpha_mid)) in LDS ([256 frames][TM + 8]
-    // halfs: 16 consecutive rows fall on distinct 16-byte bank groups), the
-    // k1 weights W1 ([TM / 32 stages][TM rows][32], swizzled like W) next to
-    // it; every wave left the stage buffers at the loop's last barrier.
-    constexpr uint32_t YS = TM + 8;
-    _Float16* Y = cg_lds;
-    _Float16* W1 = cg_lds + CG_TF * YS;
-    for (uint32_t q = tid; q < TM * TM / 8u; q += 256u) {
-      const uint32_t st = q / (TM * 4u), rem = q - st * (TM * 4u), row = rem >> 2, c = rem & 3u;
-      *reinterpret_cast<uint4*>(W1 + st * (TM * 32u) + row * 32u + ((c ^ swz_w<4>(row)) << 3)) =
-          *reinterpret_cast<const uint4*>(a.w1 + size_t(q) * 8u);
-    }
+    // Y = f16(snake(acc + bias_mid, alpha_mid)) in LDS ([32 channels][frame][64
+    // bytes], swizzled like a window); its weights go straight to registers
+    // from the fragment-ordered copy, a step ahead.
+    const uint8_t* w1 = reinterpret_cast<const uint8_t*>(a.w1) + wrd;
+    half8 wn[2][MC];
+    auto load_w1 = [&](uint32_t c) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < MC; ++j) wn[h][j] = *reinterpret_cast<const half8*>(w1 + c * WSTEP + h * 512u + j * 2048);
+    };
+    load_w1(0);
+    __syncthreads();  // every wave's tail loads have landed
 #pragma unroll
     for (int j = 0; j < MC; ++j) {
-      const uint32_t m = uint32_t(j) * 32u + (lane & 31u);
-      const float bm = m < a.M ? a.bias_mid[m] : 0.0f;
-      const float am = m < a.M ? a.alpha_mid[m] : 1.0f;
+      const uint32_t m = (wm * MC + j) * 32u + fr;
+      const float bm = a.bias_mid[m], am = snake_guard(a.alpha_mid[m]), im = 1.0f / am;
+      uint8_t* yc = cg_lds + (m >> 5) * (FT * 64u) + (m & 7u) * 2u;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const uint32_t fl = wave * 64u + uint32_t(i) * 32u + 4u * (lane >> 5);
-#pragma nounroll
+      for (int i = 0; i < FC; ++i) {
+        const uint32_t fl = wf * 32u * FC + i * 32u + 4u * (lane >> 5);
+#pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const float val = snake(__fadd_rn(acc[i][j][v], bm), am);
-          Y[(fl + 8u * uint32_t(v >> 2) + uint32_t(v & 3)) * YS + m] = _Float16(val);
+          const uint32_t row = fl + 8u * (v >> 2) + (v & 3);
+          const float val = snake(__fadd_rn(acc[i][j][v], bm), am, im);
+          *reinterpret_cast<_Float16*>(yc + row * 64u + ((((m >> 3) & 3u) ^ act_swz(row)) << 4)) = _Float16(val);
           acc[i][j][v] = 0.0f;
+          if (v % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
     __syncthreads();
 #pragma unroll
-    for (uint32_t kk = 0; kk < TM / 16u; ++kk) {
-      const uint32_t c = kk * 2u + (lane >> 5);                  // chunk of the Y row
-      const uint32_t st = kk >> 1, cs = (kk & 1u) * 2u + (lane >> 5);  // W1 stage, chunk in it
-      half8 bf[MC];
+    for (uint32_t c = 0; c < MT / 32; ++c) {
+      half8 w[2][MC], x[2][FC];
 #pragma unroll
-      for (int j = 0; j < MC; ++j) {
-        const uint32_t row = uint32_t(j) * 32u + (lane & 31u);
-        bf[j] = *reinterpret_cast<const half8*>(W1 + st * (TM * 32u) + row * 32u + ((cs ^ swz_w<4>(row)) << 3));
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int j = 0; j < MC; ++j) w[h][j] = wn[h][j];
+#pragma unroll
+        for (int i = 0; i < FC; ++i)
+          x[h][i] = *reinterpret_cast<const half8*>(cg_lds + c * (FT * 64u) + (arow + 32u * i) * 64u +
+                                                    (((2u * h + (lane >> 5)) ^ act_swz(arow)) << 4));
       }
+      if (c + 1 < MT / 32) load_w1(c + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const half8 af = *reinterpret_cast<const half8*>(Y + (wave * 64u + uint32_t(i) * 32u + (lane & 31u)) * YS + c * 8u);
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < MC; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af, bf[j], acc[i][j], 0, 0, 0);
-      }
+        for (int j = 0; j < MC; ++j)
+#pragma unroll
+          for (int i = 0; i < FC; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[h][i], w[h][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 
@@ -275,14 +321,14 @@ __global__ __launch_bounds__(256, 2) void conv_gemm_kernel(ConvGemmArgs a, uint3
     const size_t rows = size_t(a.F) * a.ostride;
 #pragma unroll
     for (int j = 0; j < MC; ++j) {
-      const uint32_t m = mt * TM + uint32_t(j) * 32u + (lane & 31u);
+      const uint32_t m = mt * MT + (wm * MC + j) * 32u + fr;
       if (m >= a.M) continue;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const uint32_t fb = f0 + wave * 64u + uint32_t(i) * 32u + 4u * (lane >> 5);
+      for (int i = 0; i < FC; ++i) {
+        const uint32_t fb0 = f0 + (wf * FC + i) * 32u + 4u * (lane >> 5);
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const uint32_t f = fb + 8u * uint32_t(v >> 2) + uint32_t(v & 3);
+          const uint32_t f = fb0 + 8u * uint32_t(v >> 2) + uint32_t(v & 3);
           if (f < a.F) a.part[(size_t(sp) * rows + size_t(f) * a.ostride + phase) * a.M + m] = acc[i][j][v];
         }
       }
@@ -290,44 +336,70 @@ __global__ __launch_bounds__(256, 2) void conv_gemm_kernel(ConvGemmArgs a, uint3
     return;
   }
   // epilogue: acc[i][j][v] = D[frame 8 (v/4) + 4 (lane/32) + v%4][channel lane%32].
-  // The residual values of a fragment are loaded together before its stores
-  // (res may be the output buffer itself, so loads cannot move past stores).
+  // Frames past F are stored like the others: they land behind the buffers'
+  // last frame, in their tails.  Every address is a wave-uniform pointer plus
+  // a lane offset that does not change from value to value.
+  const uint32_t hl = lane >> 5, cc = fr >> 3, ts = a.M * 16u;  // ts: halfs between 16-frame tiles
+  uint32_t lo[4];  // lane offsets in a plane, by the kinds of rows that a value index can have
 #pragma unroll
-  for (int j = 0; j < MC; ++j) {
-    const uint32_t m = mt * TM + uint32_t(j) * 32u + (lane & 31u);
-    if (m >= a.M) continue;
+  for (uint32_t e = 0; e < 4; ++e) {
+    uint32_t row, chunk;
+    if constexpr (OS == 1) {
+      row = 4u * hl * 32u;
+      chunk = cc ^ (2u * hl) ^ e;  // e: (v % 4 / 2) ^ (v / 4 % 2)
+    } else if constexpr (OS == 2) {
+      row = (8u * hl + phase) * 32u;
+      chunk = cc ^ e ^ hl;
+    } else if constexpr (OS == 4) {
+      row = hl * ts + phase * 32u;
+      chunk = cc ^ ((2u * e + (phase >> 1)) & 3u) ^ (e >> 1);
+    } else {
+      row = 2u * hl * ts + phase * 32u;
+      chunk = cc ^ ((phase >> 1) & 3u) ^ e;  // e: v % 2
+    }
+    lo[e] = row + (chunk << 3) + (fr & 7u);
+  }
+  const uint32_t lres = 4u * hl * OS * a.ldres + fr, ly = 4u * hl * OS * a.ldy + fr;
+  // The residual values of the next fragment are loaded before this one's
+  // stores (the residual may be the output buffer itself; a value is read and
+  // written by the same lane, before the stores of any later fragment).
+  float rv[2][16];
+  auto load_res = [&](float (&r)[16], int q) {
+    const float* p = a.res + (size_t(f0 + (wf * FC + q % FC) * 32u) * OS + phase) * a.ldres + mt * MT + (wm * MC + q / FC) * 32u;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) r[v] = p[size_t(8 * (v >> 2) + (v & 3)) * OS * a.ldres + lres];
+  };
+  if (a.res) load_res(rv[0], 0);
+#pragma unroll
+  for (int q = 0; q < MC * FC; ++q) {
+    const int j = q / FC, i = q % FC;
+    if (a.res && q + 1 < MC * FC) load_res(rv[(q + 1) & 1], q + 1);
+    const uint32_t mb = mt * MT + (wm * MC + j) * 32u, m = mb + fr, fb0 = f0 + (wf * FC + i) * 32u;
     const float bias = a.bias[m];
     const float gam = a.gamma ? a.gamma[m] : 1.0f;
-    const float alp = a.alpha ? a.alpha[m] : 1.0f;
+    const float alp = a.alpha ? snake_guard(a.alpha[m]) : 1.0f, inv = 1.0f / alp;
+    float* y32 = a.y32 + (size_t(fb0) * OS + phase) * a.ldy + mb;
+    const size_t hb = size_t(fb0 / 16u * OS) * ts + (mb >> 5) * 512u;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const uint32_t fb = f0 + wave * 64u + uint32_t(i) * 32u + 4u * (lane >> 5);
-      float rv[16];
-      if (a.res) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const uint32_t f = fb + 8u * uint32_t(v >> 2) + uint32_t(v & 3);
-          rv[v] = f < a.F ? a.res[(size_t(f) * a.ostride + phase) * a.ldres + m] : 0.0f;
-        }
+    for (int v = 0; v < 16; ++v) {
+      const uint32_t Q = v >> 2, e = v & 3;
+      float val = __fadd_rn(acc[i][j][v], bias);
+      if (a.gelu) val = gelu_as(val);
+      if (a.gamma) val = __fmul_rn(val, gam);
+      if (a.res) val = __fadd_rn(rv[q & 1][v], val);
+      if (a.y32) (y32 + size_t(8 * Q + e) * OS * a.ldy)[ly] = val;
+      if (a.alpha) val = snake(val, alp, inv);
+      if (a.yh) {
+        const _Float16 h = _Float16(val);
+        const uint32_t kind = OS == 1 ? (e >> 1) ^ (Q & 1u) : OS == 8 ? (e & 1u) : e;
+        const uint32_t k = OS == 1   ? (Q >> 1) * ts + (8u * (Q & 1u) + e) * 32u
+                           : OS == 2 ? Q * ts + 2u * e * 32u
+                           : OS == 4 ? 2u * Q * ts + 4u * e * 32u
+                                     : (4u * Q + (e >> 1)) * ts + 8u * (e & 1u) * 32u;
+        (a.yh + hb + k)[lo[kind]] = h;
+        if (a.yl) (a.yl + hb + k)[lo[kind]] = _Float16(__fsub_rn(val, float(h)));
       }
-      // not unrolled: 2 x MC x 16 inlined snake evaluations in one block spill
-#pragma nounroll
-      for (int v = 0; v < 16; ++v) {
-        const uint32_t f = fb + 8u * uint32_t(v >> 2) + uint32_t(v & 3);
-        if (f >= a.F) continue;
-        const size_t row = size_t(f) * a.ostride + phase;
-        float val = __fadd_rn(acc[i][j][v], bias);
-        if (a.gelu) val = gelu_as(val);
-        if (a.gamma) val = __fmul_rn(val, gam);
-        if (a.res) val = __fadd_rn(rv[v], val);
-        if (a.y32) a.y32[row * a.ldy + m] = val;
-        if (a.alpha) val = snake(val, alp);
-        if (a.yh) {
-          const _Float16 h = _Float16(val);
-          a.yh[row * a.ldh + m] = h;
-          if (a.yl) a.yl[row * a.ldh + m] = _Float16(__fsub_rn(val, float(h)));
-        }
-      }
+      if (v % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
@@ -347,11 +419,15 @@ __global__ __launch_bounds__(256) void conv_split_reduce_kernel(ConvGemmArgs a, 
   if (a.gamma) val = __fmul_rn(val, a.gamma[m]);
   if (a.res) val = __fadd_rn(a.res[row * a.ldres + m], val);
   if (a.y32) a.y32[row * a.ldy + m] = val;
-  if (a.alpha) val = snake(val, a.alpha[m]);
+  if (a.alpha) {
+    const float alp = snake_guard(a.alpha[m]);
+    val = snake(val, alp, 1.0f / alp);
+  }
   if (a.yh) {
     const _Float16 h = _Float16(val);
-    a.yh[row * a.ldh + m] = h;
-    if (a.yl) a.yl[row * a.ldh + m] = _Float16(__fsub_rn(val, float(h)));
+    const size_t o = act_off(uint32_t(row), m, a.M);
+    a.yh[o] = h;
+    if (a.yl) a.yl[o] = _Float16(__fsub_rn(val, float(h)));
   }
 }
 
@@ -498,13 +574,15 @@ __global__ __launch_bounds__(256) void codec_scaled_residual_kernel(float* x, co
   x[i] = __fadd_rn(x[i], __fmul_rn(p[i], scale[i % D]));
 }
 
-__global__ __launch_bounds__(256) void codec_split16_kernel(const float* x, _Float16* hi, _Float16* lo, size_t n) {
+__global__ __launch_bounds__(256) void codec_split16_kernel(const float* x, _Float16* hi, _Float16* lo, size_t n,
+                                                            uint32_t C) {
   const size_t i = size_t(blockIdx.x) * 256u + threadIdx.x;
   if (i >= n) return;
   const float v = x[i];
   const _Float16 h = _Float16(v);
-  hi[i] = h;
-  lo[i] = _Float16(__fsub_rn(v, float(h)));
+  const size_t o = act_off(uint32_t(i / C), uint32_t(i % C), C);
+  hi[o] = h;
+  if (lo) lo[o] = _Float16(__fsub_rn(v, float(h)));
 }
 
 // forward_codec_convnext_block front (codec.rs:3444-3460): depthwise causal
@@ -552,8 +630,9 @@ __global__ __launch_bounds__(256) void codec_dwconv_ln_kernel(const float* x, ui
     const uint32_t c = tid + 256u * k;
     const float y = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(d[k], mean), scale), ln_w[c]), ln_b[c]);
     const _Float16 h = _Float16(y);
-    hi[size_t(f) * 1024u + c] = h;
-    lo[size_t(f) * 1024u + c] = _Float16(__fsub_rn(y, float(h)));
+    const size_t o = act_off(f, c, 1024u);
+    hi[o] = h;
+    lo[o] = _Float16(__fsub_rn(y, float(h)));
   }
 }
 
@@ -573,7 +652,7 @@ __global__ __launch_bounds__(256) void codec_out_conv_kernel(const _Float16* x, 
     const uint32_t r = e / 12u, c = e - r * 12u;
     const int32_t src = int32_t(t0) + int32_t(r) - 6;
     uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (src >= 0 && src < int32_t(T)) v = *reinterpret_cast<const uint4*>(x + size_t(src) * 96u + c * 8u);
+    if (src >= 0 && src < int32_t(T)) v = *reinterpret_cast<const uint4*>(x + act_off(uint32_t(src), c * 8u, 96u));
     uint32_t* d = reinterpret_cast<uint32_t*>(xs + r * OC_ROW + c * 8u);
     d[0] = v.x;
     d[1] = v.y;
@@ -597,40 +676,38 @@ __global__ __launch_bounds__(256) void codec_out_conv_kernel(const _Float16* x, 
   out[t] = tanhf(y);
 }
 
-template <int MC, int KC, int PL, bool FU = false>
+template <int G, int PL, int MC, int FC, int WMG, int NB, int NA, bool FU, int OS>
 hipError_t conv_gemm_launch(const ConvGemmArgs& a, uint32_t phases, hipStream_t s) {
-  constexpr uint32_t TM = 32 * MC, CH = KC / 8;
+  constexpr uint32_t MT = 32 * MC * WMG, FT = 32 * FC * (4 / WMG), AT = FT / 16 + (G == 7 ? 4 : G == 1 ? 0 : 1);
+  constexpr uint32_t lds = NB * MT * 64 + NA * PL * AT * 1024;
+  static_assert(!FU || FT * MT * 2 <= lds, "the k1 conv's input must fit the stage buffers");
   const int32_t last = a.off0 + int32_t(a.G - 1) * a.ostep;
-  const int32_t wbase = a.off0 < last ? a.off0 : last;
-  const uint32_t halo = uint32_t((a.off0 < last ? last : a.off0) - wbase);
-  const uint32_t AR = CG_TF + halo;
-  if (size_t(PL) * AR * CH + size_t(a.G) * TM * CH > 256u * CG_MAXLD) return hipErrorInvalidValue;
-  size_t lds = 2u * (size_t(PL) * AR + size_t(a.G) * TM) * KC * sizeof(_Float16);
-  if (FU) lds = std::max(lds, (size_t(CG_TF) * (TM + 8) + size_t(TM) * TM) * sizeof(_Float16));
-  if (lds > 160u * 1024u) return hipErrorInvalidValue;
-  const uint32_t m_tiles = (a.M + TM - 1) / TM, f_tiles = (a.F + CG_TF - 1) / CG_TF;
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_gemm_kernel<MC, KC, PL, FU>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
-  // K split when the grid would leave CUs idle: each split keeps >= 4 stages
-  const uint32_t nst = a.C / KC, blocks = m_tiles * f_tiles * phases;
+  const int32_t wbase = a.off0 < last ? a.off0 : last, wend = a.off0 < last ? last : a.off0;
+  // window: frames f0 + wbase .. f0 + FT - 1 + wend, from the 16-frame tile that holds its first
+  if (wend > 0 || wbase < -ACT_GUARD) return hipErrorInvalidValue;
+  const int32_t tile0 = -((15 - wbase) / 16), shift = wbase - 16 * tile0;
+  const uint32_t a_tiles = (uint32_t(shift + (wend - wbase)) + FT + 15u) / 16u;
+  if (a_tiles > AT) return hipErrorInvalidValue;
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_gemm_kernel<G, PL, MC, FC, WMG, NB, NA, FU, OS>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (attr != hipSuccess) return attr;
+  const uint32_t m_tiles = (a.M + MT - 1) / MT, f_tiles = (a.F + FT - 1) / FT;
+  // K split when the grid would leave CUs idle: each split keeps >= 2 stages
+  const uint32_t nst = a.C / 32, blocks = m_tiles * f_tiles * phases;
   const size_t rows = size_t(a.F) * phases;
   uint32_t splits = 1;
   if (a.part && !FU) {
-    while (splits < 8 && blocks * splits < 256u && nst / (2 * splits) >= 4 &&
+    while (splits < 8 && blocks * splits < 256u && nst / (2 * splits) >= 2 &&
            size_t(2 * splits) * rows * a.M <= a.part_cap)
       splits *= 2;
   }
   // frame-tile-major block order when the weights of every (phase, m tile)
   // fit in an XCD's L2 next to the streamed input windows
-  const size_t wbytes = size_t(phases) * m_tiles * a.G * TM * a.C * sizeof(_Float16);
+  const size_t wbytes = size_t(phases) * m_tiles * a.G * MT * a.C * sizeof(_Float16);
   const uint32_t fmajor = wbytes <= CG_FMAJOR_WEIGHT_BYTES ? 1u : 0u;
-  conv_gemm_kernel<MC, KC, PL, FU><<<dim3(m_tiles * f_tiles * phases, 1, splits), 256, lds, s>>>(
-      a, m_tiles, f_tiles, halo, wbase, a.off0 - wbase, a.ostep, fmajor);
+  conv_gemm_kernel<G, PL, MC, FC, WMG, NB, NA, FU, OS><<<dim3(m_tiles * f_tiles * phases, 1, splits), 256, lds, s>>>(
+      a, m_tiles, f_tiles, tile0, a_tiles, shift + a.off0 - wbase, a.ostep, fmajor);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || splits == 1) return e;
   const size_t n = rows * a.M;
@@ -640,37 +717,37 @@ hipError_t conv_gemm_launch(const ConvGemmArgs& a, uint32_t phases, hipStream_t 
 
 }  // namespace
 
-ConvTile conv_tile(uint32_t M, uint32_t G, bool split) {
-  (void)split;
-  ConvTile t;
-  t.mc = (M % 128u != 0 && M % 96u == 0) ? 3u : 4u;
-  t.kc = G > 1 ? 16u : 32u;
-  return t;
+uint32_t conv_tile_rows(uint32_t M) { return M % 192u == 0 ? 192u : M % 96u == 0 ? 96u : 256u; }
+
+size_t conv_packed_halfs(uint32_t phases, uint32_t M, uint32_t G, uint32_t C) {
+  const uint32_t MT = conv_tile_rows(M);
+  return size_t(phases) * ((M + MT - 1) / MT) * MT * G * C;
 }
 
-size_t conv_packed_halfs(uint32_t phases, uint32_t M, uint32_t G, uint32_t C, ConvTile t) {
-  const uint32_t TM = 32 * t.mc;
-  return size_t(phases) * ((M + TM - 1) / TM) * TM * G * C;
-}
-
-hipError_t launch_conv_gemm(const ConvGemmArgs& a, uint32_t phases, ConvTile t, hipStream_t s) {
-  if (a.C == 0 || a.C % t.kc || a.F == 0 || a.M == 0 || a.G == 0 || phases == 0) return hipErrorInvalidValue;
-  if (a.ldx % 8u || (a.yh && a.ldh % 2u)) return hipErrorInvalidValue;
+hipError_t launch_conv_gemm(const ConvGemmArgs& a, uint32_t phases, hipStream_t s) {
+  if (a.C == 0 || a.C % 32 || a.F == 0 || a.M == 0 || a.M % 32 || phases == 0) return hipErrorInvalidValue;
+  if (uint64_t(a.F) * phases > 0x7fffffffull) return hipErrorInvalidValue;
   const bool split = a.xl != nullptr;
-  if (t.mc == 4 && t.kc == 16) return split ? conv_gemm_launch<4, 16, 2>(a, phases, s) : conv_gemm_launch<4, 16, 1>(a, phases, s);
-  if (t.mc == 4 && t.kc == 32) return split ? conv_gemm_launch<4, 32, 2>(a, phases, s) : conv_gemm_launch<4, 32, 1>(a, phases, s);
-  if (t.mc == 3 && t.kc == 16) return split ? conv_gemm_launch<3, 16, 2>(a, phases, s) : conv_gemm_launch<3, 16, 1>(a, phases, s);
-  if (t.mc == 3 && t.kc == 32) return split ? conv_gemm_launch<3, 32, 2>(a, phases, s) : conv_gemm_launch<3, 32, 1>(a, phases, s);
+  const uint32_t MT = conv_tile_rows(a.M);
+  if (a.M % MT || a.ostride != phases) return hipErrorInvalidValue;
+  const uint32_t os = a.ostride;
+  if (MT == 192 && a.G == 7 && !split && os == 1) return conv_gemm_launch<7, 1, 3, 2, 2, 3, 2, false, 1>(a, phases, s);
+  if (MT == 192 && a.G == 1 && !split && os == 1) return conv_gemm_launch<1, 1, 3, 2, 2, 3, 3, false, 1>(a, phases, s);
+  if (MT == 192 && a.G == 2 && split && os == 8) return conv_gemm_launch<2, 2, 3, 2, 2, 3, 2, false, 8>(a, phases, s);
+  if (MT == 192 && a.G == 2 && split && os == 4) return conv_gemm_launch<2, 2, 3, 2, 2, 3, 2, false, 4>(a, phases, s);
+  if (MT == 96 && a.G == 2 && split && os == 2) return conv_gemm_launch<2, 2, 3, 2, 1, 2, 2, false, 2>(a, phases, s);
+  if (MT == 256 && a.G == 1 && split && os == 2) return conv_gemm_launch<1, 2, 4, 2, 2, 2, 2, false, 2>(a, phases, s);
+  if (MT == 256 && a.G == 1 && split && os == 1) return conv_gemm_launch<1, 2, 4, 2, 2, 2, 2, false, 1>(a, phases, s);
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_residual_unit(const ConvGemmArgs& a, ConvTile t, hipStream_t s) {
-  if (!a.w1 || !a.bias_mid || !a.alpha_mid || a.M % 32u || a.M > 32u * t.mc || t.kc != 16 || a.xl ||
-      a.C != a.M || a.ldx % 8u)
+bool residual_unit_fits(uint32_t M) { return M == 96 || M == 192; }
+
+hipError_t launch_residual_unit(const ConvGemmArgs& a, hipStream_t s) {
+  if (!a.w1 || !a.bias_mid || !a.alpha_mid || !residual_unit_fits(a.M) || a.G != 7 || a.xl || a.C != a.M || a.F == 0)
     return hipErrorInvalidValue;
-  if (t.mc == 3) return conv_gemm_launch<3, 16, 1, true>(a, 1, s);
-  if (t.mc == 4) return conv_gemm_launch<4, 16, 1, true>(a, 1, s);
-  return hipErrorInvalidValue;
+  if (a.M == 192) return conv_gemm_launch<7, 1, 3, 2, 2, 3, 2, true, 1>(a, 1, s);
+  return conv_gemm_launch<7, 1, 3, 2, 1, 4, 2, true, 1>(a, 1, s);
 }
 
 hipError_t launch_codec_rvq(const RvqArgs& a, hipStream_t s) {
@@ -706,9 +783,10 @@ hipError_t launch_codec_scaled_residual(float* x, const float* p, const float* s
   return hipGetLastError();
 }
 
-hipError_t launch_codec_split16(const float* x, _Float16* hi, _Float16* lo, size_t n, hipStream_t s) {
+hipError_t launch_codec_split16(const float* x, _Float16* hi, _Float16* lo, size_t frames, uint32_t C, hipStream_t s) {
+  const size_t n = frames * C;
   if (n == 0) return hipSuccess;
-  codec_split16_kernel<<<uint32_t((n + 255) / 256), 256, 0, s>>>(x, hi, lo, n);
+  codec_split16_kernel<<<uint32_t((n + 255) / 256), 256, 0, s>>>(x, hi, lo, n, C);
   return hipGetLastError();
 }
 

@@ -65,7 +65,6 @@ float half_to_float(uint16_t h) {
 struct ConvW {
   _Float16* w = nullptr;
   float* bias = nullptr;
-  ConvTile tile{4, 32};
   uint32_t G = 1, M = 0, C = 0, phases = 1;
 };
 
@@ -133,7 +132,7 @@ class CodecEngine {
     if (out_cap < need) cfail("decoder output buffer holds %zu floats, %zu needed", out_cap, need);
     if (frames == 0) return 0;
     upload(up32_, hidden, size_t(frames) * H);
-    to_f16(up32_, a16_, size_t(frames) * H);
+    CHK(launch_codec_split16(up32_, a16_, nullptr, frames, H, stream_));
     const void* r = decoder(frames, stop_block);
     download(out, static_cast<const float*>(r), need);
     return need;
@@ -184,7 +183,7 @@ class CodecEngine {
     recording_ = false;
     CHK(hipStreamSynchronize(stream_));
     double total_flops = 0.0;
-    for (const Rec& r : rec_) total_flops += r.flops;
+    for (const Rec& r : rec_) total_flops += r.part ? 0.0 : r.flops;
     const Rec* one = nullptr;
     for (const Rec& r : rec_)
       if (r.name == what) one = &r;
@@ -194,9 +193,9 @@ class CodecEngine {
     CHK(hipEventCreate(&e1));
     auto launch = [&] {
       if (one && one->phases == 0)
-        CHK(launch_residual_unit(one->a, one->tile, stream_));
+        CHK(launch_residual_unit(one->a, stream_));
       else if (one)
-        CHK(launch_conv_gemm(one->a, one->phases, one->tile, stream_));
+        CHK(launch_conv_gemm(one->a, one->phases, stream_));
       else
         waveform(n, nullptr, samples_);
     };
@@ -220,6 +219,14 @@ class CodecEngine {
     CHK(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T)));
     allocs_.push_back(p);
     return static_cast<T*>(p);
+  }
+  // an f16 activation plane of n elements, between its zero guard and its tail
+  // (both sized for the widest plane, so that any channel count finds them)
+  _Float16* plane(size_t n) {
+    const size_t guard = size_t(ACT_GUARD) * EXP, tail = size_t(ACT_TAIL) * EXP;
+    _Float16* p = dalloc<_Float16>(guard + n + tail);
+    CHK(hipMemset(p, 0, guard * sizeof(_Float16)));
+    return p + guard;
   }
   template <class T>
   T* upload_vec(const std::vector<T>& v) {
@@ -251,22 +258,21 @@ class CodecEngine {
     return d;
   }
   template <class Src>
-  ConvW packed(uint32_t phases, uint32_t M, uint32_t G, uint32_t C, bool split, Src src) {
+  ConvW packed(uint32_t phases, uint32_t M, uint32_t G, uint32_t C, Src src) {
     ConvW c;
-    c.tile = conv_tile(M, G, split);
     c.G = G;
     c.M = M;
     c.C = C;
     c.phases = phases;
-    std::vector<uint16_t> h(conv_packed_halfs(phases, M, G, C, c.tile));
-    pack_conv_weights(h.data(), phases, M, G, C, c.tile, src);
+    std::vector<uint16_t> h(conv_packed_halfs(phases, M, G, C));
+    pack_conv_weights(h.data(), phases, M, G, C, src);
     c.w = reinterpret_cast<_Float16*>(upload_vec(h));
     return c;
   }
   // causal_conv_1d weight, ggml [k][in][out] (index tap + k*in_i + k*in*o)
   ConvW conv1d(const std::string& p, uint32_t k, uint32_t cin, uint32_t cout) {
     const uint16_t* w = bits(p + ".conv.weight", {k, cin, cout});
-    ConvW c = packed(1, cout, k, cin, false, [&](uint32_t, uint32_t m, uint32_t g, uint32_t ch) {
+    ConvW c = packed(1, cout, k, cin, [&](uint32_t, uint32_t m, uint32_t g, uint32_t ch) {
       return w[g + size_t(k) * ch + size_t(k) * cin * m];
     });
     c.bias = vec(p + ".conv.bias", {cout});
@@ -277,7 +283,7 @@ class CodecEngine {
   ConvW conv_t(const std::string& p, uint32_t stride, uint32_t k, uint32_t cin, uint32_t cout) {
     const uint16_t* w = bits(p + ".conv.weight", {k, cout, cin});
     if (k % stride) cfail("%s: kernel %u is not a multiple of stride %u", p.c_str(), k, stride);
-    ConvW c = packed(stride, cout, k / stride, cin, true, [&](uint32_t r, uint32_t m, uint32_t j, uint32_t ch) {
+    ConvW c = packed(stride, cout, k / stride, cin, [&](uint32_t r, uint32_t m, uint32_t j, uint32_t ch) {
       return w[(r + j * stride) + size_t(k) * m + size_t(k) * cout * ch];
     });
     c.bias = vec(p + ".conv.bias", {cout});
@@ -286,7 +292,7 @@ class CodecEngine {
   // linear [out][in] rows
   ConvW linear(const std::string& p, uint32_t in, uint32_t out) {
     const uint16_t* w = bits(p + ".weight", {in, out});
-    ConvW c = packed(1, out, 1, in, true, [&](uint32_t, uint32_t m, uint32_t, uint32_t ch) {
+    ConvW c = packed(1, out, 1, in, [&](uint32_t, uint32_t m, uint32_t, uint32_t ch) {
       return w[size_t(m) * in + ch];
     });
     c.bias = vec(p + ".bias", {out});
@@ -402,20 +408,20 @@ class CodecEngine {
     prs_ = dalloc<float>(npad_);
     part_cap_ = gemm_part_floats(uint32_t(npad_), QKV);
     part_ = dalloc<float>(part_cap_);
-    up32_ = dalloc<float>(4 * F * H);
-    upx_ = dalloc<float>(4 * F * H);
-    qh_ = dalloc<_Float16>(4 * F * H);
-    ql_ = dalloc<_Float16>(4 * F * H);
-    ph_ = dalloc<_Float16>(4 * F * EXP);
-    pl_ = dalloc<_Float16>(4 * F * EXP);
+    up32_ = dalloc<float>(4 * F * H + ACT_TAIL * EXP);
+    upx_ = dalloc<float>(4 * F * H + ACT_TAIL * EXP);
+    qh_ = plane(4 * F * H);
+    ql_ = plane(4 * F * H);
+    ph_ = plane(4 * F * EXP);
+    pl_ = plane(4 * F * EXP);
     const size_t big = F * 196608;  // largest decoder activation: frames x channels
-    x32_ = dalloc<float>(big);
-    a16_ = dalloc<_Float16>(big);
-    b16_ = dalloc<_Float16>(big);
-    dh_ = dalloc<_Float16>(big);
-    dl_ = dalloc<_Float16>(big);
+    x32_ = dalloc<float>(big + ACT_TAIL * EXP);
+    a16_ = plane(big);
+    b16_ = plane(big);
+    dh_ = plane(big);
+    dl_ = plane(big);
     samples_ = dalloc<float>(F * SAMPLES_PER_FRAME);
-    cpart_cap_ = F * 32768;  // K-split partial sums of the short-grid products
+    cpart_cap_ = std::max<size_t>(F * 32768, size_t(1) << 24);  // K-split partial sums of the short-grid products
     cpart_ = dalloc<float>(cpart_cap_);
   }
 
@@ -440,11 +446,6 @@ class CodecEngine {
     CHK(hipMemcpyAsync(h, d, n * 4, hipMemcpyDeviceToHost, stream_));
     CHK(hipStreamSynchronize(stream_));
   }
-  void to_f16(const float* x, _Float16* h, size_t n) {
-    // f16 plane only: split16 with the lo plane written to the b16 buffer
-    CHK(launch_codec_split16(x, h, b16_, n, stream_));
-  }
-
   void rvq(uint32_t n, const int32_t* codes_dev) {
     RvqArgs a{};
     a.codes = codes_dev ? codes_dev : codes_;
@@ -506,7 +507,6 @@ class CodecEngine {
     ConvGemmArgs a{};
     a.xh = xh;
     a.xl = xl;
-    a.ldx = w.C;
     a.C = w.C;
     a.F = frames;
     a.G = w.G;
@@ -519,18 +519,18 @@ class CodecEngine {
     return a;
   }
   void run(const ConvGemmArgs& a, const ConvW& w, const char* name) {
-    CHK(launch_conv_gemm(a, w.phases, w.tile, stream_));
+    CHK(launch_conv_gemm(a, w.phases, stream_));
     if (recording_) {
       const double flops = 2.0 * double(a.F) * w.phases * w.M * w.G * w.C;
-      rec_.push_back(Rec{name, a, w.phases, w.tile, flops});
+      rec_.push_back(Rec{name, a, w.phases, flops});
     }
   }
   struct Rec {
     std::string name;
     ConvGemmArgs a;
     uint32_t phases;
-    ConvTile tile;
     double flops;  // 2 x multiply-adds of the convolution (the reference's arithmetic)
+    bool part = false;  // counted in another record already
     // phases 0: a fused residual unit (launch_residual_unit)
   };
   bool recording_ = false;
@@ -543,7 +543,7 @@ class CodecEngine {
     uint32_t F = n;
     for (uint32_t s = 0; s < 2; ++s) {
       const Stage& S = stages_[s];
-      CHK(launch_codec_split16(in, qh_, ql_, size_t(F) * H, stream_));
+      CHK(launch_codec_split16(in, qh_, ql_, F, H, stream_));
       ConvGemmArgs c = cargs(S.ct, qh_, ql_, F);  // conv_transpose, stride 2, kernel 2: one tap per phase
       c.off0 = 0;
       c.ostep = -1;
@@ -558,7 +558,6 @@ class CodecEngine {
       p1.gelu = 1;
       p1.yh = ph_;
       p1.yl = pl_;
-      p1.ldh = EXP;
       run(p1, S.pw1, s ? "up2_pw1" : "up1_pw1");
       ConvGemmArgs p2 = cargs(S.pw2, ph_, pl_, F);
       p2.off0 = 0;
@@ -570,7 +569,6 @@ class CodecEngine {
       p2.ldy = H;
       if (s == 1 && to_decoder) {
         p2.yh = a16_;
-        p2.ldh = H;
       }
       run(p2, S.pw2, s ? "up2_pw2" : "up1_pw2");
       in = upx_;
@@ -586,7 +584,6 @@ class CodecEngine {
       c.y32 = x32_;
       c.ldy = co;
     }
-    c.ldh = co;
     if (r < 2) {  // the next residual unit's conv0 input
       c.alpha = B.res[r + 1].a0;
       c.yh = a16_;
@@ -618,7 +615,6 @@ class CodecEngine {
     e.alpha = blocks_[0].alpha;
     e.yh = dh_;
     e.yl = dl_;
-    e.ldh = ENTRY;
     if (stop_block == 0) {
       e.y32 = x32_;
       e.ldy = ENTRY;
@@ -637,15 +633,13 @@ class CodecEngine {
       t.ldy = co;
       t.alpha = B.res[0].a0;
       t.yh = a16_;
-      t.ldh = co;
       run(t, B.ct, names_[b][0].c_str());
       F *= RATES[b];
       const uint32_t dil[3] = {1, 3, 9};
       const bool stop_here = stop_block == b + 1;
       for (uint32_t r = 0; r < 3; ++r) {
         const Res& R = B.res[r];
-        const bool fused = co % 32u == 0 && co <= 32u * R.c0.tile.mc && R.c1.tile.mc == R.c0.tile.mc && R.c0.tile.mc <= 4;
-        if (fused) {  // k7 conv + snake + k1 conv in one launch (the block holds every channel)
+        if (residual_unit_fits(co)) {  // k7 conv + snake + k1 conv in one launch (the block holds every channel)
           // the k7 conv reads other tiles' rows (its halo), so the unit's f16
           // output goes to the other buffer: units read a16, b16, a16 and
           // write b16, a16, b16
@@ -664,10 +658,26 @@ class CodecEngine {
           set_unit_outputs(u, B, b, r, co, stop_here);
           if (u.yh == a16_) u.yh = uout;  // dh_ / dl_ outputs are separate buffers already
           if (r == 2 && b == 3) out_in = uout;
-          CHK(launch_residual_unit(u, R.c0.tile, stream_));
+          CHK(launch_residual_unit(u, stream_));
           if (recording_)
-            rec_.push_back(Rec{names_[b][1 + 2 * r].substr(0, 5) + "_unit", u, 0, R.c0.tile,
+            rec_.push_back(Rec{names_[b][1 + 2 * r].substr(0, 5) + "_unit", u, 0,
                                2.0 * double(F) * co * (7.0 * co + co)});
+          if (recording_ && co == 192) {  // its convolutions by themselves, for time() only
+            ConvGemmArgs c0 = cargs(R.c0, uin, nullptr, F), c1 = u;
+            c0.off0 = u.off0;
+            c0.ostep = u.ostep;
+            c0.alpha = R.a1;
+            c0.yh = uout;
+            c1.xh = uout;
+            c1.G = 1;
+            c1.off0 = 0;
+            c1.ostep = 1;
+            c1.w = R.c1.w;
+            c1.w1 = nullptr;
+            if (c1.yh == uout) c1.yh = uin;
+            rec_.push_back(Rec{names_[b][1 + 2 * r], c0, 1, 2.0 * double(F) * co * 7.0 * co, true});
+            rec_.push_back(Rec{names_[b][2 + 2 * r], c1, 1, 2.0 * double(F) * co * co, true});
+          }
           continue;
         }
         ConvGemmArgs c0 = cargs(R.c0, a16_, nullptr, F);
@@ -675,7 +685,6 @@ class CodecEngine {
         c0.ostep = int32_t(dil[r]);
         c0.alpha = R.a1;
         c0.yh = b16_;
-        c0.ldh = co;
         run(c0, R.c0, names_[b][1 + 2 * r].c_str());
         ConvGemmArgs c1 = cargs(R.c1, b16_, nullptr, F);
         c1.off0 = 0;

@@ -120,6 +120,24 @@ def test_decoder_checkpoints_match_oracle(codec, oracle, frames):
     assert err.max() < 1e-2 and err.mean() < 1e-3, (err.max(), err.mean())
 
 
+@pytest.mark.parametrize("frames", [1, 16, 33, 129])
+def test_decoder_ragged_lengths_after_a_longer_call(codec, oracle, frames):
+    """Frame counts at the edges of the 16-frame activation tiles and of the
+    128- and 256-frame output tiles, on buffers that a longer decode has left
+    full: what lies past a call's last frame must not reach its outputs.  The
+    first block's checkpoint against the oracle, and all four against the same
+    frames of a longer call (every stage is causal): f16 inputs, as above."""
+    rng = np.random.default_rng(50)
+    hid = rng.standard_normal((160, 1024)).astype(np.float32)
+    full = [codec.decoder(hid, stop) for stop in range(6)]
+    for stop in range(6):
+        got = codec.decoder(hid[:frames], stop)
+        want = full[stop][: got.shape[0]]
+        assert got.shape == want.shape
+        assert np.max(np.abs(got - want)) <= (1e-2 if stop == 5 else 5e-3 * np.max(np.abs(want))), stop
+    assert _rel(codec.decoder(hid[:frames], 1), oracle.decoder(hid[:frames], 1)) < 5e-3
+
+
 def test_decode_waveform_matches_oracle(codec, oracle):
     n = 16
     codes = random_codes(n, seed=13)
