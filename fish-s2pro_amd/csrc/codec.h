@@ -109,15 +109,9 @@ struct RvqArgs {
 hipError_t launch_codec_rvq(const RvqArgs& a, hipStream_t s);
 
 // RoPE on the q and k parts of qkv rows [T][3072] (16 heads of 64, adjacent
-// pairs) from a (cos, sin) table [position][32].
-hipError_t launch_codec_rope(float* qkv, uint32_t T, const float2* table, hipStream_t s);
-
-// Causal attention over a 128-frame window: 16 heads of 64, scale 1/8.
-hipError_t launch_codec_attention(const float* qkv, uint32_t T, float* out, hipStream_t s);
-
-// x[t][i] = x[t][i] + p[t][i] * scale[i]
-hipError_t launch_codec_scaled_residual(float* x, const float* p, const float* scale, uint32_t T, uint32_t D,
-                                        hipStream_t s);
+// pairs) from a (cos, sin) table [position][32], then causal attention over a
+// 128-frame window, scale 1/8.
+hipError_t launch_codec_attention(const float* qkv, uint32_t T, const float2* table, float* out, hipStream_t s);
 
 // x [frames][C] -> planes hi = f16(x) and, unless null, lo = f16(x - hi)
 hipError_t launch_codec_split16(const float* x, _Float16* hi, _Float16* lo, size_t frames, uint32_t C, hipStream_t s);

@@ -464,34 +464,29 @@ __global__ __launch_bounds__(256) void codec_check_codes_kernel(const int32_t* c
   if (c < 0 || c >= size) *err = 1u;
 }
 
-// apply_rope_normal (attention.rs:172-206) on q and k of one frame: pairs
+// apply_rope_normal (attention.rs:172-206) on four values of a head: pairs
 // (x0, x1) -> (x0 c - x1 s, x0 s + x1 c) with the table's (cos, sin).
-__global__ __launch_bounds__(256) void codec_rope_kernel(float* qkv, const float2* table) {
-  const uint32_t t = blockIdx.x;
-  float* row = qkv + size_t(t) * 3072u;
-#pragma unroll
-  for (uint32_t k = 0; k < 4; ++k) {
-    const uint32_t p = threadIdx.x + 256u * k;  // pair 0..1023 over q (0..511) and k (512..1023)
-    const uint32_t i = p & 31u;
-    float* e = row + 2u * p;
-    const float2 cs = table[size_t(t) * 32u + i];
-    const float x0 = e[0], x1 = e[1];
-    e[0] = __fsub_rn(__fmul_rn(x0, cs.x), __fmul_rn(x1, cs.y));
-    e[1] = __fadd_rn(__fmul_rn(x0, cs.y), __fmul_rn(x1, cs.x));
-  }
+__device__ __forceinline__ float4 rope4(float4 x, const float2* cs) {
+  const float4 t = *reinterpret_cast<const float4*>(cs);  // c0, s0, c1, s1
+  return make_float4(__fsub_rn(__fmul_rn(x.x, t.x), __fmul_rn(x.y, t.y)),
+                     __fadd_rn(__fmul_rn(x.x, t.y), __fmul_rn(x.y, t.x)),
+                     __fsub_rn(__fmul_rn(x.z, t.z), __fmul_rn(x.w, t.w)),
+                     __fadd_rn(__fmul_rn(x.z, t.w), __fmul_rn(x.w, t.z)));
 }
 
 // Windowed causal attention of the post-module transformer
 // (forward_codec_transformer_layer_with_window, codec.rs:3278-3300, over
 // gqa_decode_attention, attention.rs:208-247): block = 16 queries x one head,
-// the 143 keys / values those queries see ([q0 - 127, q0 + 15]) staged in LDS
+// the 143 keys / values those queries see ([q0 - 127, q0 + 15]) staged in LDS,
+// q and k turned by RoPE as they are
 // (key rows padded to 68 floats: 16-byte aligned, and a 16-lane phase of
 // float4 reads covers all 64 banks).  A wave takes 4 queries: lane j scores
 // keys j and j + 64 of the query's window (four partial sums per dot
 // product), softmax over the wave, the probabilities go through wave-private
 // LDS, and lane d sums p_k v_k[d] (four partial sums).
 constexpr uint32_t CA_Q = 16, CA_W = 128, CA_K = CA_Q + CA_W - 1, CA_KS = 68;
-__global__ __launch_bounds__(256) void codec_attn_kernel(const float* qkv, uint32_t T, float* out) {
+__global__ __launch_bounds__(256) void codec_attn_kernel(const float* qkv, uint32_t T, const float2* table,
+                                                         float* out) {
   __shared__ __align__(16) float ks[CA_K * CA_KS];
   __shared__ __align__(16) float vs[CA_K * 64];
   __shared__ __align__(16) float qs[CA_Q * 64];
@@ -503,13 +498,16 @@ __global__ __launch_bounds__(256) void codec_attn_kernel(const float* qkv, uint3
   for (uint32_t e = tid; e < nk * 16u; e += 256u) {
     const uint32_t r = e >> 4, d4 = (e & 15u) * 4u;
     const float* src = qkv + size_t(kstart + r) * 3072u + h * 64u + d4;
-    *reinterpret_cast<float4*>(ks + r * CA_KS + d4) = *reinterpret_cast<const float4*>(src + 1024);
+    *reinterpret_cast<float4*>(ks + r * CA_KS + d4) =
+        rope4(*reinterpret_cast<const float4*>(src + 1024), table + size_t(kstart + r) * 32u + d4 / 2u);
     *reinterpret_cast<float4*>(vs + r * 64u + d4) = *reinterpret_cast<const float4*>(src + 2048);
   }
   {
     const uint32_t r = tid >> 4, d4 = (tid & 15u) * 4u;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (q0 + r < T) v = *reinterpret_cast<const float4*>(qkv + size_t(q0 + r) * 3072u + h * 64u + d4);
+    if (q0 + r < T)
+      v = rope4(*reinterpret_cast<const float4*>(qkv + size_t(q0 + r) * 3072u + h * 64u + d4),
+                table + size_t(q0 + r) * 32u + d4 / 2u);
     *reinterpret_cast<float4*>(qs + r * 64u + d4) = v;
   }
   __syncthreads();
@@ -565,13 +563,6 @@ __global__ __launch_bounds__(256) void codec_attn_kernel(const float* qkv, uint3
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-}
-
-__global__ __launch_bounds__(256) void codec_scaled_residual_kernel(float* x, const float* p, const float* scale,
-                                                                    size_t n, uint32_t D) {
-  const size_t i = size_t(blockIdx.x) * 256u + threadIdx.x;
-  if (i >= n) return;
-  x[i] = __fadd_rn(x[i], __fmul_rn(p[i], scale[i % D]));
 }
 
 __global__ __launch_bounds__(256) void codec_split16_kernel(const float* x, _Float16* hi, _Float16* lo, size_t n,
@@ -715,6 +706,18 @@ hipError_t conv_gemm_launch(const ConvGemmArgs& a, uint32_t phases, hipStream_t 
   return hipGetLastError();
 }
 
+// Frames per wave: 64, or 32 where those tiles would leave fewer than two
+// blocks per CU (37 code frames, us: transposed convs 34 / 50 / 43 / 33 -> 30 /
+// 38 / 36 / 26, residual units of blocks 3 and 4 52 / 39 -> 43 / 31; at 512 code
+// frames the 32-frame tiles lose, 376 -> 424 for block 3's transposed conv).
+template <int G, int PL, int MC, int WMG, int NB, int NA, bool FU, int OS>
+hipError_t conv_gemm_frames(const ConvGemmArgs& a, uint32_t phases, hipStream_t s) {
+  constexpr uint32_t MT = 32 * MC * WMG, FT = 64 * (4 / WMG);
+  const uint32_t blocks = (a.M + MT - 1) / MT * ((a.F + FT - 1) / FT) * phases;
+  if (blocks < 512u) return conv_gemm_launch<G, PL, MC, 1, WMG, NB, NA, FU, OS>(a, phases, s);
+  return conv_gemm_launch<G, PL, MC, 2, WMG, NB, NA, FU, OS>(a, phases, s);
+}
+
 }  // namespace
 
 uint32_t conv_tile_rows(uint32_t M) { return M % 192u == 0 ? 192u : M % 96u == 0 ? 96u : 256u; }
@@ -731,13 +734,13 @@ hipError_t launch_conv_gemm(const ConvGemmArgs& a, uint32_t phases, hipStream_t 
   const uint32_t MT = conv_tile_rows(a.M);
   if (a.M % MT || a.ostride != phases) return hipErrorInvalidValue;
   const uint32_t os = a.ostride;
-  if (MT == 192 && a.G == 7 && !split && os == 1) return conv_gemm_launch<7, 1, 3, 2, 2, 3, 2, false, 1>(a, phases, s);
-  if (MT == 192 && a.G == 1 && !split && os == 1) return conv_gemm_launch<1, 1, 3, 2, 2, 3, 3, false, 1>(a, phases, s);
-  if (MT == 192 && a.G == 2 && split && os == 8) return conv_gemm_launch<2, 2, 3, 2, 2, 3, 2, false, 8>(a, phases, s);
-  if (MT == 192 && a.G == 2 && split && os == 4) return conv_gemm_launch<2, 2, 3, 2, 2, 3, 2, false, 4>(a, phases, s);
-  if (MT == 96 && a.G == 2 && split && os == 2) return conv_gemm_launch<2, 2, 3, 2, 1, 2, 2, false, 2>(a, phases, s);
-  if (MT == 256 && a.G == 1 && split && os == 2) return conv_gemm_launch<1, 2, 4, 2, 2, 2, 2, false, 2>(a, phases, s);
-  if (MT == 256 && a.G == 1 && split && os == 1) return conv_gemm_launch<1, 2, 4, 2, 2, 2, 2, false, 1>(a, phases, s);
+  if (MT == 192 && a.G == 7 && !split && os == 1) return conv_gemm_frames<7, 1, 3, 2, 3, 2, false, 1>(a, phases, s);
+  if (MT == 192 && a.G == 1 && !split && os == 1) return conv_gemm_frames<1, 1, 3, 2, 3, 3, false, 1>(a, phases, s);
+  if (MT == 192 && a.G == 2 && split && os == 8) return conv_gemm_frames<2, 2, 3, 2, 3, 2, false, 8>(a, phases, s);
+  if (MT == 192 && a.G == 2 && split && os == 4) return conv_gemm_frames<2, 2, 3, 2, 3, 2, false, 4>(a, phases, s);
+  if (MT == 96 && a.G == 2 && split && os == 2) return conv_gemm_frames<2, 2, 3, 1, 2, 2, false, 2>(a, phases, s);
+  if (MT == 256 && a.G == 1 && split && os == 2) return conv_gemm_frames<1, 2, 4, 2, 2, 2, false, 2>(a, phases, s);
+  if (MT == 256 && a.G == 1 && split && os == 1) return conv_gemm_frames<1, 2, 4, 2, 2, 2, false, 1>(a, phases, s);
   return hipErrorInvalidValue;
 }
 
@@ -746,8 +749,8 @@ bool residual_unit_fits(uint32_t M) { return M == 96 || M == 192; }
 hipError_t launch_residual_unit(const ConvGemmArgs& a, hipStream_t s) {
   if (!a.w1 || !a.bias_mid || !a.alpha_mid || !residual_unit_fits(a.M) || a.G != 7 || a.xl || a.C != a.M || a.F == 0)
     return hipErrorInvalidValue;
-  if (a.M == 192) return conv_gemm_launch<7, 1, 3, 2, 2, 3, 2, true, 1>(a, 1, s);
-  return conv_gemm_launch<7, 1, 3, 2, 1, 4, 2, true, 1>(a, 1, s);
+  if (a.M == 192) return conv_gemm_frames<7, 1, 3, 2, 3, 2, true, 1>(a, 1, s);
+  return conv_gemm_frames<7, 1, 3, 1, 4, 2, true, 1>(a, 1, s);
 }
 
 hipError_t launch_codec_rvq(const RvqArgs& a, hipStream_t s) {
@@ -763,23 +766,9 @@ hipError_t launch_codec_check_codes(const int32_t* codes, uint32_t F, uint32_t* 
   return hipGetLastError();
 }
 
-hipError_t launch_codec_rope(float* qkv, uint32_t T, const float2* table, hipStream_t s) {
+hipError_t launch_codec_attention(const float* qkv, uint32_t T, const float2* table, float* out, hipStream_t s) {
   if (T == 0) return hipSuccess;
-  codec_rope_kernel<<<T, 256, 0, s>>>(qkv, table);
-  return hipGetLastError();
-}
-
-hipError_t launch_codec_attention(const float* qkv, uint32_t T, float* out, hipStream_t s) {
-  if (T == 0) return hipSuccess;
-  codec_attn_kernel<<<dim3((T + CA_Q - 1) / CA_Q, 16), 256, 0, s>>>(qkv, T, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_codec_scaled_residual(float* x, const float* p, const float* scale, uint32_t T, uint32_t D,
-                                        hipStream_t s) {
-  const size_t n = size_t(T) * D;
-  if (n == 0) return hipSuccess;
-  codec_scaled_residual_kernel<<<uint32_t((n + 255) / 256), 256, 0, s>>>(x, p, scale, n, D);
+  codec_attn_kernel<<<dim3((T + CA_Q - 1) / CA_Q, 16), 256, 0, s>>>(qkv, T, table, out);
   return hipGetLastError();
 }
 

@@ -4,8 +4,8 @@
 //
 // Weights come from the codec GGUF (decode-side tensors, names and dims as
 // the reference's registry reads them) and stay resident in HBM: small
-// vectors as f32, transformer linears as their F16 rows (the MFMA prefill
-// GEMM's layout), convolution weights packed for conv_gemm_kernel.  Buffers
+// vectors as f32, transformer linears in the fragment order of the prefill
+// product, convolution weights packed for conv_gemm_kernel.  Buffers
 // are sized once for max_frames code frames.
 
 #include <hip/hip_runtime.h>
@@ -250,11 +250,19 @@ class CodecEngine {
     for (size_t i = 0; i < v.size(); ++i) v[i] = half_to_float(p[i]);
     return upload_vec(v);
   }
-  uint8_t* rows(const std::string& name, std::vector<uint64_t> dims) {
+  // an F16 linear [out][in] in the fragment order of the prefill product
+  uint8_t* linear_tiles(const std::string& name, std::vector<uint64_t> dims) {
     const GgufTensor& t = tensor(name, dims);
-    uint8_t* d = dalloc<uint8_t>(t.bytes + 256);
-    CHK(hipMemcpy(d, t.data, t.bytes, hipMemcpyHostToDevice));
-    CHK(hipMemset(d + t.bytes, 0, 256));
+    const uint32_t in = uint32_t(dims[0]), out = uint32_t(dims[1]);
+    uint8_t* d = dalloc<uint8_t>(size_t(bmm_rows_pad(out)) * in * 2);
+    void* src = nullptr;
+    CHK(hipMalloc(&src, t.bytes));
+    hipError_t e = hipMemcpy(src, t.data, t.bytes, hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+      e = launch_tile_f16(static_cast<const uint16_t*>(src), in, out, 0, NO_ROW, reinterpret_cast<uint16_t*>(d), stream_);
+    if (e == hipSuccess) e = hipStreamSynchronize(stream_);
+    (void)hipFree(src);
+    CHK(e);
     return d;
   }
   template <class Src>
@@ -333,11 +341,11 @@ class CodecEngine {
       L.ffn_norm = vec(p + ".ffn_norm.weight", {H});
       L.als = vec(p + ".attention_layer_scale.gamma", {H});
       L.fls = vec(p + ".ffn_layer_scale.gamma", {H});
-      L.wqkv = rows(p + ".attention.wqkv.weight", {H, QKV});
-      L.wo = rows(p + ".attention.wo.weight", {H, H});
-      L.w1 = rows(p + ".feed_forward.w1.weight", {H, FFN});
-      L.w2 = rows(p + ".feed_forward.w2.weight", {FFN, H});
-      L.w3 = rows(p + ".feed_forward.w3.weight", {H, FFN});
+      L.wqkv = linear_tiles(p + ".attention.wqkv.weight", {H, QKV});
+      L.wo = linear_tiles(p + ".attention.wo.weight", {H, H});
+      L.w1 = linear_tiles(p + ".feed_forward.w1.weight", {H, FFN});
+      L.w2 = linear_tiles(p + ".feed_forward.w2.weight", {FFN, H});
+      L.w3 = linear_tiles(p + ".feed_forward.w3.weight", {H, FFN});
     }
     post_norm_ = vec("quantizer.post_module.norm.weight", {H});
     for (uint32_t s = 0; s < 2; ++s) {
@@ -402,7 +410,6 @@ class CodecEngine {
     qkv_ = dalloc<float>(F * QKV);
     att_ = dalloc<float>(F * H);
     act_ = dalloc<float>(F * FFN);
-    proj_ = dalloc<float>(F * H);
     pxh_ = dalloc<_Float16>(npad_ * FFN);
     pxl_ = dalloc<_Float16>(npad_ * FFN);
     prs_ = dalloc<float>(npad_);
@@ -461,12 +468,14 @@ class CodecEngine {
     CHK(launch_codec_rvq(a, stream_));
   }
 
+  // y (op)= product of the planes in pxh_ / pxl_; scale: y += scale * product,
+  // after which the planes of y (RMSNorm gain next, nullable) are the input of
+  // the next product
   void gemm(const uint8_t* w, const uint8_t* w3, uint32_t in, uint32_t out, int epi, uint32_t n, float* y,
-            uint32_t ldy) {
+            uint32_t ldy, const float* scale = nullptr, const float* next = nullptr) {
     GemmArgs g{};
-    g.w = w;
-    g.w3 = w3;
-    g.row_bytes = size_t(in) * 2;
+    g.wt = w;
+    g.wt3 = w3;
     g.M = out;
     g.K = in;
     g.xh = pxh_;
@@ -477,6 +486,8 @@ class CodecEngine {
     g.ldy = ldy;
     g.part = part_;
     g.part_cap = part_cap_;
+    g.scale = scale;
+    if (next) g.next = GemmNext{next, 1e-5f, gemm_rows_pad(n), pxh_, pxl_, prs_};
     CHK(launch_gemm_mfma(W_F16, epi, g, stream_));
   }
   void split(const float* x, uint32_t ld, const float* norm, uint32_t n, uint32_t k) {
@@ -487,18 +498,14 @@ class CodecEngine {
   void post_module(uint32_t n) {
     for (uint32_t l = 0; l < LAYERS; ++l) {
       const Layer& L = layers_[l];
-      split(lat_, H, L.attn_norm, n, H);
+      if (l == 0) split(lat_, H, L.attn_norm, n, H);
       gemm(L.wqkv, nullptr, H, QKV, EPI_STORE, n, qkv_, QKV);
-      CHK(launch_codec_rope(qkv_, n, rope_, stream_));
-      CHK(launch_codec_attention(qkv_, n, att_, stream_));
+      CHK(launch_codec_attention(qkv_, n, rope_, att_, stream_));
       split(att_, H, nullptr, n, H);
-      gemm(L.wo, nullptr, H, H, EPI_STORE, n, proj_, H);
-      CHK(launch_codec_scaled_residual(lat_, proj_, L.als, n, H, stream_));
-      split(lat_, H, L.ffn_norm, n, H);
+      gemm(L.wo, nullptr, H, H, EPI_RESID, n, lat_, H, L.als, L.ffn_norm);
       gemm(L.w1, L.w3, H, FFN, EPI_SWIGLU_FAST, n, act_, FFN);
       split(act_, FFN, nullptr, n, FFN);
-      gemm(L.w2, nullptr, FFN, H, EPI_STORE, n, proj_, H);
-      CHK(launch_codec_scaled_residual(lat_, proj_, L.fls, n, H, stream_));
+      gemm(L.w2, nullptr, FFN, H, EPI_RESID, n, lat_, H, L.fls, l + 1 < LAYERS ? layers_[l + 1].attn_norm : nullptr);
     }
     CHK(launch_rms_norm(lat_, post_norm_, hid_, H, n, 1e-5f, nullptr, stream_));
   }
@@ -732,7 +739,7 @@ class CodecEngine {
   size_t npad_ = 0, part_cap_ = 0;
   int32_t* codes_ = nullptr;
   uint32_t* err_ = nullptr;
-  float *lat_ = nullptr, *hid_ = nullptr, *qkv_ = nullptr, *att_ = nullptr, *act_ = nullptr, *proj_ = nullptr;
+  float *lat_ = nullptr, *hid_ = nullptr, *qkv_ = nullptr, *att_ = nullptr, *act_ = nullptr;
   _Float16 *pxh_ = nullptr, *pxl_ = nullptr;
   float *prs_ = nullptr, *part_ = nullptr;
   float *up32_ = nullptr, *upx_ = nullptr;

@@ -208,7 +208,8 @@ class Engine {
   void validate_prompt(const int32_t* prompt, size_t cols);
   void validate_tokens(const int32_t* flat, size_t n_tok);
   void mm(const DevLin& L, const DevLin* L3, int epi, const float* x, uint32_t ldx, const float* norm, float eps,
-          uint32_t n, uint32_t npad, float* y, uint32_t ldy);
+          uint32_t n, uint32_t npad, float* y, uint32_t ldy,
+          const float* next = nullptr);
   // batched columns (3..16): split planes + skinny MFMA product
   void mm_skinny(const DevLin& L, const DevLin* L3, int epi, const float* x, uint32_t ldx, const float* norm,
                  float eps, uint32_t n, float* y, uint32_t ldy, uint32_t row_base, uint32_t extra_row,
@@ -1076,10 +1077,12 @@ void Engine::enqueue_frame(const SamplerCfg& cfg, uint32_t nseq, size_t codes_st
 // QK-norm + RoPE + KV append for all of the chunk's positions, then causal
 // attention of each token over the cache.  One slot (`seq`) at a time;
 // leaves the last token's residual row in decode column 0 for the output head.
+// x null: the product before has left this one's planes (`next`, its RMSNorm gain).
 void Engine::mm(const DevLin& L, const DevLin* L3, int epi, const float* x, uint32_t ldx, const float* norm, float eps,
-                uint32_t n, uint32_t npad, float* y, uint32_t ldy) {
-  HIPC(launch_split_rows(x, ldx, norm, eps, n, npad, L.in, pxh_, pxl_, prs_, nullptr, stream_));
+                uint32_t n, uint32_t npad, float* y, uint32_t ldy, const float* next) {
+  if (x) HIPC(launch_split_rows(x, ldx, norm, eps, n, npad, L.in, pxh_, pxl_, prs_, nullptr, stream_));
   GemmArgs g{};
+  if (next) g.next = GemmNext{next, spec.eps, npad, pxh_, pxl_, prs_};
   g.w = L.w;
   g.w3 = L3 ? L3->w : nullptr;
   if (L.wt && (!L3 || L3->wt)) {
@@ -1192,7 +1195,7 @@ void Engine::enqueue_prefill(const int32_t* prompt_dev, size_t n_tok, uint32_t s
       const SlowLayer& L = slow_[l];
       float* kcl = kvp(kc_, size_t(seq) * slot_kv_ + size_t(l) * kv * s.max_seq_len);
       float* vcl = kvp(vc_, size_t(seq) * slot_kv_ + size_t(l) * kv * s.max_seq_len);
-      mm(L.wqkv, nullptr, EPI_STORE, ph_, s.dim, L.attn_norm, s.eps, nc, npad, pqkv_, qkv_w);
+      mm(L.wqkv, nullptr, EPI_STORE, l == 0 ? ph_ : nullptr, s.dim, L.attn_norm, s.eps, nc, npad, pqkv_, qkv_w);
       QkvPostArgs qa{};
       qa.qkv = pqkv_;
       qa.q_out = pq_;
@@ -1230,9 +1233,10 @@ void Engine::enqueue_prefill(const int32_t* prompt_dev, size_t n_tok, uint32_t s
       pa.part = ppart_;
       pa.part_cap = ppart_cap_;
       HIPC(launch_attention_prefill(pa, stream_));
-      mm(L.wo, nullptr, EPI_RESID, patt_, q, nullptr, 0.0f, nc, npad, ph_, s.dim);
-      mm(L.w1, &L.w3, EPI_SWIGLU_SLOW, ph_, s.dim, L.ffn_norm, s.eps, nc, npad, pact_, s.ffn);
-      mm(L.w2, nullptr, EPI_RESID, pact_, s.ffn, nullptr, 0.0f, nc, npad, ph_, s.dim);
+      mm(L.wo, nullptr, EPI_RESID, patt_, q, nullptr, 0.0f, nc, npad, ph_, s.dim, L.ffn_norm);
+      mm(L.w1, &L.w3, EPI_SWIGLU_SLOW, nullptr, s.dim, L.ffn_norm, s.eps, nc, npad, pact_, s.ffn);
+      mm(L.w2, nullptr, EPI_RESID, pact_, s.ffn, nullptr, 0.0f, nc, npad, ph_, s.dim,
+         l + 1 < s.slow_layers ? slow_[l + 1].attn_norm : nullptr);
     }
     HIPC(launch_add_position(st, nc, 1, stream_));
     t += nc;

@@ -302,10 +302,22 @@ hipError_t launch_split_rows(const float* x, uint32_t ldx, const float* norm, fl
 
 // MFMA product y[n][m] (op)= rs[n] * sum_k W[m][k] * x[n][k] for n < N, m < M,
 // x given as the split planes; epilogues as for launch_gemv (SwiGLU uses w3).
+// scale (nullable, EPI_RESID): y[n][m] += scale[m] * product.
+// next (EPI_RESID): the rows y are the next product's input: their planes are
+// written as by launch_split_rows (for short products in one pass with the
+// K splits' sum).  Its planes and rs may be this product's own.
 // part (nullable): workspace of part_cap floats for K-split partial sums
 // (gemm_part_floats(Npad, M) floats lets every short-M product split as it would).
 // wt (and wt3): the weights in the fragment order of launch_tile_f16 /
 // launch_tile_q (then with the scales ws, ws3), or null and the rows themselves.
+struct GemmNext {
+  const float* norm;  // nullable
+  float eps;
+  uint32_t npad;      // 0: no next product
+  _Float16* xh;
+  _Float16* xl;
+  float* rs;
+};
 struct GemmArgs {
   const uint8_t* w;
   const uint8_t* w3;
@@ -323,6 +335,8 @@ struct GemmArgs {
   uint32_t ldy;
   float* part;
   size_t part_cap;
+  const float* scale;
+  GemmNext next;
 };
 size_t gemm_part_floats(uint32_t n_pad, uint32_t m);
 hipError_t launch_gemm_mfma(uint32_t wtype, int epi, const GemmArgs& a, hipStream_t s);

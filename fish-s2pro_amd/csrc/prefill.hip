@@ -101,6 +101,57 @@ __device__ __forceinline__ float split_scale(float mx) {
   return r;
 }
 
+// RMSNorm (if has_norm) and split of row n, held as float4s tid + 256 i (zeros
+// past the row's end) with the gains g; the block's 256 threads.
+template <int R>
+__device__ __forceinline__ void split_row_regs(float4 (&v)[R], const float4 (&g)[R], bool has_norm, float eps,
+                                               uint32_t n, uint32_t K, _Float16* xh, _Float16* xl, float* rs,
+                                               uint32_t* err, float* red) {
+  const uint32_t tid = threadIdx.x, K4 = K / 4;
+  float scale = 1.0f;
+  if (has_norm) {
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < R; ++i) ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+    const float tot = block_reduce_sum4(ss, red);
+    scale = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(tot, float(K)), eps)));
+  }
+  float mx = 0.0f;
+  bool nf = false;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (has_norm) {
+      v[i].x = __fmul_rn(__fmul_rn(v[i].x, scale), g[i].x);
+      v[i].y = __fmul_rn(__fmul_rn(v[i].y, scale), g[i].y);
+      v[i].z = __fmul_rn(__fmul_rn(v[i].z, scale), g[i].z);
+      v[i].w = __fmul_rn(__fmul_rn(v[i].w, scale), g[i].w);
+    }
+    mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
+    // fmaxf drops NaN: non-finite values are flagged on their own
+    nf = nf || !(fabsf(v[i].x) <= 3.4028235e38f) || !(fabsf(v[i].y) <= 3.4028235e38f) ||
+         !(fabsf(v[i].z) <= 3.4028235e38f) || !(fabsf(v[i].w) <= 3.4028235e38f);
+  }
+  if (__any(nf) && (tid & 63u) == 0 && err) atomicOr(err, ERR_NONFINITE);
+  const float r = split_scale(block_reduce_max4(mx, red));
+  const float inv = 1.0f / r;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const uint32_t j = tid + 256u * i;
+    if (j >= K4) continue;
+    const float e[4] = {v[i].x * inv, v[i].y * inv, v[i].z * inv, v[i].w * inv};
+    _Float16 h[4], l[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      h[c] = _Float16(e[c]);
+      l[c] = _Float16(e[c] - float(h[c]));
+    }
+    const size_t o = plane_off(n, 4 * j, K) + (j & 1u) * 4u;
+    *reinterpret_cast<uint2*>(xh + o) = *reinterpret_cast<const uint2*>(h);
+    *reinterpret_cast<uint2*>(xl + o) = *reinterpret_cast<const uint2*>(l);
+  }
+  if (tid == 0) rs[n] = r;
+}
+
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* x, uint32_t ldx, const float* norm, float eps,
                                                          uint32_t N, uint32_t K, _Float16* xh, _Float16* xl,
                                                          float* rs, uint32_t* err) {
@@ -124,48 +175,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* x, uint32_
       v[i] = j < K4 ? *reinterpret_cast<const float4*>(xr + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
       g[i] = (norm && j < K4) ? *reinterpret_cast<const float4*>(norm + 4 * j) : make_float4(1.f, 1.f, 1.f, 1.f);
     }
-    float scale = 1.0f;
-    if (norm) {
-      float ss = 0.0f;
-#pragma unroll
-      for (int i = 0; i < SR_REG; ++i) ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
-      const float tot = block_reduce_sum4(ss, red);
-      scale = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(tot, float(K)), eps)));
-    }
-    float mx = 0.0f;
-    bool nf = false;
-#pragma unroll
-    for (int i = 0; i < SR_REG; ++i) {
-      if (norm) {
-        v[i].x = __fmul_rn(__fmul_rn(v[i].x, scale), g[i].x);
-        v[i].y = __fmul_rn(__fmul_rn(v[i].y, scale), g[i].y);
-        v[i].z = __fmul_rn(__fmul_rn(v[i].z, scale), g[i].z);
-        v[i].w = __fmul_rn(__fmul_rn(v[i].w, scale), g[i].w);
-      }
-      mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
-      // fmaxf drops NaN: non-finite values are flagged on their own
-      nf = nf || !(fabsf(v[i].x) <= 3.4028235e38f) || !(fabsf(v[i].y) <= 3.4028235e38f) ||
-           !(fabsf(v[i].z) <= 3.4028235e38f) || !(fabsf(v[i].w) <= 3.4028235e38f);
-    }
-    if (__any(nf) && (tid & 63u) == 0 && err) atomicOr(err, ERR_NONFINITE);
-    const float r = split_scale(block_reduce_max4(mx, red));
-    const float inv = 1.0f / r;
-#pragma unroll
-    for (int i = 0; i < SR_REG; ++i) {
-      const uint32_t j = tid + 256u * i;
-      if (j >= K4) continue;
-      const float e[4] = {v[i].x * inv, v[i].y * inv, v[i].z * inv, v[i].w * inv};
-      _Float16 h[4], l[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        h[c] = _Float16(e[c]);
-        l[c] = _Float16(e[c] - float(h[c]));
-      }
-      const size_t o = plane_off(n, 4 * j, K) + (j & 1u) * 4u;
-      *reinterpret_cast<uint2*>(xh + o) = *reinterpret_cast<const uint2*>(h);
-      *reinterpret_cast<uint2*>(xl + o) = *reinterpret_cast<const uint2*>(l);
-    }
-    if (tid == 0) rs[n] = r;
+    split_row_regs<SR_REG>(v, g, norm != nullptr, eps, n, K, xh, xl, rs, err, red);
     return;
   }
   float scale = 1.0f;
@@ -298,7 +308,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, const floatx16 
             const float gg = g[tm] * a.rs[n];
             float* dst = a.y + size_t(n) * a.ldy + m;
             if constexpr (EPI == EPI_STORE) *dst = gg;
-            else *dst = __fadd_rn(*dst, gg);
+            else *dst = __fadd_rn(*dst, a.scale ? __fmul_rn(gg, a.scale[m]) : gg);
           }
         }
       }
@@ -514,7 +524,7 @@ __device__ __forceinline__ void gemm_store(const GemmArgs& a, const floatx16 (&a
             const float g = acc[i][j][v] * r;
             float* dst = a.y + size_t(n) * a.ldy + m;
             if constexpr (EPI == EPI_STORE) *dst = g;
-            else *dst = __fadd_rn(*dst, g);
+            else *dst = __fadd_rn(*dst, a.scale ? __fmul_rn(g, a.scale[m]) : g);
           }
         }
       }
@@ -815,8 +825,77 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmArgs a, uint
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     if constexpr (EPI == EPI_STORE) dst[e] = v[e];
-    else dst[e] = __fadd_rn(dst[e], v[e]);
+    else dst[e] = __fadd_rn(dst[e], a.scale ? __fmul_rn(v[e], a.scale[m + e]) : v[e]);
   }
+}
+
+// The sum of the K splits, the residual and the next product's RMSNorm and
+// split in one pass over the row (one block per row, M <= 1024 R): the values
+// and the order of every addition are those of gemm_split_reduce_kernel and
+// split_rows_kernel, whose second read of the rows and second launch it saves
+// (256-token prompt 8.33 -> 8.27 ms, 37 code frames 1.605 -> 1.573 ms; past
+// GEMM_WIDE_N rows the launch is nothing and the two kernels are as fast,
+// 1500-token prompt 34.2 against 34.5 ms).
+template <int R>
+__global__ __launch_bounds__(256) void gemm_reduce_split_kernel(GemmArgs a, uint32_t splits) {
+  __shared__ float red[4];
+  const uint32_t n = blockIdx.x, tid = threadIdx.x, K = a.M, K4 = K / 4;
+  if (n >= a.N) {
+    for (uint32_t k = tid * 8u; k < K; k += 2048u) {
+      *reinterpret_cast<uint4*>(a.next.xh + plane_off(n, k, K)) = make_uint4(0u, 0u, 0u, 0u);
+      *reinterpret_cast<uint4*>(a.next.xl + plane_off(n, k, K)) = make_uint4(0u, 0u, 0u, 0u);
+    }
+    if (tid == 0) a.next.rs[n] = 1.0f;
+    return;
+  }
+  const size_t plane = size_t(a.N) * K;
+  const float* p = a.part + size_t(n) * K;
+  float* y = a.y + size_t(n) * a.ldy;
+  const float r = a.rs[n];
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f), one = make_float4(1.f, 1.f, 1.f, 1.f);
+  float4 v[R], g[R], o[R], c[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const uint32_t j = tid + 256u * i;
+    const bool in = j < K4;
+    v[i] = in ? *reinterpret_cast<const float4*>(p + 4 * j) : zero;
+    o[i] = in ? *reinterpret_cast<const float4*>(y + 4 * j) : zero;
+    g[i] = in && a.next.norm ? *reinterpret_cast<const float4*>(a.next.norm + 4 * j) : one;
+    c[i] = in && a.scale ? *reinterpret_cast<const float4*>(a.scale + 4 * j) : one;
+  }
+  // splits 1 .. in batches whose loads are in flight together
+  for (uint32_t k0 = 1; k0 < splits; k0 += 4) {
+    float4 t[4][R];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const uint32_t j = tid + 256u * i;
+        t[k][i] = j < K4 ? *reinterpret_cast<const float4*>(p + min(k0 + k, splits - 1u) * plane + 4 * j) : zero;
+      }
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      if (k0 + k >= splits) break;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        v[i].x += t[k][i].x;
+        v[i].y += t[k][i].y;
+        v[i].z += t[k][i].z;
+        v[i].w += t[k][i].w;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const uint32_t j = tid + 256u * i;
+    // (a gain of exactly one changes nothing)
+    v[i].x = __fadd_rn(o[i].x, __fmul_rn(v[i].x * r, c[i].x));
+    v[i].y = __fadd_rn(o[i].y, __fmul_rn(v[i].y * r, c[i].y));
+    v[i].z = __fadd_rn(o[i].z, __fmul_rn(v[i].z * r, c[i].z));
+    v[i].w = __fadd_rn(o[i].w, __fmul_rn(v[i].w * r, c[i].w));
+    if (j < K4) *reinterpret_cast<float4*>(y + 4 * j) = v[i];
+  }
+  split_row_regs<R>(v, g, a.next.norm != nullptr, a.next.eps, n, K, a.next.xh, a.next.xl, a.next.rs, nullptr, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -1347,13 +1426,29 @@ static hipError_t gemm_dma(int epi, const GemmArgs& a, const GemmPlan& p, hipStr
   }
 }
 
+constexpr uint32_t GEMM_NEXT_MAX = 3072;  // widest row of gemm_reduce_split_kernel
+static bool gemm_next_fused(const GemmArgs& a, uint32_t splits) {
+  return a.next.npad && splits > 1 && a.N <= GEMM_WIDE_N && a.M <= GEMM_NEXT_MAX && a.M % 32 == 0 && a.ldy % 4 == 0;
+}
 static hipError_t gemm_reduce(int epi, const GemmArgs& a, uint32_t splits, hipStream_t s) {
+  if (gemm_next_fused(a, splits)) {
+    hipLaunchKernelGGL((gemm_reduce_split_kernel<GEMM_NEXT_MAX / 1024>), dim3(a.next.npad), dim3(256), 0, s, a, splits);
+    return hipGetLastError();
+  }
   const dim3 rgrid(uint32_t((size_t(a.N) * (a.M / 4u) + 255u) / 256u)), block(256);
   if (epi == EPI_STORE)
     hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI_STORE>), rgrid, block, 0, s, a, splits);
   else
     hipLaunchKernelGGL((gemm_split_reduce_kernel<EPI_RESID>), rgrid, block, 0, s, a, splits);
   return hipGetLastError();
+}
+
+// What follows the product kernel: the splits' sum and the next product's planes.
+static hipError_t gemm_finish(int epi, const GemmArgs& a, uint32_t splits, hipStream_t s) {
+  const hipError_t e = splits == 1 ? hipSuccess : gemm_reduce(epi, a, splits, s);
+  if (e != hipSuccess || !a.next.npad || gemm_next_fused(a, splits)) return e;
+  return launch_split_rows(a.y, a.ldy, a.next.norm, a.next.eps, a.N, a.next.npad, a.M, a.next.xh, a.next.xl, a.next.rs,
+                           nullptr, s);
 }
 
 template <uint32_t WT>
@@ -1380,7 +1475,7 @@ static hipError_t gemm_epi(int epi, const GemmArgs& a, uint32_t m_tiles, uint32_
     default: return hipErrorInvalidValue;
   }
   const hipError_t e = hipGetLastError();
-  return e != hipSuccess || splits == 1 ? e : gemm_reduce(epi, a, splits, s);
+  return e != hipSuccess ? e : gemm_finish(epi, a, splits, s);
 }
 
 uint32_t gemm_rows_pad(uint32_t n) { return (n + TN - 1) / TN * TN; }
@@ -1392,8 +1487,8 @@ size_t gemm_part_floats(uint32_t n_pad, uint32_t m) {
 
 hipError_t launch_gemm_mfma(uint32_t wtype, int epi, const GemmArgs& a, hipStream_t s) {
   if (a.K % KS || a.M == 0 || a.N == 0) return hipErrorInvalidValue;
+  if ((a.scale || a.next.npad) && epi != EPI_RESID) return hipErrorInvalidValue;
   const bool dual = epi == EPI_SWIGLU_SLOW || epi == EPI_SWIGLU_FAST;
-  if (dual && !a.w3) return hipErrorInvalidValue;
   if (a.wt) {
     if ((dual && !a.wt3) || (wtype != W_F16 && (!a.ws || (dual && !a.ws3)))) return hipErrorInvalidValue;
     const GemmPlan p = gemm_plan(a, dual, wtype != W_F16);
@@ -1401,8 +1496,9 @@ hipError_t launch_gemm_mfma(uint32_t wtype, int epi, const GemmArgs& a, hipStrea
                          : wtype == W_Q8_0 ? gemm_dma<W_Q8_0>(epi, a, p, s)
                          : wtype == W_Q4_0 ? gemm_dma<W_Q4_0>(epi, a, p, s)
                                            : hipErrorInvalidValue;
-    return e != hipSuccess || p.splits == 1 ? e : gemm_reduce(epi, a, p.splits, s);
+    return e != hipSuccess ? e : gemm_finish(epi, a, p.splits, s);
   }
+  if (!a.w || (dual && !a.w3)) return hipErrorInvalidValue;
   const uint32_t m_tiles = dual ? (a.M + 63u) / 64u : (a.M + TM - 1u) / TM;
   const uint32_t n_tiles = gemm_rows_pad(a.N) / TN;
   // short-M products: split K so that the grid covers the 256 CUs (each split
