@@ -195,7 +195,7 @@ class Engine {
   void enqueue_fast_frame(const SamplerCfg& cfg, uint32_t nseq, const uint32_t* done);
   bool fold_greedy(const SamplerCfg& cfg, uint32_t nseq) const;
   void enqueue_frame(const SamplerCfg& cfg, uint32_t nseq, size_t codes_stride);
-  void enqueue_prefill(const int32_t* prompt_dev, size_t n_tok, uint32_t seq);
+  void enqueue_prefill(const int32_t* prompt_dev, const size_t* cols, uint32_t n, uint32_t seq);
   void enqueue_prefill_gemv(const int32_t* prompt_dev, size_t n_tok, uint32_t seq);
   void ensure_slots(uint32_t n);
   void ensure_tiled();
@@ -1075,8 +1075,7 @@ void Engine::enqueue_frame(const SamplerCfg& cfg, uint32_t nseq, size_t codes_st
 // chunks of up to prefill_chunk_ tokens go through each layer together: every
 // linear is one MFMA product over the chunk (weights read once per chunk),
 // QK-norm + RoPE + KV append for all of the chunk's positions, then causal
-// attention of each token over the cache.  One slot (`seq`) at a time;
-// leaves the last token's residual row in decode column 0 for the output head.
+// attention of each token over the cache.
 // x null: the product before has left this one's planes (`next`, its RMSNorm gain).
 void Engine::mm(const DevLin& L, const DevLin* L3, int epi, const float* x, uint32_t ldx, const float* norm, float eps,
                 uint32_t n, uint32_t npad, float* y, uint32_t ldy, const float* next) {
@@ -1160,88 +1159,117 @@ void Engine::enqueue_prefill_gemv(const int32_t* prompt_dev, size_t n_tok, uint3
   if (nc > 1) HIPC(hipMemcpyAsync(h_, h_ + size_t(nc - 1) * s.dim, size_t(s.dim) * 4, hipMemcpyDeviceToDevice, stream_));
 }
 
-void Engine::enqueue_prefill(const int32_t* prompt_dev, size_t n_tok, uint32_t seq) {
-  if (prefill_gemv_) {
-    enqueue_prefill_gemv(prompt_dev, n_tok, seq);
-    return;
-  }
+// The prompts of n requests (slot seq + i, cols[i] tokens, one after another in
+// prompt_dev) go through the layers together: a pass takes the next
+// prefill_chunk_ tokens of whatever requests they belong to, the products run
+// over all of them (8 requests of 300 tokens: 8 products of 300 rows become one
+// of 2048 and one of 352, whose tiles fill the CUs), and QK-norm, RoPE, KV append
+// and attention run request by request on its rows.  Leaves request i's last
+// residual row in decode column i.
+void Engine::enqueue_prefill(const int32_t* prompt_dev, const size_t* cols, uint32_t n, uint32_t seq) {
   const s2hip_spec& s = spec;
   const uint32_t cdim = s.num_codebooks + 1;
   const uint32_t q = s.heads * s.head_dim, kv = s.kv_heads * s.head_dim, qkv_w = q + 2 * kv;
-  DevState* st = st_ + seq;
-  size_t t = 0;
-  uint32_t nc = 0;
-  while (t < n_tok) {
-    nc = uint32_t(std::min<size_t>(prefill_chunk_, n_tok - t));
+  struct Segment {
+    uint32_t req, row, count;  // rows row .. row + count - 1 of the pass are the request's next tokens
+    bool last;
+  };
+  std::vector<Segment> segs;
+  uint32_t req = 0;
+  size_t at = 0, tok = 0;  // tokens of request `req`, and of all, already through
+  while (req < n) {
+    segs.clear();
+    uint32_t nc = 0;
+    while (req < n && nc < prefill_chunk_) {
+      const uint32_t c = uint32_t(std::min<size_t>(prefill_chunk_ - nc, cols[req] - at));
+      at += c;
+      const bool last = at == cols[req];
+      segs.push_back(Segment{req, nc, c, last});
+      nc += c;
+      if (last) {
+        ++req;
+        at = 0;
+      }
+    }
     const uint32_t npad = gemm_rows_pad(nc);
-    EmbedArgs ea{};
-    ea.tokens = prompt_dev + t * cdim;
-    ea.emb = emb_;
-    ea.cb_emb = cb_emb_;
-    ea.h = ph_;
-    ea.n = nc;
-    ea.dim = s.dim;
-    ea.vocab = s.vocab;
-    ea.cb_rows = uint32_t(cb_rows_);
-    ea.num_codebooks = s.num_codebooks;
-    ea.codebook_size = s.codebook_size;
-    ea.sem_begin = s.semantic_begin;
-    ea.sem_end = s.semantic_end;
-    ea.sem_scale = 1.0f / std::sqrt(float(cdim));
-    ea.scale_enabled = s.scale_codebook_embeddings;
-    ea.err = &st->err;
-    HIPC(launch_embed(ea, stream_));
+    for (const Segment& g : segs) {
+      EmbedArgs ea{};
+      ea.tokens = prompt_dev + (tok + g.row) * cdim;
+      ea.emb = emb_;
+      ea.cb_emb = cb_emb_;
+      ea.h = ph_ + size_t(g.row) * s.dim;
+      ea.n = g.count;
+      ea.dim = s.dim;
+      ea.vocab = s.vocab;
+      ea.cb_rows = uint32_t(cb_rows_);
+      ea.num_codebooks = s.num_codebooks;
+      ea.codebook_size = s.codebook_size;
+      ea.sem_begin = s.semantic_begin;
+      ea.sem_end = s.semantic_end;
+      ea.sem_scale = 1.0f / std::sqrt(float(cdim));
+      ea.scale_enabled = s.scale_codebook_embeddings;
+      ea.err = &st_[seq + g.req].err;
+      HIPC(launch_embed(ea, stream_));
+    }
     for (uint32_t l = 0; l < s.slow_layers; ++l) {
       const SlowLayer& L = slow_[l];
-      float* kcl = kvp(kc_, size_t(seq) * slot_kv_ + size_t(l) * kv * s.max_seq_len);
-      float* vcl = kvp(vc_, size_t(seq) * slot_kv_ + size_t(l) * kv * s.max_seq_len);
       mm(L.wqkv, nullptr, EPI_STORE, l == 0 ? ph_ : nullptr, s.dim, L.attn_norm, s.eps, nc, npad, pqkv_, qkv_w);
-      QkvPostArgs qa{};
-      qa.qkv = pqkv_;
-      qa.q_out = pq_;
-      qa.k_cache = kcl;
-      qa.v_cache = vcl;
-      qa.q_norm = L.q_norm;
-      qa.k_norm = L.k_norm;
-      qa.rope = rope_slow_;
-      qa.pos_ptr = &st->n_past;
-      qa.pos_offset = 0;
-      qa.H = s.heads;
-      qa.Hkv = s.kv_heads;
-      qa.hd = s.head_dim;
-      qa.max_seq = s.max_seq_len;
-      qa.ncol = nc;
-      qa.eps = s.eps;
-      qa.err = &st->err;
-      qa.kv_f16 = kv_f16_;
-      HIPC(launch_qkv_post(qa, stream_));
-      PrefillAttnArgs pa{};
-      pa.q = pq_;
-      pa.k_cache = kcl;
-      pa.v_cache = vcl;
-      pa.out = patt_;
-      pa.pos_ptr = &st->n_past;
-      pa.pos_offset = 0;
-      pa.N = nc;
-      pa.H = s.heads;
-      pa.Hkv = s.kv_heads;
-      pa.hd = s.head_dim;
-      pa.max_seq = s.max_seq_len;
-      pa.scale = 1.0f / std::sqrt(float(s.head_dim));  // slow_ar.rs:59-61
-      pa.kv_f16 = kv_f16_;
-      pa.err = &st->err;
-      pa.part = ppart_;
-      pa.part_cap = ppart_cap_;
-      HIPC(launch_attention_prefill(pa, stream_));
+      for (const Segment& g : segs) {
+        const uint32_t sq = seq + g.req;
+        DevState* st = st_ + sq;
+        float* kcl = kvp(kc_, size_t(sq) * slot_kv_ + size_t(l) * kv * s.max_seq_len);
+        float* vcl = kvp(vc_, size_t(sq) * slot_kv_ + size_t(l) * kv * s.max_seq_len);
+        QkvPostArgs qa{};
+        qa.qkv = pqkv_ + size_t(g.row) * qkv_w;
+        qa.q_out = pq_ + size_t(g.row) * q;
+        qa.k_cache = kcl;
+        qa.v_cache = vcl;
+        qa.q_norm = L.q_norm;
+        qa.k_norm = L.k_norm;
+        qa.rope = rope_slow_;
+        qa.pos_ptr = &st->n_past;
+        qa.pos_offset = 0;
+        qa.H = s.heads;
+        qa.Hkv = s.kv_heads;
+        qa.hd = s.head_dim;
+        qa.max_seq = s.max_seq_len;
+        qa.ncol = g.count;
+        qa.eps = s.eps;
+        qa.err = &st->err;
+        qa.kv_f16 = kv_f16_;
+        HIPC(launch_qkv_post(qa, stream_));
+        PrefillAttnArgs pa{};
+        pa.q = pq_ + size_t(g.row) * q;
+        pa.k_cache = kcl;
+        pa.v_cache = vcl;
+        pa.out = patt_ + size_t(g.row) * q;
+        pa.pos_ptr = &st->n_past;
+        pa.pos_offset = 0;
+        pa.N = g.count;
+        pa.H = s.heads;
+        pa.Hkv = s.kv_heads;
+        pa.hd = s.head_dim;
+        pa.max_seq = s.max_seq_len;
+        pa.scale = 1.0f / std::sqrt(float(s.head_dim));  // slow_ar.rs:59-61
+        pa.kv_f16 = kv_f16_;
+        pa.err = &st->err;
+        pa.part = ppart_;
+        pa.part_cap = ppart_cap_;
+        HIPC(launch_attention_prefill(pa, stream_));
+      }
       mm(L.wo, nullptr, EPI_RESID, patt_, q, nullptr, 0.0f, nc, npad, ph_, s.dim, L.ffn_norm);
       mm(L.w1, &L.w3, EPI_SWIGLU_SLOW, nullptr, s.dim, L.ffn_norm, s.eps, nc, npad, pact_, s.ffn);
       mm(L.w2, nullptr, EPI_RESID, pact_, s.ffn, nullptr, 0.0f, nc, npad, ph_, s.dim,
          l + 1 < s.slow_layers ? slow_[l + 1].attn_norm : nullptr);
     }
-    HIPC(launch_add_position(st, nc, 1, stream_));
-    t += nc;
+    for (const Segment& g : segs) {
+      HIPC(launch_add_position(st_ + seq + g.req, g.count, 1, stream_));
+      if (g.last)
+        HIPC(hipMemcpyAsync(h_ + size_t(g.req) * s.dim, ph_ + size_t(g.row + g.count - 1) * s.dim, size_t(s.dim) * 4,
+                            hipMemcpyDeviceToDevice, stream_));
+    }
+    tok += nc;
   }
-  if (nc) HIPC(hipMemcpyAsync(h_, ph_ + size_t(nc - 1) * s.dim, size_t(s.dim) * 4, hipMemcpyDeviceToDevice, stream_));
 }
 
 void Engine::ensure_prompt(size_t n_int) {
@@ -1433,7 +1461,7 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
       enqueue_prefill_gemv(prompt_dev_, n_tok, slot);
       lin_err_ = nullptr;
     } else {
-      enqueue_prefill(prompt_dev_, n_tok, slot);
+      enqueue_prefill(prompt_dev_, &n_tok, 1, slot);
     }
     enqueue_head(1, hn_, logits_c_, logits_out != nullptr, nullptr);
     HIPC(hipMemcpyAsync(hidden_out, hn_, s.dim * 4, hipMemcpyDeviceToHost, stream_));
@@ -1585,11 +1613,14 @@ void Engine::generate(uint32_t nseq, const int32_t* const* prompts, const size_t
   hipEvent_t ev[3];
   for (auto& e : ev) HIPC(hipEventCreate(&e));
   HIPC(hipEventRecord(ev[0], stream_));
-  // prompt prefill and the first semantic sample, request by request
+  // prompt prefill, then the first semantic sample, request by request
+  if (!prefill_gemv_) enqueue_prefill(prompt_dev_, cols, nseq, 0);
   {
     size_t off = 0;
     for (uint32_t b = 0; b < nseq; ++b) {
-      enqueue_prefill(prompt_dev_ + off, cols[b], b);
+      if (prefill_gemv_) enqueue_prefill_gemv(prompt_dev_ + off, cols[b], b);
+      else if (b)  // its last row, to the column the head reads
+        HIPC(hipMemcpyAsync(h_, h_ + size_t(b) * s.dim, size_t(s.dim) * 4, hipMemcpyDeviceToDevice, stream_));
       off += cols[b] * cdim;
       enqueue_head(1, hn_ + size_t(b) * s.dim, logits_c_ + size_t(b) * n_cand_, false, nullptr);
       SampleArgs sa{};
