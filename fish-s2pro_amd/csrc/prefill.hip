@@ -1022,8 +1022,8 @@ __global__ __launch_bounds__(SK_WAVES * 64) void skinny_mfma_kernel(SkinnyArgs a
 // Causal GQA attention for a prompt chunk on the MFMA units: query c
 // (0 <= c < N) sits at position base + c and attends cache positions
 // 0 .. base + c (its own K/V already appended).
-//   Block (32 queries, kv head g, key split sp), wave w = q head g * rep + w;
-//   the waves share each 32-key K/V tile in LDS.  Per tile a wave computes
+//   Block (32 QG queries, kv head g, key split sp), wave w = q head g * rep + w
+//   % 4 and queries 32 (w / 4) ..; the waves share each 32-key K/V tile in LDS.  Per tile a wave computes
 //   the scores transposed, S^T = K Q^T (v_mfma_f32_32x32x16_f16, K as A from
 //   LDS, the wave's Q as B in registers), so a lane owns one query and 16 of
 //   the tile's keys: the online softmax (running max and sum per query, f32)
@@ -1054,26 +1054,37 @@ __device__ __forceinline__ void split_h(float x, _Float16& h, _Float16& l) {
 // position of key j (0..31) of a tile in the transposed V layout: bits 2 and 3 swapped
 __device__ __forceinline__ uint32_t vt_pos(uint32_t j) { return (j & ~12u) | ((j & 4u) << 1) | ((j & 8u) >> 1); }
 
-template <int HD, bool KH>
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillAttnArgs a, uint32_t splits) {
+// exp(x) for x <= 0: exp2 of the rounded product x log2(e), corrected by the
+// product's remainder (two fused multiply-adds), so the hardware exp2's
+// accuracy is that of the result; half the operations of expf.
+__device__ __forceinline__ float exp_neg(float x) {
+  const float t = x * 1.44269502f;
+  const float lo = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -t));
+  const float e = __builtin_amdgcn_exp2f(t);
+  return fmaf(e, lo * 0.693147181f, e);
+}
+
+template <int HD, bool KH, int QG>
+__global__ __launch_bounds__(256 * QG, 2) void attn_prefill_kernel(PrefillAttnArgs a, uint32_t splits) {
   using KT = std::conditional_t<KH, uint16_t, float>;  // cache element: f16 bits or f32
   constexpr int DS = HD / 16;          // 16-wide k steps of the scores
   constexpr int DT = HD / 32;          // 32-wide output tiles
   constexpr int KP = HD + 8;           // padded K row (halfs)
   constexpr int VP = AT + 8;           // padded V^T row (halfs)
-  constexpr int KF4 = AT * HD / 4 / 256;   // K float4 per thread per tile
-  constexpr int VG = HD * (AT / 4) / 256;  // V (dim, 4-key group) pairs per thread per tile
+  constexpr uint32_t NT = 256 * QG;       // threads
+  constexpr int KF4 = AT * HD / 4 / NT;   // K float4 per thread per tile
+  constexpr int VG = HD * (AT / 4) / NT;  // V (dim, 4-key group) pairs per thread per tile
   __shared__ _Float16 ks[2][AT][KP];   // hi, lo planes
   __shared__ _Float16 vts[2][HD][VP];
   __shared__ uint32_t bad;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t q0 = blockIdx.x * AQ, g = blockIdx.y, sp = blockIdx.z;
-  const uint32_t rep = a.H / a.Hkv;
-  const bool active = wave < rep;
-  const uint32_t h = g * rep + (active ? wave : 0u);
+  const uint32_t qb = blockIdx.x * (AQ * QG), g = blockIdx.y, sp = blockIdx.z;
+  const uint32_t rep = a.H / a.Hkv, q0 = qb + AQ * (wave / 4u);  // this wave's first query
+  const bool active = (wave & 3u) < rep && q0 < a.N;
+  const uint32_t h = g * rep + ((wave & 3u) < rep ? wave & 3u : 0u);
   const uint32_t base = *a.pos_ptr + a.pos_offset;
-  const uint32_t nq = min(uint32_t(AQ), a.N - q0);
-  const uint32_t t_end = base + q0 + nq;  // keys needed by the last query
+  const uint32_t nq = q0 < a.N ? min(uint32_t(AQ), a.N - q0) : 0u;
+  const uint32_t t_end = base + min(qb + AQ * QG, a.N);  // keys needed by the block's last query
   // this block's run of whole tiles
   const uint32_t n_tiles = (t_end + AT - 1) / AT, per = (n_tiles + splits - 1) / splits;
   const uint32_t tile_lo = min(sp * per, n_tiles), tile_hi = min(tile_lo + per, n_tiles);
@@ -1084,7 +1095,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillAttnArgs a,
   // the wave's queries as the B operand of S^T: query q0 + fr, dims 16 ds + fk .. + 7
   half8 qh[DS], ql[DS];
   {
-    const uint32_t qi = q0 + min(fr, nq - 1u);
+    const uint32_t qi = min(q0 + fr, a.N - 1u);
     const float* qrow = a.q + size_t(qi) * a.H * HD + size_t(h) * HD + fk;
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) {
@@ -1111,7 +1122,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillAttnArgs a,
   auto load_tile = [&](uint32_t t0) {
 #pragma unroll
     for (int j = 0; j < KF4; ++j) {
-      const uint32_t f = tid + 256u * j, key = f / (HD / 4), d = (f % (HD / 4)) * 4u;
+      const uint32_t f = tid + NT * j, key = f / (HD / 4), d = (f % (HD / 4)) * 4u;
       const uint32_t t = min(t0 + key, a.max_seq - 1u);
       if constexpr (KH) {
         const uint2 r = *reinterpret_cast<const uint2*>(kc + size_t(t) * HD + d);
@@ -1127,7 +1138,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillAttnArgs a,
     }
 #pragma unroll
     for (int j = 0; j < VG; ++j) {
-      const uint32_t p = tid + 256u * j, d = p % HD, k0 = 4u * (p / HD);
+      const uint32_t p = tid + NT * j, d = p % HD, k0 = 4u * (p / HD);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const uint32_t t = t0 + k0 + i;
@@ -1141,7 +1152,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillAttnArgs a,
   auto store_tile = [&]() {
 #pragma unroll
     for (int j = 0; j < KF4; ++j) {
-      const uint32_t f = tid + 256u * j, key = f / (HD / 4), d = (f % (HD / 4)) * 4u;
+      const uint32_t f = tid + NT * j, key = f / (HD / 4), d = (f % (HD / 4)) * 4u;
       const float x[4] = {kr[j].x, kr[j].y, kr[j].z, kr[j].w};
       _Float16 hh[4], ll[4];
 #pragma unroll
@@ -1154,7 +1165,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillAttnArgs a,
     }
 #pragma unroll
     for (int j = 0; j < VG; ++j) {
-      const uint32_t p = tid + 256u * j, d = p % HD, k0 = 4u * (p / HD);
+      const uint32_t p = tid + NT * j, d = p % HD, k0 = 4u * (p / HD);
       _Float16 hh[4], ll[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1180,7 +1191,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillAttnArgs a,
     store_tile();
     __syncthreads();
     if (tile + 1 < tile_hi) load_tile(t0 + AT);  // in flight during this tile
-    if (!active) continue;
+    if (!active || t0 > base + q0 + nq - 1u) continue;  // (a tile past this wave's queries)
     // S^T[key][query]: lane holds query fr, keys 8 (v / 4) + 4 (lane / 32) + v % 4
     floatx16 sacc = floatx16{};
 #pragma unroll
@@ -1202,11 +1213,11 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillAttnArgs a,
     }
     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
     const float mn = fmaxf(m, mt);
-    const float corr = (m == -INFINITY) ? 0.0f : expf(m - mn);
+    const float corr = (m == -INFINITY) ? 0.0f : exp_neg(m - mn);
     float ps = 0.0f;
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      s[v] = (s[v] == -INFINITY) ? 0.0f : expf(s[v] - mn);
+      s[v] = (s[v] == -INFINITY) ? 0.0f : exp_neg(s[v] - mn);
       ps += s[v];
     }
     ps += __shfl_xor(ps, 32, 64);
@@ -1548,11 +1559,22 @@ size_t attn_prefill_part_floats(uint32_t n, uint32_t heads, uint32_t hd) {
   return size_t(ATTN_MAX_SPLITS) * n * heads * (hd + 4);
 }
 
+// Two query groups per block (8 waves sharing each K / V tile, which halves the
+// tile's conversion and staging per wave) past 256 queries: 1500 tokens 191 ->
+// 147 us, 389 30.3 -> 24.9; 256 tokens leave too few blocks for it (19.7 and
+// 20.3 us, the first layers 14.5 and 19.2).
+static bool attn_wide(uint32_t n) { return n > 256u; }
 template <int HD>
 static void attn_prefill_launch(const PrefillAttnArgs& a, uint32_t splits, hipStream_t s) {
-  const dim3 grid((a.N + AQ - 1) / AQ, a.Hkv, splits);
-  hipLaunchKernelGGL((a.kv_f16 ? attn_prefill_kernel<HD, true> : attn_prefill_kernel<HD, false>), grid, dim3(256), 0,
-                     s, a, splits);
+  if (attn_wide(a.N)) {
+    const dim3 grid((a.N + 2 * AQ - 1) / (2 * AQ), a.Hkv, splits);
+    hipLaunchKernelGGL((a.kv_f16 ? attn_prefill_kernel<HD, true, 2> : attn_prefill_kernel<HD, false, 2>), grid, dim3(512),
+                       0, s, a, splits);
+  } else {
+    const dim3 grid((a.N + AQ - 1) / AQ, a.Hkv, splits);
+    hipLaunchKernelGGL((a.kv_f16 ? attn_prefill_kernel<HD, true, 1> : attn_prefill_kernel<HD, false, 1>), grid, dim3(256),
+                       0, s, a, splits);
+  }
   if (splits > 1)
     hipLaunchKernelGGL((attn_prefill_merge_kernel<HD>), dim3((a.N * a.H * (HD / 4) + 255) / 256), dim3(256), 0, s, a,
                        splits);
@@ -1561,7 +1583,7 @@ static void attn_prefill_launch(const PrefillAttnArgs& a, uint32_t splits, hipSt
 hipError_t launch_attention_prefill(const PrefillAttnArgs& a, hipStream_t s) {
   if (!a.pos_ptr || a.H % a.Hkv || a.H / a.Hkv > 4 || a.N == 0) return hipErrorInvalidValue;
   // key splits so that the grid covers the CUs twice over (two blocks fit a CU)
-  const uint32_t blocks = (a.N + AQ - 1) / AQ * a.Hkv;
+  const uint32_t qpb = attn_wide(a.N) ? 2 * AQ : AQ, blocks = (a.N + qpb - 1) / qpb * a.Hkv;
   uint32_t splits = 1;
   while (splits < ATTN_MAX_SPLITS && blocks * splits < 512u &&
          size_t(splits + 1) * a.N * a.H * (a.hd + 4) <= a.part_cap && a.part)

@@ -24,7 +24,7 @@ def _rel(a, b):
 
 
 @pytest.mark.parametrize("weights", sorted(TYPES))
-@pytest.mark.parametrize("ffn,lengths", [(1536, (1, 2, 3, 4, 5, 17, 63, 65, 129, 257, 770, 2100)), (1504, (5, 33, 300))])
+@pytest.mark.parametrize("ffn,lengths", [(1536, (1, 2, 3, 4, 5, 17, 63, 65, 129, 257, 289, 321, 770, 2100)), (1504, (5, 33, 300))])
 def test_prefill_lengths_match_oracle(model_dir, weights, ffn, lengths):
     from s2hip import Engine
 
