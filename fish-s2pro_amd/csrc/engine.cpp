@@ -115,6 +115,16 @@ struct FastLayer {
   DevLin wqkv, wo, w1, w2, w3;
 };
 
+// Sets a flag for the lifetime of the scope.
+struct FlagScope {
+  bool& flag;
+  const bool was;
+  explicit FlagScope(bool& f) : flag(f), was(f) { flag = true; }
+  ~FlagScope() { flag = was; }
+  FlagScope(const FlagScope&) = delete;
+  FlagScope& operator=(const FlagScope&) = delete;
+};
+
 std::string lname(const char* pre, uint32_t l, const char* suf) {
   return std::string(pre) + "." + std::to_string(l) + "." + suf;
 }
@@ -252,9 +262,10 @@ class Engine {
   bool tiled_ = false, repacked_ = false;
   uint32_t* lin_err_ = nullptr;  // error word of the linears (null: slot 0's)
   uint32_t bmm_min_cols_ = 2;  // columns from which F16 linears use the batched product
-  // Set while a call is re-run after ERR_F16_RANGE: every multi-column linear
-  // then takes the per-column paths (two-column GEMV, or the skinny product
-  // over rows split with a whole-row scale), which have no per-wave range.
+  // Set while a call is re-run after ERR_F16_RANGE, and during calls of one or
+  // two columns: every multi-column linear then takes the per-column paths
+  // (two-column GEMV, or the skinny product over rows split with a whole-row
+  // scale), which have no per-wave range.
   bool bmm_off_ = false;
   bool any_f16_range(uint32_t nseq) const { return any_err(nseq, ERR_F16_RANGE); }
   bool any_err(uint32_t nseq, uint32_t bits) const {
@@ -1492,13 +1503,17 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
 // the device: a prefix of three codes is two passes over the weights where four
 // passes, and a copy to the host and a wait per code, took 0.84 ms.  Four columns
 // a pass on the batched product took 0.30 ms but were further off 64-bit sums
-// (1.0e-6 against 6.7e-7).
+// (1.0e-6 against 6.7e-7).  Every linear takes the f32 GEMVs whatever its width: the
+// batched product's range is a matter of the activations, and its copies are there
+// only once a longer call has built them.
 void Engine::fast_logits(const float* hidden, const uint32_t* prefix, size_t plen, float* logits) {
   select();
   const s2hip_spec& s = spec;
   if (plen >= s.num_codebooks) fail("fast prefix too long: " + std::to_string(plen) + " codes");
   for (size_t j = 0; j < plen; ++j)
     if (prefix[j] >= s.codebook_size) fail("fast prefix code out of range");
+  ensure_repacked();
+  const FlagScope gemvs(bmm_off_);
   const size_t n = plen + 1;
   uint32_t cols = 0;
   for (size_t p0 = 0; p0 < n; p0 += cols) {

@@ -1,0 +1,71 @@
+"""fast_logits at widths without a two-column GEMV (multiples of 256 other than
+512, 1536, 2560, 4096 and 9728), against the oracle and against itself: what the
+call returns is decided by its inputs, not by which copies of the weights earlier
+calls have built."""
+
+import shutil
+
+import numpy as np
+import pytest
+
+import gguf_util
+from conftest import make_prompt
+from oracle import oracle as O
+from s2hip import synth
+
+pytestmark = pytest.mark.gpu
+
+SHAPE = synth.TINY.with_(name="w1024", slow_layers=2, dim=1024, ffn=2048, heads=16, kv_heads=4, fast_ffn=2048,
+                         fast_heads=16, fast_kv_heads=4, vocab=2304, semantic_begin=1024, semantic_end=2047,
+                         im_end_id=1000)
+TYPES = {"f16": synth.GGML_F16, "q8_0": synth.GGML_Q8_0, "q4_0": synth.GGML_Q4_0}
+PREFIXES = (0, 1, 2, 3, 8, 9)
+
+
+def _rel(a, b):
+    return float(np.max(np.abs(a - b)) / max(1e-30, float(np.max(np.abs(b)))))
+
+
+def _inputs(seed):
+    rng = np.random.default_rng(seed)
+    return rng.standard_normal(SHAPE.dim).astype(np.float32), rng.integers(0, SHAPE.codebook_size, 9).astype(np.uint32)
+
+
+def _outlier_gguf(model_dir, tmp_path, prefix, layers):
+    path = str(tmp_path / "outlier.gguf")
+    shutil.copyfile(synth.ensure_gguf(SHAPE, model_dir), path)
+    for l in range(layers):
+        for w in ("w1", "w3"):
+            gguf_util.scale_rows(path, f"{prefix}.{l}.feed_forward.{w}.weight", [300], 1000.0)
+    return path
+
+
+def test_fast_logits_with_an_outlier_channel_after_a_generation(model_dir, tmp_path):
+    """Channel 300 of the Fast-AR FFN lies past the headroom of the batched
+    product, whose copies the generation before has built."""
+    from s2hip import Engine
+
+    path = _outlier_gguf(model_dir, tmp_path, "fast_layers", SHAPE.fast_layers)
+    o = O.OracleModel(path, 64, SHAPE.im_end_id)
+    hidden, codes = _inputs(1)
+    with Engine(path, 64, SHAPE.im_end_id) as e:
+        e.generate_codes(make_prompt(SHAPE, 7, seed=1), 2, min_tokens_before_end=100)
+        for n in PREFIXES:
+            got, want = e.fast_logits(hidden, codes[:n]), o.fast_logits(hidden, codes[:n])
+            assert np.all(np.isfinite(got)) and _rel(got, want) < 1e-4, n
+
+
+@pytest.mark.parametrize("weights", sorted(TYPES))
+def test_fast_logits_do_not_depend_on_earlier_calls(model_dir, weights):
+    from s2hip import Engine
+
+    path = synth.ensure_gguf(SHAPE.with_(linear_type=TYPES[weights]), model_dir)
+    o = O.OracleModel(path, 64, SHAPE.im_end_id)
+    hidden, codes = _inputs(2)
+    with Engine(path, 64, SHAPE.im_end_id) as e:
+        cold = [e.fast_logits(hidden, codes[:n]) for n in PREFIXES]
+        e.eval(make_prompt(SHAPE, 5, seed=2))
+        e.generate_codes(make_prompt(SHAPE, 7, seed=3), 2, min_tokens_before_end=100)
+        for n, want in zip(PREFIXES, cold):
+            assert np.array_equal(e.fast_logits(hidden, codes[:n]), want), n
+            assert _rel(want, o.fast_logits(hidden, codes[:n])) < 1e-4, n
