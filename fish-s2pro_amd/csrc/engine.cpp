@@ -115,11 +115,11 @@ struct FastLayer {
   DevLin wqkv, wo, w1, w2, w3;
 };
 
-// Sets a flag for the lifetime of the scope.
+// Sets a flag for the lifetime of the scope (if `on`).
 struct FlagScope {
   bool& flag;
   const bool was;
-  explicit FlagScope(bool& f) : flag(f), was(f) { flag = true; }
+  explicit FlagScope(bool& f, bool on = true) : flag(f), was(f) { flag = was || on; }
   ~FlagScope() { flag = was; }
   FlagScope(const FlagScope&) = delete;
   FlagScope& operator=(const FlagScope&) = delete;
@@ -1456,11 +1456,14 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
   validate_tokens(flat, n_tok);
   ensure_slots(slot + 1);
   // a few tokens: the decode kernels (a product's 64-token tile would stand
-  // nearly empty).  Beyond the batched product's range (three and four
-  // tokens), the call runs again on the prefill products.
+  // nearly empty), one and two on the GEMVs, three and four on the batched
+  // product.  Beyond its range the call runs again on the prefill products.  The
+  // copies that a length can use are built first and the others not used, so that
+  // its bits do not depend on earlier calls.
   bool few = n_tok <= PREFILL_COLS;
-  if (few && n_tok <= 2) ensure_repacked();
-  else ensure_tiled();
+  const bool gemvs = n_tok <= 2;
+  if (few) ensure_repacked();
+  if (!gemvs) ensure_tiled();
   ensure_prompt(n_tok * cdim);
   HIPC(hipMemcpyAsync(prompt_dev_, flat, n_tok * cdim * 4, hipMemcpyHostToDevice, stream_));
   uint32_t e = 0;
@@ -1469,6 +1472,7 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
     HIPC(hipMemsetAsync(&st_[slot].done, 0, sizeof(uint32_t), stream_));
     HIPC(hipMemsetAsync(&st_[slot].err, 0, sizeof(uint32_t), stream_));
     if (few || prefill_gemv_) {
+      const FlagScope off(bmm_off_, gemvs);
       lin_err_ = &st_[slot].err;
       enqueue_prefill_gemv(prompt_dev_, n_tok, slot);
       lin_err_ = nullptr;

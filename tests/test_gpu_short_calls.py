@@ -1,7 +1,7 @@
-"""fast_logits at widths without a two-column GEMV (multiples of 256 other than
-512, 1536, 2560, 4096 and 9728), against the oracle and against itself: what the
-call returns is decided by its inputs, not by which copies of the weights earlier
-calls have built."""
+"""fast_logits and eval of one to four tokens at widths without a two-column
+GEMV (multiples of 256 other than 512, 1536, 2560, 4096 and 9728), against the
+oracle and against themselves: what such a call returns is decided by its inputs,
+not by which copies of the weights earlier calls have built."""
 
 import shutil
 
@@ -69,3 +69,20 @@ def test_fast_logits_do_not_depend_on_earlier_calls(model_dir, weights):
         for n, want in zip(PREFIXES, cold):
             assert np.array_equal(e.fast_logits(hidden, codes[:n]), want), n
             assert _rel(want, o.fast_logits(hidden, codes[:n])) < 1e-4, n
+
+
+@pytest.mark.parametrize("weights", sorted(TYPES))
+def test_short_evals_do_not_depend_on_earlier_calls(model_dir, weights):
+    from s2hip import Engine
+
+    path = synth.ensure_gguf(SHAPE.with_(linear_type=TYPES[weights]), model_dir)
+    with Engine(path, 64, SHAPE.im_end_id) as warm:
+        warm.eval(make_prompt(SHAPE, 5, seed=2))
+        warm.generate_codes(make_prompt(SHAPE, 7, seed=3), 2, min_tokens_before_end=100)
+        for n in (1, 2, 3, 4):
+            prompt = make_prompt(SHAPE, n, seed=n)
+            with Engine(path, 64, SHAPE.im_end_id) as cold:
+                want = cold.eval(prompt)
+            warm.reset()
+            got = warm.eval(prompt)
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), n
