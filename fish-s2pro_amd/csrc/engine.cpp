@@ -216,6 +216,7 @@ class Engine {
   uint8_t* try_dalloc(size_t bytes);
   void bmm(const DevLin& L, const DevLin* L3, int epi, uint32_t ncol, const float* x, uint32_t ldx, const float* norm,
            float eps, float* y, uint32_t ldy, const uint32_t* done, uint32_t* err, uint32_t waves = 0);
+  bool decode_takes_shape() const;
   void validate_prompt(const int32_t* prompt, size_t cols);
   void validate_tokens(const int32_t* flat, size_t n_tok);
   void mm(const DevLin& L, const DevLin* L3, int epi, const float* x, uint32_t ldx, const float* norm, float eps,
@@ -672,7 +673,7 @@ void Engine::gemv(const DevLin& L, const DevLin* L3, int epi, uint32_t ncol, con
   uint32_t c = 0;
   while (c < ncol) {
     uint32_t w = 8;
-    while (w > 1 && (w > ncol - c || size_t(w) * L.in * 4 > 150 * 1024)) w >>= 1;
+    while (w > 1 && (w > ncol - c || size_t(w) * L.in > GEMV_MAX_IN)) w >>= 1;
     GemvArgs a{};
     a.w = L.w;
     a.w3 = L3 ? L3->w : nullptr;
@@ -1444,6 +1445,15 @@ void Engine::validate_tokens(const int32_t* flat, size_t n_tok) {
   }
 }
 
+// Whether launch_gemv and launch_attention take the Slow-AR shape: a GEMV stages
+// its input row in LDS, and the attention packs the head count into a byte and the
+// slot's cache size into a word.
+bool Engine::decode_takes_shape() const {
+  const s2hip_spec& s = spec;
+  return std::max({s.dim, s.heads * s.head_dim, s.ffn}) <= GEMV_MAX_IN && s.heads <= ATTN_MAX_HEADS &&
+         slot_kv_ <= UINT32_MAX;
+}
+
 void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* logits_out, uint32_t slot) {
   select();
   const s2hip_spec& s = spec;
@@ -1459,11 +1469,12 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
   // nearly empty), one and two on the GEMVs, three and four on the batched
   // product.  Beyond its range the call runs again on the prefill products.  The
   // copies that a length can use are built first and the others not used, so that
-  // its bits do not depend on earlier calls.
-  bool few = n_tok <= PREFILL_COLS;
+  // its bits do not depend on earlier calls.  (A shape that the decode kernels
+  // refuse has the prefill products at every length.)
+  bool few = n_tok <= PREFILL_COLS && decode_takes_shape();
   const bool gemvs = n_tok <= 2;
   if (few) ensure_repacked();
-  if (!gemvs) ensure_tiled();
+  if (!few || !gemvs) ensure_tiled();
   ensure_prompt(n_tok * cdim);
   HIPC(hipMemcpyAsync(prompt_dev_, flat, n_tok * cdim * 4, hipMemcpyHostToDevice, stream_));
   uint32_t e = 0;

@@ -118,7 +118,9 @@ struct SamplerCfg {
   int32_t top_k;
 };
 
-// GEMV over `ncol` input columns (1, 2, 4 or 8).
+// GEMV over `ncol` input columns (1, 2, 4 or 8), ncol * in <= GEMV_MAX_IN (the
+// columns are staged in LDS: 150 of a CU's 160 KiB).
+constexpr uint32_t GEMV_MAX_IN = 38400;
 hipError_t launch_gemv(uint32_t wtype, int epi, int ncol, const GemvArgs& a, hipStream_t s);
 
 // Per-column RMSNorm: y[c] = (x[c] * scale_c) * w.
@@ -202,6 +204,7 @@ struct AttnArgs {
 enum : uint32_t { ATTN_SPLIT = 0u, ATTN_FUSED = 1u };
 constexpr uint32_t ATTN_CHUNK = 32;         // cache positions per decode attention block
 constexpr uint32_t ATTN_MAX_CHUNKS = 1024;  // max_seq <= 32768
+constexpr uint32_t ATTN_MAX_HEADS = 255;    // one byte of the shape word
 uint32_t attention_chunks(uint32_t max_seq, uint32_t mode);
 hipError_t launch_attention(const AttnArgs& a, hipStream_t s);
 

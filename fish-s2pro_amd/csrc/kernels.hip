@@ -3235,7 +3235,7 @@ hipError_t launch_gemv(uint32_t wtype, int epi, int ncol, const GemvArgs& a, hip
       default: return gemv_direct_epi<W_Q4_0>(epi, ncol, a, s);
     }
   }
-  if (size_t(ncol) * a.in * sizeof(float) > 150 * 1024) return hipErrorInvalidValue;
+  if (size_t(ncol) * a.in > GEMV_MAX_IN) return hipErrorInvalidValue;
   switch (wtype) {
     case W_F16: return gemv_pick_epi<W_F16>(epi, ncol, a, s);
     case W_Q8_0: return gemv_pick_epi<W_Q8_0>(epi, ncol, a, s);
@@ -3309,7 +3309,7 @@ hipError_t launch_attention(const AttnArgs& args, hipStream_t s) {
   if (a.cols_per_seq == 0) a.cols_per_seq = a.ncol;  // one sequence
   if (a.ncol == 0 || a.ncol % a.cols_per_seq || a.cols_per_seq > 4 || a.ncol > 64) return hipErrorInvalidValue;
   if (a.ncol > a.cols_per_seq && a.seq_stride_words == 0 && (a.pos_ptr || a.done)) return hipErrorInvalidValue;
-  if (a.H % a.Hkv || a.H / a.Hkv > 4 || a.H > 255 || a.seq_stride_words > 255 || a.seq_stride_kv > UINT32_MAX)
+  if (a.H % a.Hkv || a.H / a.Hkv > 4 || a.H > ATTN_MAX_HEADS || a.seq_stride_words > 255 || a.seq_stride_kv > UINT32_MAX)
     return hipErrorInvalidValue;
   if (a.max_chunks != attention_chunks(a.max_seq, a.mode) || a.check_from > a.max_chunks) return hipErrorInvalidValue;
   if (a.qkv_rows) {

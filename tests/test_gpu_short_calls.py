@@ -86,3 +86,25 @@ def test_short_evals_do_not_depend_on_earlier_calls(model_dir, weights):
             warm.reset()
             got = warm.eval(prompt)
             assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), n
+
+
+# an input row wider than the decode GEMV stages in LDS (38400 floats), and more
+# heads than the decode attention takes (255)
+WIDE = {"ffn": dict(ffn=40960), "heads": dict(heads=256, kv_heads=64)}
+
+
+@pytest.mark.parametrize("what", sorted(WIDE))
+def test_short_evals_of_shapes_past_the_decode_kernels(model_dir, what):
+    """Such a model's prompts of any length go through the prompt products."""
+    from s2hip import Engine
+
+    shape = synth.TINY.with_(name="wide_" + what, slow_layers=1, fast_layers=1, vocab=2304, semantic_begin=1024,
+                             semantic_end=2047, im_end_id=1000, **WIDE[what])
+    path = synth.ensure_gguf(shape, model_dir)
+    o = O.OracleModel(path, 64, shape.im_end_id)
+    with Engine(path, 64, shape.im_end_id) as e:
+        for n in (5, 1, 2, 3, 4):
+            prompt = make_prompt(shape, n, seed=n)
+            (hg, lg), (ho, lo) = e.eval(prompt), o.eval(prompt)
+            assert _rel(hg, ho) < 1e-4 and _rel(lg, lo) < 1e-4, n
+        assert e.n_past == 15
