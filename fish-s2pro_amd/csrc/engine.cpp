@@ -1467,7 +1467,9 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
   ensure_slots(slot + 1);
   // a few tokens: the decode kernels (a product's 64-token tile would stand
   // nearly empty), one and two on the GEMVs, three and four on the batched
-  // product.  Beyond its range the call runs again on the prefill products.  The
+  // product.  Beyond its range, or where the result is not finite (which the
+  // prefill attention tells apart: an error if a layer has read such a value,
+  // else the result as it is), the call runs again on the prefill products.  The
   // copies that a length can use are built first and the others not used, so that
   // its bits do not depend on earlier calls.  (A shape that the decode kernels
   // refuse has the prefill products at every length.)
@@ -1497,11 +1499,9 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
     HIPC(hipStreamSynchronize(stream_));
     e = st_host_[slot].err;
     if (!few) break;
-    if (!(e & ERR_F16_RANGE)) {
-      for (uint32_t i = 0; i < s.dim; ++i)
-        if (!std::isfinite(hidden_out[i])) e |= ERR_F16_RANGE;
-      break;
-    }
+    bool finite = true;
+    for (uint32_t i = 0; i < s.dim && finite; ++i) finite = std::isfinite(hidden_out[i]);
+    if (finite && !(e & ERR_F16_RANGE)) break;
     few = false;
     ensure_tiled();
     HIPC(hipMemcpyAsync(&st_[slot].n_past, &n_past_host[slot], sizeof(uint32_t), hipMemcpyHostToDevice, stream_));

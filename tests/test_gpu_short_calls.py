@@ -108,3 +108,22 @@ def test_short_evals_of_shapes_past_the_decode_kernels(model_dir, what):
             (hg, lg), (ho, lo) = e.eval(prompt), o.eval(prompt)
             assert _rel(hg, ho) < 1e-4 and _rel(lg, lo) < 1e-4, n
         assert e.n_past == 15
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5])
+def test_non_finite_activations_are_answered_alike_at_every_length(model_dir, tmp_path, n):
+    """A NaN that the last layer's FFN makes reaches nothing but the outputs, which
+    are returned; one that a later layer's attention reads is an error."""
+    from s2hip import Engine, S2HipError
+
+    for layer in (SHAPE.slow_layers - 1, 0):
+        path = str(tmp_path / f"nan{layer}.gguf")
+        shutil.copyfile(synth.ensure_gguf(SHAPE, model_dir), path)
+        gguf_util.scale_rows(path, f"layers.{layer}.feed_forward.w2.weight", [17], np.inf)
+        with Engine(path, 64, SHAPE.im_end_id) as e:
+            if layer:
+                hidden, _ = e.eval(make_prompt(SHAPE, n, seed=n))
+                assert not np.all(np.isfinite(hidden)) and e.n_past == n
+            else:
+                with pytest.raises(S2HipError, match="not finite"):
+                    e.eval(make_prompt(SHAPE, n, seed=n))
