@@ -189,10 +189,11 @@ class Engine {
             const float* norm, float eps, float* y, uint32_t ldy, uint32_t row_base, uint32_t extra_row, uint32_t out_rows,
             const uint32_t* done, const GreedyFold* fold = nullptr);
   // linear over ncol columns: GEMV kernels for 1-2, skinny MFMA for more
-  // (bmm_waves: waves per tile when the batched product serves it, 0 = its default)
+  // (err: word for ERR_F16_RANGE; bmm_waves: waves per tile when the batched product serves it, 0 = its default)
   void lin(const DevLin& L, const DevLin* L3, int epi, uint32_t ncol, const float* x, uint32_t ldx,
            const float* norm, float eps, float* y, uint32_t ldy, uint32_t row_base, uint32_t extra_row,
-           uint32_t out_rows, const uint32_t* done, uint32_t bmm_waves = 0, const GreedyFold* fold = nullptr);
+           uint32_t out_rows, const uint32_t* done, uint32_t* err, uint32_t bmm_waves = 0,
+           const GreedyFold* fold = nullptr);
   // ncol = nseq * cps columns of slots seq0 .. seq0 + nseq - 1 in h_
   // advance: add cps to each unfinished slot's n_past afterwards (the frame
   // loop leaves it to its sampler instead)
@@ -225,7 +226,7 @@ class Engine {
   // batched columns (3..16): split planes + skinny MFMA product
   void mm_skinny(const DevLin& L, const DevLin* L3, int epi, const float* x, uint32_t ldx, const float* norm,
                  float eps, uint32_t n, float* y, uint32_t ldy, uint32_t row_base, uint32_t extra_row,
-                 uint32_t out_rows, const uint32_t* done);
+                 uint32_t out_rows, const uint32_t* done, uint32_t* err);
   bool uses_bmm(const DevLin& L, const DevLin* L3, uint32_t ncol) const;
   L2Warm warm_for(const DevLin& L, const DevLin* L3, uint32_t ncol, bool norm, uint32_t pct_begin,
                   uint32_t pct_end) const;
@@ -261,7 +262,6 @@ class Engine {
   DevLin head_full_, fast_out_;
   DevLin head_cand_;  // the candidate rows of the head (tiled copy only)
   bool tiled_ = false, repacked_ = false;
-  uint32_t* lin_err_ = nullptr;  // error word of the linears (null: slot 0's)
   uint32_t bmm_min_cols_ = 2;  // columns from which F16 linears use the batched product
   // Set while a call is re-run after ERR_F16_RANGE, and during calls of one or
   // two columns: every multi-column linear then takes the per-column paths
@@ -739,13 +739,13 @@ bool Engine::uses_bmm(const DevLin& L, const DevLin* L3, uint32_t ncol) const {
 
 void Engine::lin(const DevLin& L, const DevLin* L3, int epi, uint32_t ncol, const float* x, uint32_t ldx,
                  const float* norm, float eps, float* y, uint32_t ldy, uint32_t row_base, uint32_t extra_row,
-                 uint32_t out_rows, const uint32_t* done, uint32_t bmm_waves, const GreedyFold* fold) {
+                 uint32_t out_rows, const uint32_t* done, uint32_t* err, uint32_t bmm_waves, const GreedyFold* fold) {
   if (fold) {  // one column (checked by gemv), never on the batched product
     gemv(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, row_base, extra_row, out_rows, done, fold);
     return;
   }
   if (uses_bmm(L, L3, ncol)) {
-    bmm(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, done, lin_err_ ? lin_err_ : &st_->err, bmm_waves);
+    bmm(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, done, err, bmm_waves);
     return;
   }
   if (ncol <= 2 || L.in % 256) {
@@ -755,7 +755,7 @@ void Engine::lin(const DevLin& L, const DevLin* L3, int epi, uint32_t ncol, cons
   for (uint32_t c = 0; c < ncol; c += 16) {
     const uint32_t n = std::min(16u, ncol - c);
     mm_skinny(L, L3, epi, x + size_t(c) * ldx, ldx, norm, eps, n, y + size_t(c) * ldy, ldy, row_base, extra_row,
-              out_rows, done);
+              out_rows, done, err);
   }
 }
 
@@ -833,7 +833,8 @@ void Engine::enqueue_slow_layers(uint32_t nseq, uint32_t cps, uint32_t seq0, con
   for (uint32_t l = 0; l < s.slow_layers; ++l) {
     const SlowLayer& L = slow_[l];
     prof_mark(PROF_NONE);
-    lin(L.wqkv, nullptr, EPI_STORE, ncol, h_, s.dim, L.attn_norm, s.eps, qkv_, qkv_w, 0, NO_ROW, L.wqkv.out, done);
+    lin(L.wqkv, nullptr, EPI_STORE, ncol, h_, s.dim, L.attn_norm, s.eps, qkv_, qkv_w, 0, NO_ROW, L.wqkv.out,
+        done, &st->err);
     prof_mark(PROF_LINEAR);
     AttnArgs aa{};
     aa.qkv = qkv_;
@@ -869,9 +870,10 @@ void Engine::enqueue_slow_layers(uint32_t nseq, uint32_t cps, uint32_t seq0, con
     aa.warm = warm_for(L.wo, nullptr, ncol, false, 0, warm_slow_);
     HIPC(launch_attention(aa, stream_));
     prof_mark(PROF_ATTN);
-    lin(L.wo, nullptr, EPI_RESID, ncol, att_, q, nullptr, 0.0f, h_, s.dim, 0, NO_ROW, L.wo.out, done);
-    lin(L.w1, &L.w3, EPI_SWIGLU_SLOW, ncol, h_, s.dim, L.ffn_norm, s.eps, act_, s.ffn, 0, NO_ROW, L.w1.out, done);
-    lin(L.w2, nullptr, EPI_RESID, ncol, act_, s.ffn, nullptr, 0.0f, h_, s.dim, 0, NO_ROW, L.w2.out, done);
+    lin(L.wo, nullptr, EPI_RESID, ncol, att_, q, nullptr, 0.0f, h_, s.dim, 0, NO_ROW, L.wo.out, done, &st->err);
+    lin(L.w1, &L.w3, EPI_SWIGLU_SLOW, ncol, h_, s.dim, L.ffn_norm, s.eps, act_, s.ffn, 0, NO_ROW, L.w1.out,
+        done, &st->err);
+    lin(L.w2, nullptr, EPI_RESID, ncol, act_, s.ffn, nullptr, 0.0f, h_, s.dim, 0, NO_ROW, L.w2.out, done, &st->err);
     prof_mark(PROF_LINEAR);
   }
   if (advance) HIPC(launch_add_position(st, cps, nseq, stream_));
@@ -888,12 +890,12 @@ void Engine::enqueue_head(uint32_t ncol, float* hn, float* logits, bool full, co
     // normalised row to hn, which the Fast-AR and the full head read)
     gemv_xn_ = hn;
     lin(head_cand_, nullptr, EPI_STORE, 1, h_, s.dim, norm_, s.eps, logits, n_cand_, s.semantic_begin, head_extra_,
-        n_cand_, done);
+        n_cand_, done, &st_->err);
     gemv_xn_ = nullptr;
   } else {
     HIPC(launch_rms_norm(h_, norm_, hn, s.dim, ncol, s.eps, done, stream_));
     lin(head_cand_, nullptr, EPI_STORE, ncol, hn, s.dim, nullptr, 0.0f, logits, n_cand_, s.semantic_begin,
-        head_extra_, n_cand_, done);
+        head_extra_, n_cand_, done, &st_->err);
   }
   if (full)
     gemv(head_full_, nullptr, EPI_STORE, 1, hn, s.dim, nullptr, 0.0f, logits_full_, s.vocab, 0, NO_ROW, s.vocab, done);
@@ -914,7 +916,7 @@ void Engine::enqueue_fast_layers(uint32_t nseq, uint32_t cps, uint32_t p0, const
     const bool table = l == 0 && fast_table_ && ncol == 1 && (code || fold);
     if (!table)
       lin(L.wqkv, nullptr, EPI_STORE, ncol, fh_, s.dim, L.attn_norm, s.fast_eps, fqkv_, w, 0, NO_ROW, L.wqkv.out,
-          done, 0, l == 0 ? fold : nullptr);
+          done, &st_->err, 0, l == 0 ? fold : nullptr);
     AttnArgs aa{};
     aa.qkv = fqkv_;
     if (table) {
@@ -960,14 +962,16 @@ void Engine::enqueue_fast_layers(uint32_t nseq, uint32_t cps, uint32_t p0, const
     const uint32_t res_ld = last_only ? cps * s.dim : s.dim;
     aa.warm = warm_for(L.wo, nullptr, fcols, false, 0, warm_fast_);
     HIPC(launch_attention(aa, stream_));
-    lin(L.wo, nullptr, EPI_RESID, fcols, att_in, att_ld, nullptr, 0.0f, res, res_ld, 0, NO_ROW, L.wo.out, done);
+    lin(L.wo, nullptr, EPI_RESID, fcols, att_in, att_ld, nullptr, 0.0f, res, res_ld, 0, NO_ROW, L.wo.out,
+        done, &st_->err);
     // one wave per tile from 8 columns: the Fast-AR weights are re-read every
     // sub-step and this product runs warm (batch 8: 22.3 us against 24.2 us
     // with the two waves that suit the Slow-AR layers; 3-7 columns keep two
     // waves; 2 columns take the GEMV)
     lin(L.w1, &L.w3, EPI_SWIGLU_FAST, fcols, res, res_ld, L.ffn_norm, s.fast_eps, fact_, s.fast_ffn, 0, NO_ROW,
-        L.w1.out, done, fcols >= 8 && (L.w1.out + 15) / 16 >= 512 ? 1u : 0u);
-    lin(L.w2, nullptr, EPI_RESID, fcols, fact_, s.fast_ffn, nullptr, 0.0f, res, res_ld, 0, NO_ROW, L.w2.out, done);
+        L.w1.out, done, &st_->err, fcols >= 8 && (L.w1.out + 15) / 16 >= 512 ? 1u : 0u);
+    lin(L.w2, nullptr, EPI_RESID, fcols, fact_, s.fast_ffn, nullptr, 0.0f, res, res_ld, 0, NO_ROW, L.w2.out,
+        done, &st_->err);
   }
 }
 
@@ -1000,7 +1004,7 @@ void Engine::enqueue_fast_frame(const SamplerCfg& cfg, uint32_t nseq, const uint
     enqueue_fast_layers(nseq, cps, p0, done, gf.logits ? &gf : nullptr, code);
     // the last position of each slot: rows cps - 1, 2 cps - 1, ...
     lin(fast_out_, nullptr, EPI_STORE, nseq, fh_ + size_t(cps - 1) * s.dim, cps * s.dim, fast_norm_, s.fast_eps,
-        flogits_, s.codebook_size, 0, NO_ROW, s.codebook_size, done);
+        flogits_, s.codebook_size, 0, NO_ROW, s.codebook_size, done, &st_->err);
     p0 += cps;
     cps = 1;
     if (fold && cb + 1 < s.num_codebooks) {
@@ -1121,9 +1125,8 @@ void Engine::mm(const DevLin& L, const DevLin* L3, int epi, const float* x, uint
 // tokens); S2HIP_PREFILL_GEMV=1 selects it, for comparisons.
 void Engine::mm_skinny(const DevLin& L, const DevLin* L3, int epi, const float* x, uint32_t ldx, const float* norm,
                        float eps, uint32_t n, float* y, uint32_t ldy, uint32_t row_base, uint32_t extra_row,
-                       uint32_t out_rows, const uint32_t* done) {
-  HIPC(launch_split_rows(x, ldx, norm, eps, n, 16, L.in, pxh_, pxl_, prs_,
-                         lin_err_ ? lin_err_ : &st_->err, stream_));
+                       uint32_t out_rows, const uint32_t* done, uint32_t* err) {
+  HIPC(launch_split_rows(x, ldx, norm, eps, n, 16, L.in, pxh_, pxl_, prs_, err, stream_));
   SkinnyArgs g{};
   g.w = L.w;
   g.w3 = L3 ? L3->w : nullptr;
@@ -1486,9 +1489,7 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
     HIPC(hipMemsetAsync(&st_[slot].err, 0, sizeof(uint32_t), stream_));
     if (few || prefill_gemv_) {
       const FlagScope off(bmm_off_, gemvs);
-      lin_err_ = &st_[slot].err;
       enqueue_prefill_gemv(prompt_dev_, n_tok, slot);
-      lin_err_ = nullptr;
     } else {
       enqueue_prefill(prompt_dev_, &n_tok, 1, slot);
     }
@@ -1855,7 +1856,7 @@ void Engine::ensure_fast_table() {
   // the same one-column call a sub-step makes (enqueue_fast_layers, layer 0)
   for (uint32_t c = 0; c < s.codebook_size; ++c)
     lin(L, nullptr, EPI_STORE, 1, x.as<float>() + size_t(c) * s.dim, s.dim, fast_[0].attn_norm, s.fast_eps,
-        tab + size_t(c) * w, w, 0, NO_ROW, L.out, nullptr);
+        tab + size_t(c) * w, w, 0, NO_ROW, L.out, nullptr, &st_->err);
   HIPC(hipStreamSynchronize(stream_));
   fast_table_ = tab;
 }
@@ -1912,7 +1913,7 @@ void Engine::op_linear(const void* w, uint32_t type, size_t in, size_t out, cons
   }
   if (ncol >= 3 && ncol <= 16 && in % 256 == 0)  // the whole-row-scale product
     mm_skinny(L, nullptr, EPI_STORE, dx.as<float>(), uint32_t(in), nullptr, 0.0f, uint32_t(ncol), dy.as<float>(),
-              uint32_t(out), 0, NO_ROW, uint32_t(out), nullptr);
+              uint32_t(out), 0, NO_ROW, uint32_t(out), nullptr, &st_->err);
   else
     gemv(L, nullptr, EPI_STORE, uint32_t(ncol), dx.as<float>(), uint32_t(in), nullptr, 0.0f, dy.as<float>(),
          uint32_t(out), 0, NO_ROW, uint32_t(out), nullptr);
@@ -2216,14 +2217,14 @@ void Engine::time_kernel(const std::string& full_name, uint32_t reps, double* av
                   float eps, float* y, uint32_t ldy) {
     if (force == 's') {
       if (L.in % 256) fail("skinny product needs in % 256 == 0");
-      mm_skinny(L, L3, epi, x, ldx, norm, eps, ncol, y, ldy, 0, NO_ROW, L.out, nullptr);
+      mm_skinny(L, L3, epi, x, ldx, norm, eps, ncol, y, ldy, 0, NO_ROW, L.out, nullptr, &st_->err);
     } else if (force == 'g') {
       gemv(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, 0, NO_ROW, L.out, nullptr);
     } else if (force == 't') {
       if (!L.wt || L.in % 256) fail("no batched-product copy of this matrix (in % 256 == 0 only)");
       bmm(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, nullptr, &st_->err, waves);
     } else {
-      lin(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, 0, NO_ROW, L.out, nullptr);
+      lin(L, L3, epi, ncol, x, ldx, norm, eps, y, ldy, 0, NO_ROW, L.out, nullptr, &st_->err);
     }
   };
   const uint32_t q = s.heads * s.head_dim, kv = s.kv_heads * s.head_dim;

@@ -127,3 +127,26 @@ def test_non_finite_activations_are_answered_alike_at_every_length(model_dir, tm
             else:
                 with pytest.raises(S2HipError, match="not finite"):
                     e.eval(make_prompt(SHAPE, n, seed=n))
+
+
+def test_a_failed_call_on_another_slot_leaves_range_errors_where_they_are_read(model_dir, tmp_path, monkeypatch):
+    """More heads than the decode attention takes, and prompts forced through it:
+    eval on slot 3 fails while it launches.  fast_codebooks then still sees that its
+    outlier channel is beyond the batched product's range, and runs again."""
+    from s2hip import Engine, S2HipError
+
+    shape = SHAPE.with_(name="w1024h256", heads=256, kv_heads=64)
+    path = str(tmp_path / "outlier.gguf")
+    shutil.copyfile(synth.ensure_gguf(shape, model_dir), path)
+    for l in range(shape.fast_layers):
+        for w in ("w1", "w3"):
+            gguf_util.scale_rows(path, f"fast_layers.{l}.feed_forward.{w}.weight", [300], 1000.0)
+    o = O.OracleModel(path, 64, shape.im_end_id)
+    hidden, _ = _inputs(3)
+    monkeypatch.setenv("S2HIP_PREFILL_GEMV", "1")
+    with Engine(path, 64, shape.im_end_id) as e:
+        with pytest.raises(S2HipError, match="launch_attention"):
+            e.eval_slot(3, make_prompt(shape, 5, seed=3))
+        got = e.fast_codebooks(hidden, 7)
+        want = o.fast_codebooks(hidden, 7, 0.0, 1.0, 0, 0)
+        assert np.array_equal(got[0], want[0])
