@@ -22,6 +22,7 @@
 #include <memory>
 #include <stdexcept>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "expf_glibc.h"
@@ -173,11 +174,13 @@ class Engine {
   template <class T>
   T* dalloc(size_t count, size_t pad = 0) {
     void* p = nullptr;
-    HIPC(hipMalloc(&p, count * sizeof(T) + pad));
-    count_device_alloc();
-    allocs_.push_back(p);
+    hipError_t e = device_alloc(&p, count * sizeof(T) + pad);
+    if (e == hipErrorOutOfMemory && drop_tiled()) e = device_alloc(&p, count * sizeof(T) + pad);
+    hip_check(e, "hipMalloc");
     return static_cast<T*>(p);
   }
+  hipError_t device_alloc(void** p, size_t bytes);
+  void dfree(void* p);
   void upload(void* dst, const void* src, size_t bytes);
   DevLin load_lin(const GgufFile& g, const std::string& name, uint64_t in, uint64_t out);
   float* load_norm(const GgufFile& g, const std::string& name, uint64_t n);
@@ -211,6 +214,9 @@ class Engine {
   void enqueue_prefill_gemv(const int32_t* prompt_dev, size_t n_tok, uint32_t seq);
   void ensure_slots(uint32_t n);
   void ensure_tiled();
+  bool drop_tiled();
+  template <class F>
+  void each_linear(F f);
   void ensure_repacked();
   void repack(DevLin& L);
   void tile(DevLin& L, uint32_t rows, uint32_t row_base, uint32_t extra_row);
@@ -235,7 +241,8 @@ class Engine {
   void check_state_err(uint32_t nseq = 1);
 
   hipStream_t stream_ = nullptr;
-  std::vector<void*> allocs_;
+  std::unordered_map<void*, size_t> allocs_;  // device allocations and their bytes
+  size_t alloc_bytes_ = 0, alloc_limit_ = SIZE_MAX;
   uint8_t* scratch_dev_ = nullptr;  // this device's `scratch` (hipGetSymbolAddress at set-up)
   // S2HIP_FLAG_PROFILE: events between the Slow-AR kernel groups of one frame
   // (booked after each frame into slow_prof)
@@ -308,7 +315,7 @@ class Engine {
   float *kc_ = nullptr, *vc_ = nullptr;
   size_t slot_kv_ = 0, fslot_kv_ = 0;  // floats per slot in the slow / fast caches
   uint32_t kv_slots_ = 0;
-  uint64_t kv_gen_ = 0;  // bumped whenever the caches are reallocated
+  uint64_t kv_gen_ = 0;  // bumped whenever the caches are reallocated (or the tiled copies dropped)
   float2 *rope_slow_ = nullptr, *rope_fast_ = nullptr;
   uint32_t attn_chunks_ = 1;
   uint32_t attn_mode_ = ATTN_SPLIT;
@@ -499,8 +506,11 @@ Engine::Engine(const s2hip_config& cfg) {
   fast_table_off_ = getenv("S2HIP_NO_FAST_TABLE") != nullptr;
   prefill_gemv_ = getenv("S2HIP_PREFILL_GEMV") != nullptr;
   attn_chunks_ = attention_chunks(s.max_seq_len, attn_mode_);
-  // S2HIP_BMM_MIN_COLS=n: F16 linears over >= n columns use the batched MFMA
-  // product (0 disables it)
+  // S2HIP_DEVICE_BYTES=n: the engine holds at most n bytes of device memory; an
+  // allocation beyond fails as out of memory (what it holds by now stays)
+  if (const char* v = getenv("S2HIP_DEVICE_BYTES")) alloc_limit_ = std::max<size_t>(strtoull(v, nullptr, 10), alloc_bytes_);
+  // S2HIP_BMM_MIN_COLS=n: linears over >= n columns use the batched MFMA product
+  // (0: the copies that it and the prefill products read are never made)
   if (const char* v = getenv("S2HIP_BMM_MIN_COLS")) bmm_min_cols_ = uint32_t(strtoul(v, nullptr, 10));
   // S2HIP_L2_WARM=blocks[,depth[,slow%[,fast%[,step%]]]]: the warming blocks
   // that decode attention, the step embedding and the Fast-AR sampler carry
@@ -579,7 +589,7 @@ Engine::~Engine() {
   for (hipEvent_t e : prof_ev_) (void)hipEventDestroy(e);
   if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
   if (graph_) (void)hipGraphDestroy(graph_);
-  for (void* p : allocs_) (void)hipFree(p);
+  for (const auto& a : allocs_) (void)hipFree(a.first);
   for (int i = 0; i < 2; ++i) {
     if (staging_[i]) (void)hipHostFree(staging_[i]);
     if (staging_ev_[i]) (void)hipEventDestroy(staging_ev_[i]);
@@ -1292,22 +1302,26 @@ void Engine::ensure_prompt(size_t n_int) {
   if (n_int <= prompt_cap_) return;
   if (prompt_dev_) {
     HIPC(hipStreamSynchronize(stream_));
-    HIPC(hipFree(prompt_dev_));
-    allocs_.erase(std::find(allocs_.begin(), allocs_.end(), static_cast<void*>(prompt_dev_)));
+    dfree(prompt_dev_);
+    prompt_dev_ = nullptr;
+    prompt_cap_ = 0;
   }
-  prompt_cap_ = std::max<size_t>(n_int, 4096);
-  prompt_dev_ = dalloc<int32_t>(prompt_cap_);
+  const size_t cap = std::max<size_t>(n_int, 4096);
+  prompt_dev_ = dalloc<int32_t>(cap);
+  prompt_cap_ = cap;
 }
 
 void Engine::ensure_codes(size_t n_int) {
   if (n_int <= codes_cap_ && codes_dev_) return;
   if (codes_dev_) {
     HIPC(hipStreamSynchronize(stream_));
-    HIPC(hipFree(codes_dev_));
-    allocs_.erase(std::find(allocs_.begin(), allocs_.end(), static_cast<void*>(codes_dev_)));
+    dfree(codes_dev_);
+    codes_dev_ = nullptr;
+    codes_cap_ = 0;
   }
-  codes_cap_ = std::max<size_t>(n_int, 16 * 1024);
-  codes_dev_ = dalloc<int32_t>(codes_cap_);
+  const size_t cap = std::max<size_t>(n_int, 16 * 1024);
+  codes_dev_ = dalloc<int32_t>(cap);
+  codes_cap_ = cap;
 }
 
 void Engine::ensure_slots(uint32_t n) {
@@ -1323,15 +1337,14 @@ void Engine::ensure_slots(uint32_t n) {
     HIPC(hipMemset(nb, 0, kv_bytes));
     if (*p) {
       HIPC(hipMemcpy(nb, *p, old_bytes, hipMemcpyDeviceToDevice));
-      HIPC(hipFree(*p));
-      allocs_.erase(std::find(allocs_.begin(), allocs_.end(), static_cast<void*>(*p)));
+      dfree(*p);
     }
     *p = nb;
   }
   for (float** p : {&fkc_, &fvc_}) {
     if (*p) {
-      HIPC(hipFree(*p));
-      allocs_.erase(std::find(allocs_.begin(), allocs_.end(), static_cast<void*>(*p)));
+      dfree(*p);
+      *p = nullptr;
     }
     *p = dalloc<float>(size_t(n) * fslot_kv_);
     HIPC(hipMemset(*p, 0, size_t(n) * fslot_kv_ * 4));
@@ -1369,43 +1382,83 @@ void Engine::tile(DevLin& L, uint32_t rows, uint32_t row_base, uint32_t extra_ro
   L.wt = w;
 }
 
-// Device memory for a copy that only speeds later calls up: null when there is
-// none left (the products then read the rows themselves).
-uint8_t* Engine::try_dalloc(size_t bytes) {
-  void* p = nullptr;
-  if (hipMalloc(&p, bytes) != hipSuccess) {
+hipError_t Engine::device_alloc(void** p, size_t bytes) {
+  const hipError_t e = bytes > alloc_limit_ - alloc_bytes_ ? hipErrorOutOfMemory : hipMalloc(p, bytes);
+  if (e != hipSuccess) {
     (void)hipGetLastError();
-    return nullptr;
+    return e;
   }
   count_device_alloc();
-  allocs_.push_back(p);
+  allocs_.emplace(*p, bytes);
+  alloc_bytes_ += bytes;
+  return e;
+}
+
+void Engine::dfree(void* p) {
+  const auto it = allocs_.find(p);
+  alloc_bytes_ -= it->second;
+  allocs_.erase(it);
+  HIPC(hipFree(p));
+}
+
+template <class F>
+void Engine::each_linear(F f) {
+  for (auto& L : slow_)
+    for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) f(*d);
+  for (auto& L : fast_)
+    for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) f(*d);
+  f(fast_out_);
+}
+
+// Device memory for a copy that only speeds later calls up: null when that would
+// leave less than COPY_RESERVE to the device's other users (the products then
+// read the rows themselves).
+constexpr size_t COPY_RESERVE = size_t(1) << 30;
+uint8_t* Engine::try_dalloc(size_t bytes) {
+  size_t free_bytes = 0, total = 0;
+  HIPC(hipMemGetInfo(&free_bytes, &total));
+  void* p = nullptr;
+  if (free_bytes < bytes + COPY_RESERVE || device_alloc(&p, bytes) != hipSuccess) return nullptr;
   return static_cast<uint8_t*>(p);
 }
 
 // The batched and prefill products' copies of the linears (one more HBM copy
-// of the weights), built once, the first time a call needs them.
+// of the weights), built once, the first time a call needs them.  They come after
+// everything that the call cannot do without, and leave again when a later
+// allocation finds no memory (drop_tiled).
 void Engine::ensure_tiled() {
   if (tiled_) return;
   if (bmm_min_cols_) {
-    for (auto& L : slow_)
-      for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) tile(*d, d->out, 0, NO_ROW);
-    for (auto& L : fast_)
-      for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) tile(*d, d->out, 0, NO_ROW);
-    tile(fast_out_, fast_out_.out, 0, NO_ROW);
+    each_linear([&](DevLin& L) { tile(L, L.out, 0, NO_ROW); });
     tile(head_cand_, n_cand_, spec.semantic_begin, head_extra_);
     HIPC(hipStreamSynchronize(stream_));
   }
   tiled_ = true;
 }
 
+// Gives the copies' memory back, for good; false if there are none.  A captured
+// frame reads them.
+bool Engine::drop_tiled() {
+  bool any = false;
+  HIPC(hipStreamSynchronize(stream_));
+  const auto drop = [&](DevLin& L) {
+    if (!L.wt) return;
+    dfree(L.wt);
+    L.wt = nullptr;
+    L.ws = nullptr;
+    any = true;
+  };
+  each_linear(drop);
+  drop(head_cand_);
+  tiled_ = true;
+  if (any) ++kv_gen_;
+  return any;
+}
+
 // The Q8_0 / Q4_0 linears repacked for the one-column decode GEMV, likewise.
 void Engine::ensure_repacked() {
   if (repacked_) return;
-  for (auto& L : slow_)
-    for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) repack(*d);
-  for (auto& L : fast_)
-    for (DevLin* d : {&L.wqkv, &L.wo, &L.w1, &L.w2, &L.w3}) repack(*d);
-  repack(fast_out_);
+  each_linear([&](DevLin& L) { repack(L); });
   HIPC(hipStreamSynchronize(stream_));
   repacked_ = true;
 }
@@ -1479,8 +1532,8 @@ void Engine::eval(const int32_t* flat, size_t n_tok, float* hidden_out, float* l
   bool few = n_tok <= PREFILL_COLS && decode_takes_shape();
   const bool gemvs = n_tok <= 2;
   if (few) ensure_repacked();
-  if (!few || !gemvs) ensure_tiled();
   ensure_prompt(n_tok * cdim);
+  if (!few || !gemvs) ensure_tiled();
   HIPC(hipMemcpyAsync(prompt_dev_, flat, n_tok * cdim * 4, hipMemcpyHostToDevice, stream_));
   uint32_t e = 0;
   for (;;) {
@@ -1625,11 +1678,11 @@ void Engine::generate(uint32_t nseq, const int32_t* const* prompts, const size_t
   const SamplerCfg cfg{p.temperature, p.top_p, p.top_k};
   const size_t ncodes = size_t(s.num_codebooks) * p.max_new_tokens;
   ensure_slots(nseq);
-  ensure_tiled();
   ensure_repacked();
   ensure_fast_table();
   ensure_codes(ncodes * nseq);
   ensure_prompt(total_cols * cdim);
+  ensure_tiled();
   HIPC(hipStreamSynchronize(stream_));
   // SlowArState::reset + sampler state, per slot
   for (uint32_t b = 0; b < nseq; ++b) {
@@ -1850,14 +1903,15 @@ void Engine::ensure_fast_table() {
   const DevLin& L = fast_[0].wqkv;
   const uint32_t w = (s.fast_heads + 2 * s.fast_kv_heads) * s.fast_head_dim;
   float* tab = dalloc<float>(size_t(s.codebook_size) * w);
-  TmpBuf x(size_t(s.codebook_size) * s.dim * 4);
+  float* x = dalloc<float>(size_t(s.codebook_size) * s.dim);
   HIPC(launch_dequant_rows(W_F16, reinterpret_cast<const uint8_t*>(fast_emb_), size_t(s.dim) * 2, s.codebook_size,
-                           s.dim, x.as<float>(), stream_));
+                           s.dim, x, stream_));
   // the same one-column call a sub-step makes (enqueue_fast_layers, layer 0)
   for (uint32_t c = 0; c < s.codebook_size; ++c)
-    lin(L, nullptr, EPI_STORE, 1, x.as<float>() + size_t(c) * s.dim, s.dim, fast_[0].attn_norm, s.fast_eps,
+    lin(L, nullptr, EPI_STORE, 1, x + size_t(c) * s.dim, s.dim, fast_[0].attn_norm, s.fast_eps,
         tab + size_t(c) * w, w, 0, NO_ROW, L.out, nullptr, &st_->err);
   HIPC(hipStreamSynchronize(stream_));
+  dfree(x);
   fast_table_ = tab;
 }
 
