@@ -221,11 +221,13 @@ class CodecEngine {
     return static_cast<T*>(p);
   }
   // an f16 activation plane of n elements, between its zero guard and its tail
-  // (both sized for the widest plane, so that any channel count finds them)
+  // (both sized for the widest plane, so that any channel count finds them); the
+  // guard is cleared on the codec's stream, ahead of the convolutions that read it
+  // (the null stream does not order itself with a non-blocking one)
   _Float16* plane(size_t n) {
     const size_t guard = size_t(ACT_GUARD) * EXP, tail = size_t(ACT_TAIL) * EXP;
     _Float16* p = dalloc<_Float16>(guard + n + tail);
-    CHK(hipMemset(p, 0, guard * sizeof(_Float16)));
+    CHK(hipMemsetAsync(p, 0, guard * sizeof(_Float16), stream_));
     return p + guard;
   }
   template <class T>

@@ -150,6 +150,16 @@ def test_decode_waveform_matches_oracle(codec, oracle):
     assert np.all(np.abs(res.samples) <= 1.0)
 
 
+def test_first_call_of_a_new_codec_equals_a_later_one(codec_gguf):
+    """The causal padding is cleared when the codec opens, ahead of its first call."""
+    rng = np.random.default_rng(51)
+    hid = rng.standard_normal((3, 1024)).astype(np.float32)
+    with Codec(codec_gguf, max_frames=16, device=0) as c:
+        first = c.decoder(hid)
+        c.decoder(rng.standard_normal((64, 1024)).astype(np.float32))
+        np.testing.assert_array_equal(c.decoder(hid), first)
+
+
 class _DeviceBuffer:
     """Device memory through the HIP runtime the library itself uses
     (libamdhip64, already loaded in the process by libs2hip.so)."""
