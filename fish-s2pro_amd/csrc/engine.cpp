@@ -1329,14 +1329,16 @@ void Engine::ensure_slots(uint32_t n) {
   HIPC(hipStreamSynchronize(stream_));
   // the Slow-AR caches grow with the existing slots' contents kept (slot-major
   // layout: the old buffer is a prefix of the new one); the Fast-AR caches are
-  // per-frame scratch
+  // per-frame scratch.  Fills and copies go to the engine's stream, which the null
+  // stream does not order itself with.
   const size_t eb = kv_f16_ ? 2 : 4;
   const size_t old_bytes = size_t(kv_slots_) * slot_kv_ * eb, kv_bytes = size_t(n) * slot_kv_ * eb;
   for (float** p : {&kc_, &vc_}) {
     float* nb = dalloc<float>((kv_bytes + 3) / 4);
-    HIPC(hipMemset(nb, 0, kv_bytes));
+    HIPC(hipMemsetAsync(nb, 0, kv_bytes, stream_));
     if (*p) {
-      HIPC(hipMemcpy(nb, *p, old_bytes, hipMemcpyDeviceToDevice));
+      HIPC(hipMemcpyAsync(nb, *p, old_bytes, hipMemcpyDeviceToDevice, stream_));
+      HIPC(hipStreamSynchronize(stream_));
       dfree(*p);
     }
     *p = nb;
@@ -1347,7 +1349,7 @@ void Engine::ensure_slots(uint32_t n) {
       *p = nullptr;
     }
     *p = dalloc<float>(size_t(n) * fslot_kv_);
-    HIPC(hipMemset(*p, 0, size_t(n) * fslot_kv_ * 4));
+    HIPC(hipMemsetAsync(*p, 0, size_t(n) * fslot_kv_ * 4, stream_));
   }
   kv_slots_ = n;
   ++kv_gen_;
