@@ -187,7 +187,7 @@ def test_transpose_to_time_major_matches_reference_kat_and_oracle():
 
 
 def test_codec_snake_routine_matches_glibc_snake():
-    """The device snake (sin^2 by Cody-Waite reduction + minimax polynomials,
+    """The device snake (sin^2 by Cody-Waite reduction + a fitted polynomial,
     csrc/sin_cw.h), built for the host, against the oracle's snake (glibc
     sinf, snake_activation_frame_major codec.rs:2162-2186): mostly the same
     bits, never more than 4 ulp of the larger of x and sin^2(a x) / a."""
@@ -204,3 +204,17 @@ def test_codec_snake_routine_matches_glibc_snake():
     err = np.abs(y.astype(np.float64) - ref) / np.spacing(scale)
     assert np.max(err) <= 4.0, np.max(err)
     assert np.mean(y == ref) > 0.98
+
+
+def test_codec_sine_squared_against_64_bits():
+    """sin^2 by itself: with alpha = 2^-20 and x = 2^20 u the snake is 2^20 (u + sin^2 u),
+    and for u in [-pi/2, -1] the sum (within a factor of two of both terms) is exact, so
+    y / 2^20 - u is the routine's sin^2 u.  z = u^2 is largest there, and so is the error:
+    below 1.6e-7, the half ulps of the result (3e-8), of Q times z (5.8e-8), of the inner
+    sum (2e-8) and of z (2.7e-8) and the polynomial's 2e-8."""
+    L = _lib.load()
+    u = -np.arange(np.float32(1.0).view(np.uint32), np.float32(np.pi / 2).view(np.uint32), dtype=np.uint32).view(np.float32)
+    x, a, y = u * np.float32(2.0 ** 20), np.full(u.size, 2.0 ** -20, np.float32), np.empty_like(u)
+    L.s2hip_codec_snake_host(x.ctypes.data, x.size, a.ctypes.data, y.ctypes.data)
+    err = np.abs(y.astype(np.float64) * 2.0 ** -20 - u - np.sin(u.astype(np.float64)) ** 2)
+    assert np.max(err) < 1.6e-7 and np.sqrt(np.mean(err ** 2)) < 5e-8, (np.max(err), np.sqrt(np.mean(err ** 2)))
