@@ -192,3 +192,17 @@ def test_batch_with_large_norm_gains_matches_oracle(model_dir):
         got = rb["requests"][b]
         assert got["n_frames"] == ro["n_frames"] == 12
         assert np.array_equal(got["codes"], ro["codes"]), b
+
+
+def test_batched_product_times_with_every_number_of_waves(tiny_gguf):
+    """s2hip_time_kernel's "_t<N>w<W>": 1, 2 or 4 waves per 16-row tile, and 8 for up to
+    8 columns."""
+    from s2hip import Engine, S2HipError
+
+    with Engine(tiny_gguf, 64, synth.TINY.im_end_id) as e:
+        for cols, waves in ((8, 1), (8, 2), (8, 4), (8, 8), (16, 1), (16, 2), (16, 4)):
+            us, nbytes = e.time_kernel(f"slow_w13_t{cols}w{waves}", 1)
+            assert us > 0 and nbytes > 0
+        for name in ("slow_w13_t16w8", "slow_w13_t8w3"):
+            with pytest.raises(S2HipError, match="invalid argument"):
+                e.time_kernel(name, 1)
