@@ -181,11 +181,22 @@ __global__ __launch_bounds__(256, 2) void conv_gemm_kernel(ConvGemmArgs a, uint3
 #pragma unroll
     for (int j = 0; j < MC; ++j) f.w[j] = *reinterpret_cast<const half8*>(pw + j * 2048);
   };
-  floatx16 acc[FC][MC];
+  // 32-frame waves have the registers for sums in two levels: every FL stages (16 to
+  // 28 roundings) acc goes into sum and starts again from zero.  They serve the
+  // launches of few blocks, where 256-frame tiles split the input channels up to 8
+  // ways and so kept every running sum short; these tiles split less, and the
+  // entry conv of 700 frames was 2.7e-7 off 64 bits instead of 2.0e-7 (with this
+  // 1.5e-7, for 1 to 2 % of a decode of up to 260 code frames).
+  constexpr bool TWO = FC == 1;
+  constexpr int FL = G == 1 ? 4 : 2;
+  floatx16 acc[FC][MC], sum[TWO ? FC : 1][TWO ? MC : 1];
 #pragma unroll
   for (int i = 0; i < FC; ++i)
 #pragma unroll
-    for (int j = 0; j < MC; ++j) acc[i][j] = floatx16{};
+    for (int j = 0; j < MC; ++j) {
+      acc[i][j] = floatx16{};
+      if constexpr (TWO) sum[i][j] = floatx16{};
+    }
   auto mma = [&](const Frags& f) {
 #pragma unroll
     for (int p = 0; p < PL; ++p)
@@ -254,6 +265,23 @@ __global__ __launch_bounds__(256, 2) void conv_gemm_kernel(ConvGemmArgs a, uint3
       mma(fb);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (TWO) {
+      if ((st + 1) % FL == 0) {
+#pragma unroll
+        for (int i = 0; i < FC; ++i)
+#pragma unroll
+          for (int j = 0; j < MC; ++j) {
+            sum[i][j] += acc[i][j];
+            acc[i][j] = floatx16{};
+          }
+      }
+    }
+  }
+  if constexpr (TWO) {
+#pragma unroll
+    for (int i = 0; i < FC; ++i)
+#pragma unroll
+      for (int j = 0; j < MC; ++j) acc[i][j] = sum[i][j] + acc[i][j];
   }
   // the unused tail loads have landed before LDS is used again or the block ends
   __builtin_amdgcn_s_waitcnt(wait_imm(0, true));

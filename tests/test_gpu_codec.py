@@ -285,3 +285,25 @@ def test_decode_waveform_to_wav_passes_the_reference_wav_parity(codec, oracle):
           f"PCM LSB diff max {d.max()} mean {d.mean():.3f}", flush=True)
     assert r.passed, r.failures
     assert d.max() <= 330  # the waveform bound (1e-2) in 16-bit steps
+
+
+@pytest.mark.parametrize("frames", [20, 250, 700, 2060])
+def test_entry_convolution_against_64_bits(codec_gguf, frames):
+    """The first convolution (7168 products per output, f16 inputs and weights, f32
+    sums) against the same in 64 bits, on 96 of its channels.  The error grows with the
+    root of the roundings that one running sum takes: 5.4e-7 for all 448, 2.7e-7 for
+    112, 2.0e-7 for 56; sums of 28 added up give 1.5e-7."""
+    import gguf_util
+
+    w = gguf_util.read_tensors(codec_gguf)
+    ch = np.random.default_rng(61).permutation(1536)[:96]
+    wt = w["decoder.model.0.conv.weight"].reshape(1536, 1024, 7)[ch].astype(np.float64)
+    hid = np.random.default_rng(60).standard_normal((frames, 1024)).astype(np.float32)
+    x = np.concatenate([np.zeros((6, 1024)), hid.astype(np.float16).astype(np.float64)])
+    want = np.tile(w["decoder.model.0.conv.bias"][ch].astype(np.float64), (frames, 1))
+    for t in range(7):
+        want += x[t:t + frames] @ wt[:, :, t].T
+    with Codec(codec_gguf, max_frames=520, device=0) as c:
+        got = c.decoder(hid, 0).reshape(frames, 1536)[:, ch].astype(np.float64)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert err < 1.8e-7, err
