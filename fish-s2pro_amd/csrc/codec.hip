@@ -34,6 +34,7 @@
 
 #include "codec.h"
 #include "expf_glibc.h"
+#include "launch.h"
 #include "wave.h"
 #include "sin_cw.h"
 
@@ -707,9 +708,8 @@ hipError_t conv_gemm_launch(const ConvGemmArgs& a, uint32_t phases, hipStream_t 
   const int32_t tile0 = -((15 - wbase) / 16), shift = wbase - 16 * tile0;
   const uint32_t a_tiles = (uint32_t(shift + (wend - wbase)) + FT + 15u) / 16u;
   if (a_tiles > AT) return hipErrorInvalidValue;
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_gemm_kernel<G, PL, MC, FC, WMG, NB, NA, FU, OS>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  static std::atomic<uint64_t> devices{0};
+  const hipError_t attr = allow_lds(reinterpret_cast<const void*>(&conv_gemm_kernel<G, PL, MC, FC, WMG, NB, NA, FU, OS>), lds, devices);
   if (attr != hipSuccess) return attr;
   const uint32_t m_tiles = (a.M + MT - 1) / MT, f_tiles = (a.F + FT - 1) / FT;
   // K split when the grid would leave CUs idle: each split keeps >= 2 stages

@@ -13,6 +13,7 @@
 
 #include "expf_glibc.h"
 #include "kernels.h"
+#include "launch.h"
 #include "wave.h"
 
 namespace s2 {
@@ -427,13 +428,9 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_kernel(GemvArgs a) {
 template <uint32_t WT, int NCOL, int R, int EPI>
 hipError_t gemv_launch_one(const GemvArgs& a, hipStream_t s) {
   const size_t lds = size_t(NCOL) * a.in * sizeof(float);
-  static bool configured = false;
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_kernel<WT, NCOL, R, EPI>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 1024);
-    if (e != hipSuccess) return e;
-    configured = true;
-  }
+  static std::atomic<uint64_t> devices{0};
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(gemv_kernel<WT, NCOL, R, EPI>), 160 * 1024 - 1024, devices);
+  if (e != hipSuccess) return e;
   const uint32_t rows_per_block = GEMV_WAVES * R;
   const dim3 grid((a.out + rows_per_block - 1) / rows_per_block);
   hipLaunchKernelGGL((gemv_kernel<WT, NCOL, R, EPI>), grid, dim3(GEMV_THREADS), lds, s, a);
@@ -3164,9 +3161,8 @@ __global__ __launch_bounds__(256) void copy_kernel(const float4* __restrict__ sr
 }
 
 template <class K>
-hipError_t set_max_lds(K kernel) {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                             int(sizeof(SampleShared)));
+hipError_t set_max_lds(K kernel, std::atomic<uint64_t>& devices) {
+  return allow_lds(reinterpret_cast<const void*>(kernel), uint32_t(sizeof(SampleShared)), devices);
 }
 
 }  // namespace
@@ -3366,24 +3362,18 @@ hipError_t launch_fast_begin(DevState* st, const float* slow_hidden, const uint1
 }
 
 hipError_t launch_sample_slow(const SampleArgs& a, hipStream_t s) {
-  static bool configured = false;
-  if (!configured) {
-    hipError_t e = set_max_lds(sample_slow_kernel);
-    if (e != hipSuccess) return e;
-    configured = true;
-  }
+  static std::atomic<uint64_t> devices{0};
+  const hipError_t e = set_max_lds(sample_slow_kernel, devices);
+  if (e != hipSuccess) return e;
   if (a.n > SAMPLE_MAX - 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL(sample_slow_kernel, dim3(a.n_seq ? a.n_seq : 1), dim3(SAMPLE_THREADS), sizeof(SampleShared), s, a);
   return hipGetLastError();
 }
 
 hipError_t launch_sample_fast(const SampleArgs& a, hipStream_t s) {
-  static bool configured = false;
-  if (!configured) {
-    hipError_t e = set_max_lds(sample_fast_kernel);
-    if (e != hipSuccess) return e;
-    configured = true;
-  }
+  static std::atomic<uint64_t> devices{0};
+  const hipError_t e = set_max_lds(sample_fast_kernel, devices);
+  if (e != hipSuccess) return e;
   if (a.n > SAMPLE_MAX - 1) return hipErrorInvalidValue;
   hipError_t werr = hipSuccess;
   const uint32_t wblocks = l2_warm_planes(a.warm, 1u, &werr);  // planes of one block
@@ -3395,12 +3385,9 @@ hipError_t launch_sample_fast(const SampleArgs& a, hipStream_t s) {
 
 hipError_t launch_sample_plain(const float* logits, uint32_t n, SamplerCfg cfg, int64_t always_include,
                                uint64_t* rng, uint32_t* token_out, uint32_t* err, hipStream_t s) {
-  static bool configured = false;
-  if (!configured) {
-    hipError_t e = set_max_lds(sample_plain_kernel);
-    if (e != hipSuccess) return e;
-    configured = true;
-  }
+  static std::atomic<uint64_t> devices{0};
+  const hipError_t e = set_max_lds(sample_plain_kernel, devices);
+  if (e != hipSuccess) return e;
   if (n > SAMPLE_MAX - 1 || n == 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(sample_plain_kernel, dim3(1), dim3(SAMPLE_THREADS), sizeof(SampleShared), s, logits, n, cfg,
                      always_include, rng, token_out, err);

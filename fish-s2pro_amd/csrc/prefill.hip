@@ -21,6 +21,7 @@
 
 #include "expf_glibc.h"
 #include "kernels.h"
+#include "launch.h"
 #include "qfrag.h"
 #include "wave.h"
 
@@ -1391,9 +1392,8 @@ static GemmPlan gemm_plan(const GemmArgs& a, bool dual, bool quant) {
 template <int EPI, int TMW, int TNW, int NB>
 static hipError_t gemm_f16_launch(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
   constexpr uint32_t lds = NB * (64 * TMW + 2 * 64 * TNW) * KS * 2;
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f16_dma_kernel<EPI, TMW, TNW, NB>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  static std::atomic<uint64_t> devices{0};
+  const hipError_t attr = allow_lds(reinterpret_cast<const void*>(&gemm_f16_dma_kernel<EPI, TMW, TNW, NB>), lds, devices);
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL((gemm_f16_dma_kernel<EPI, TMW, TNW, NB>), dim3(p.m_tiles * p.n_tiles * p.splits), dim3(256), lds, s,
                      a, p.m_tiles, p.n_tiles, p.splits);
@@ -1402,9 +1402,8 @@ static hipError_t gemm_f16_launch(const GemmArgs& a, const GemmPlan& p, hipStrea
 template <uint32_t WT, int EPI, int TMW, int TNW, int NB>
 static hipError_t gemm_q_launch(const GemmArgs& a, const GemmPlan& p, hipStream_t s) {
   constexpr uint32_t lds = NB * (64 * TMW * (WT == W_Q8_0 ? 32 : 16) + 512 + 2 * 64 * TNW * KS * 2);
-  static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_q_dma_kernel<WT, EPI, TMW, TNW, NB>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  static std::atomic<uint64_t> devices{0};
+  const hipError_t attr = allow_lds(reinterpret_cast<const void*>(&gemm_q_dma_kernel<WT, EPI, TMW, TNW, NB>), lds, devices);
   if (attr != hipSuccess) return attr;
   hipLaunchKernelGGL((gemm_q_dma_kernel<WT, EPI, TMW, TNW, NB>), dim3(p.m_tiles * p.n_tiles * p.splits), dim3(256), lds,
                      s, a, p.m_tiles, p.n_tiles, p.splits);

@@ -150,3 +150,23 @@ def test_a_failed_call_on_another_slot_leaves_range_errors_where_they_are_read(m
         got = e.fast_codebooks(hidden, 7)
         want = o.fast_codebooks(hidden, 7, 0.0, 1.0, 0, 0)
         assert np.array_equal(got[0], want[0])
+
+
+def test_engines_on_two_devices_of_one_process(model_dir):
+    """Prompts, decoding and sampling on a second device after a first: what a kernel
+    was granted on one device (its dynamic LDS) is asked for on the other too."""
+    import ctypes
+
+    from s2hip import Engine
+
+    count = ctypes.c_int(0)
+    ctypes.CDLL("libamdhip64.so").hipGetDeviceCount(ctypes.byref(count))
+    if count.value < 2:
+        pytest.skip("one device")
+    path = synth.ensure_gguf(SHAPE, model_dir)
+    prompt = make_prompt(SHAPE, 70, seed=4)
+    out = []
+    for device in (0, 1):
+        with Engine(path, 128, SHAPE.im_end_id, device=device) as e:
+            out.append((e.eval(prompt)[0], e.generate_codes(prompt, 3, min_tokens_before_end=100)["codes"]))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
