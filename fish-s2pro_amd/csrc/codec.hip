@@ -35,6 +35,7 @@
 #include "codec.h"
 #include "expf_glibc.h"
 #include "launch.h"
+#include "lds_dma.h"
 #include "wave.h"
 #include "sin_cw.h"
 
@@ -75,19 +76,6 @@ __device__ __forceinline__ float gelu_as(float v) {
 // inv = 1 / (guarded alpha), once per channel
 __device__ __forceinline__ float snake(float x, float alpha, float inv) { return snake_cw(x, alpha, inv); }
 
-// s_waitcnt immediate: at most `v` vector memory loads in flight, LDS reads
-// drained if `lgkm0`
-constexpr int wait_imm(int v, bool lgkm0) { return (v & 15) | ((v >> 4) << 14) | 0x70 | (lgkm0 ? 0 : 0xF00); }
-
-// One LDS-DMA load: the KiB at `base` (wave-uniform; lane i its 16 bytes at
-// 16 i) into LDS byte `lds`.  Inline assembly, so that the compiler does not
-// hold every later LDS read for it; the kernel waits itself.
-__device__ __forceinline__ void dma_kib(const uint8_t* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 1\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(lds), "v"(off), "s"(base)
-               : "memory");
-}
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); }
 
 template <int G, int PL, int MC, int FC, int WMG, int NB, int NA, bool FU, int OS>
@@ -156,13 +144,13 @@ __global__ __launch_bounds__(256, 2) void conv_gemm_kernel(ConvGemmArgs a, uint3
 #pragma unroll
     for (int j = 0; j < PW; ++j) {
       const uint32_t q = min(PW * wave + j, MT / 16u - 1u) * 1024u;
-      dma_kib(src + q, off, lds0 + buf + q);
+      dma16(src + q, off, lds0 + buf + q);
     }
   };
   auto issue_a = [&](int32_t st, uint32_t buf) {
     const uint32_t k = uint32_t(min(c0 + st, c1 - 1)) * 1024u;
 #pragma unroll
-    for (int j = 0; j < PA; ++j) dma_kib(asrc[j] + k, off, adst[j] + buf);
+    for (int j = 0; j < PA; ++j) dma16(asrc[j] + k, off, adst[j] + buf);
   };
 
   const uint32_t fr = lane & 31u;

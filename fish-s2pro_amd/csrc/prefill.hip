@@ -22,13 +22,13 @@
 #include "expf_glibc.h"
 #include "kernels.h"
 #include "launch.h"
+#include "lds_dma.h"
 #include "qfrag.h"
 #include "wave.h"
 
 namespace s2 {
 namespace {
 
-constexpr int WAVE = 64;
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
@@ -468,23 +468,6 @@ __global__ __launch_bounds__(256, 3) void gemm_mfma_kernel(GemmArgs a, uint32_t 
 // ---------------------------------------------------------------------------
 constexpr bool DUAL_EPI(int epi) { return epi == EPI_SWIGLU_SLOW || epi == EPI_SWIGLU_FAST; }
 
-// One LDS-DMA load: 16 bytes per lane from `base` (wave-uniform) + `off` into
-// the wave's 1 KiB at LDS byte `lds` (lane i at byte 16 i).  Written as inline
-// assembly so that the compiler does not treat every later LDS read as
-// dependent on it (it would wait for all loads in flight first); the kernel
-// waits for these loads itself (vmcnt) before the barrier that publishes a
-// stage.
-__device__ __forceinline__ void dma16(const uint8_t* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 1\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(lds), "v"(off), "s"(base)
-               : "memory", "m0");
-}
-
-// s_waitcnt immediate: at most `v` vector memory loads in flight, LDS reads
-// drained if `lgkm0`
-constexpr int wait_imm(int v, bool lgkm0) { return (v & 15) | ((v >> 4) << 14) | 0x70 | (lgkm0 ? 0 : 0xF00); }
-
 // Stores of a wave's 32 TMW weight slots x 32 TNW tokens from slot m_base
 // (SwiGLU: output m_base) and token n_base on:
 //   acc[i][j][v] = D[token 8 (v / 4) + 4 (lane / 32) + v % 4][weight slot lane % 32]
@@ -673,15 +656,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f16_dma_kernel(GemmArgs a, uint32
 // over a whole prompt): one rounding per block instead of six.  One barrier per stage; the other
 // block of the CU multiplies while this one reads.
 // ---------------------------------------------------------------------------
-// One LDS-DMA load with an address per lane (W bytes: 16 or 4 per lane).
-template <int W>
-__device__ __forceinline__ void dma_lane(const uint8_t* src, uint32_t lds) {
-  if constexpr (W == 16)
-    asm volatile("s_nop 1\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
-  else
-    asm volatile("s_nop 1\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
-}
-
 template <uint32_t WT, int EPI, int TMW, int TNW, int NB>
 __global__ __launch_bounds__(256, 2) void gemm_q_dma_kernel(GemmArgs a, uint32_t m_tiles, uint32_t n_tiles,
                                                             uint32_t splits) {
