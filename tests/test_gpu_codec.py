@@ -122,11 +122,11 @@ def test_decoder_checkpoints_match_oracle(codec, oracle, frames):
 
 @pytest.mark.parametrize("frames", [1, 16, 33, 129])
 def test_decoder_ragged_lengths_after_a_longer_call(codec, oracle, frames):
-    """Frame counts at the edges of the 16-frame activation tiles and of the
-    128- and 256-frame output tiles, on buffers that a longer decode has left
-    full: what lies past a call's last frame must not reach its outputs.  The
-    first block's checkpoint against the oracle, and all four against the same
-    frames of a longer call (every stage is causal): f16 inputs, as above."""
+    """Frame counts at the edges of the 16-frame activation tiles and of the 64- and
+    128-frame output tiles (32 frames per wave: few blocks), on buffers that a longer
+    decode has left full: what lies past a call's last frame must not reach its
+    outputs.  The first block's checkpoint against the oracle, and all four against the
+    same frames of a longer call (every stage is causal): f16 inputs, as above."""
     rng = np.random.default_rng(50)
     hid = rng.standard_normal((160, 1024)).astype(np.float32)
     full = [codec.decoder(hid, stop) for stop in range(6)]
@@ -307,3 +307,40 @@ def test_entry_convolution_against_64_bits(codec_gguf, frames):
         got = c.decoder(hid, 0).reshape(frames, 1536)[:, ch].astype(np.float64)
     err = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert err < 1.8e-7, err
+
+
+# A launch of 512 blocks or more takes 64 frames per wave (128- or 256-frame tiles):
+# blocks 3 and 4 from 256 latent frames on, block 2 from 512, block 1 from 2048, the
+# entry conv from 8192; the upsampling's pw1 from 2048 of its frames, its other
+# products from 8192 or 16384.
+@pytest.mark.parametrize("frames,stops", [(333, (1, 2, 3, 4, 5)), (700, (1, 2, 3, 4, 5)), (2100, (1, 2, 5)), (8211, (0, 5))])
+def test_decoder_wide_tiles_match_a_short_call(codec_gguf, frames, stops):
+    """A long decode, ragged against the wide tiles, against short ones of pieces of the
+    same input (narrow tiles, oracle-checked above): its last frames, and a piece across
+    the first tile boundary.  The decoder reaches back less than 24 latent frames (6 in
+    the entry conv, then 1 + 78 / 8 in block 1, a fraction of that in the others), so
+    past the first 24 of a piece the two are the same sums in another order."""
+    rng = np.random.default_rng(70)
+    hid = rng.standard_normal((frames, 1024)).astype(np.float32)
+    back = 24
+    with Codec(codec_gguf, max_frames=(frames + 3) // 4, device=0) as c:
+        for stop in stops:
+            full = np.asarray(c.decoder(hid, stop)).reshape(frames, -1)
+            for lo, hi in ((frames - back - 20, frames), (256 - back - 4, 262)):
+                got = np.asarray(c.decoder(hid[lo:hi], stop)).reshape(hi - lo, -1)
+                want = full[lo + back:hi]
+                err = np.max(np.abs(got[back:] - want))
+                assert err <= (1e-2 if stop == 5 else 5e-3 * np.max(np.abs(want))), (stop, lo, err)
+
+
+@pytest.mark.parametrize("frames", [1100, 4093])
+def test_upsample_wide_tiles_match_a_short_call(codec_gguf, frames):
+    """The same for the upsampling (f32-accurate products), which reaches back 6 of its
+    first stage's frames and 6 of its second's: less than 5 code frames."""
+    rng = np.random.default_rng(71)
+    hid = rng.standard_normal((frames, 1024)).astype(np.float32)
+    with Codec(codec_gguf, max_frames=frames, device=0) as c:
+        full = c.upsample(hid).reshape(frames, 4, 1024)
+        for lo, hi in ((frames - 20, frames), (120, 140), (1015, 1035)):
+            got = c.upsample(hid[lo:hi]).reshape(hi - lo, 4, 1024)
+            assert _rel(got[5:], full[lo + 5:hi]) < 1e-5, lo
