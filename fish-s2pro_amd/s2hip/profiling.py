@@ -15,7 +15,10 @@ launch against the algorithmic bytes.
 
 `mfma` averages per-dispatch SQ / GRBM counters (an MFMA counter run) for the
 kernels matching each --kernel and derives MFMA utilisation and f16 MFMA
-flops (SQ_INSTS_VALU_MFMA_MOPS_F16 x 512) per dispatch.
+flops (SQ_INSTS_VALU_MFMA_MOPS_F16 x 512) per dispatch, and from SQ_INSTS_VALU
+and the LDS counters (a second run) the share of cycles in which a SIMD issues
+vector instructions (4 cycles each) and the LDS port is busy or in conflict;
+--grid N keeps the dispatches of N threads.
 
 `tail` averages the durations of the last --count dispatches of one kernel
 in a kernel-trace CSV (e.g. bench.py's timing loop, which runs after the
@@ -33,7 +36,8 @@ in KiB per dispatch) over every dispatch of the kernel matching --kernel, and
 calibrates it against a plain copy kernel of known size: the copy reads and
 writes exactly --copy-bytes / 2 bytes each way, so
     scale = (copy_bytes / 2) / (copy counter * 1024)
-and the kernel's HBM bytes per launch = counter * 1024 * scale.
+and the kernel's HBM bytes per launch = counter * 1024 * scale.  With --last N,
+`counters` and `traffic` average the kernel's last N dispatches only.
 """
 
 import argparse
@@ -76,7 +80,7 @@ def stats(path, top):
     return "\n".join(lines)
 
 
-def counter_mean(rows, kernel_re, counter):
+def counter_mean(rows, kernel_re, counter, last=0):
     pat = re.compile(kernel_re)
     vals = []
     for r in rows:
@@ -86,15 +90,16 @@ def counter_mean(rows, kernel_re, counter):
             vals.append(float(_col(r, "Counter_Value")))
     if not vals:
         raise SystemExit(f"no {counter} samples for kernels matching {kernel_re!r}")
+    vals = vals[-last:]
     return statistics.fmean(vals), len(vals)
 
 
-def counters(path, kernel_re, copy_re, copy_bytes):
+def counters(path, kernel_re, copy_re, copy_bytes, last=0):
     rows = _rows(path)
     names = sorted({_col(r, "Counter_Name") for r in rows})
     lines = []
     for counter in names:
-        k, nk = counter_mean(rows, kernel_re, counter)
+        k, nk = counter_mean(rows, kernel_re, counter, last)
         c, nc = counter_mean(rows, copy_re, counter)
         scale = (copy_bytes / 2) / (c * 1024.0)
         lines.append(f"{counter}: kernel {k:.1f} KiB/dispatch over {nk} dispatches; copy {c:.1f} KiB/dispatch "
@@ -108,17 +113,18 @@ def _scale(rows, counter, copy_re, copy_bytes):
     return (copy_bytes / 2) / (c * 1024.0)
 
 
-def _launch_bytes(rows, counter, kernel_re, grid, scale):
+def _launch_bytes(rows, counter, kernel_re, grid, scale, last):
     pat = re.compile(kernel_re)
     vals = [float(_col(r, "Counter_Value")) for r in rows
             if _col(r, "Counter_Name") == counter and pat.search(_col(r, "Kernel_Name"))
             and (grid == "*" or _col(r, "Grid_Size") == grid)]
     if not vals:
         raise SystemExit(f"no {counter} samples for {kernel_re!r} at grid {grid}")
+    vals = vals[-last:]
     return statistics.fmean(vals) * 1024.0 * scale, len(vals)
 
 
-def traffic(fetch_csv, write_csv, copy_re, copy_bytes, specs):
+def traffic(fetch_csv, write_csv, copy_re, copy_bytes, specs, last=0):
     fr, wr = _rows(fetch_csv), _rows(write_csv)
     fs, ws = _scale(fr, "FETCH_SIZE", copy_re, copy_bytes), _scale(wr, "WRITE_SIZE", copy_re, copy_bytes)
     lines = [f"calibration: FETCH_SIZE x {fs:.4f}, WRITE_SIZE x {ws:.4f} (copy kernel moving "
@@ -127,16 +133,16 @@ def traffic(fetch_csv, write_csv, copy_re, copy_bytes, specs):
              f"{'algo MB':>9s} {'ratio':>6s}"]
     for spec in specs:
         label, kre, grid, algo = spec.split("|")
-        f, n = _launch_bytes(fr, "FETCH_SIZE", kre, grid, fs)
-        w, _ = _launch_bytes(wr, "WRITE_SIZE", kre, grid, ws)
+        f, n = _launch_bytes(fr, "FETCH_SIZE", kre, grid, fs, last)
+        w, _ = _launch_bytes(wr, "WRITE_SIZE", kre, grid, ws, last)
         a = float(algo)
         lines.append(f"{label:34s} {n:8d} {f / 1e6:10.3f} {w / 1e6:9.3f} {(f + w) / 1e6:10.3f} {a / 1e6:9.3f} "
                      f"{(f + w) / a:6.3f}")
     return "\n".join(lines)
 
 
-def mfma(path, kernel_res):
-    rows = _rows(path)
+def mfma(path, kernel_res, grid="*"):
+    rows = [r for r in _rows(path) if grid == "*" or _col(r, "Grid_Size") == grid]
     lines = []
     for kre in kernel_res:
         pat = re.compile(kre)
@@ -150,8 +156,14 @@ def mfma(path, kernel_res):
         n = max(len(v) for v in per.values())
         parts = [f"{k} {v:.0f}" for k, v in sorted(m.items())]
         if "SQ_VALU_MFMA_BUSY_CYCLES" in m and "GRBM_GUI_ACTIVE" in m:
-            # busy cycles summed over the SIMDs (4 per CU, 256 CUs)
-            parts.append(f"MFMA busy {100 * m['SQ_VALU_MFMA_BUSY_CYCLES'] / (m['GRBM_GUI_ACTIVE'] * 1024):.1f} %")
+            # busy cycles summed over the SIMDs (4 per CU, 256 CUs), active cycles over the 8 XCDs
+            parts.append(f"MFMA busy {100 * m['SQ_VALU_MFMA_BUSY_CYCLES'] / (m['GRBM_GUI_ACTIVE'] / 8 * 1024):.1f} %")
+        if "GRBM_GUI_ACTIVE" in m:
+            cycles = m["GRBM_GUI_ACTIVE"] / 8
+            for name, label, per_cycle in (("SQ_INSTS_VALU", "VALU issue", 1024 / 4), ("SQ_LDS_IDX_ACTIVE", "LDS active", 256),
+                                           ("SQ_LDS_BANK_CONFLICT", "LDS conflict", 256)):
+                if name in m:
+                    parts.append(f"{label} {100 * m[name] / (cycles * per_cycle):.1f} %")
         if "SQ_INSTS_VALU_MFMA_MOPS_F16" in m:
             parts.append(f"f16 MFMA {m['SQ_INSTS_VALU_MFMA_MOPS_F16'] * 512 / 1e9:.2f} GFLOP/dispatch")
         lines.append(f"{short_name(kre)} ({n} dispatches): " + "; ".join(parts))
@@ -213,12 +225,14 @@ def main(argv=None):
     b.add_argument("--kernel", required=True)
     b.add_argument("--copy-kernel", required=True)
     b.add_argument("--copy-bytes", type=float, required=True)
+    b.add_argument("--last", type=int, default=0)
     t = sub.add_parser("traffic")
     t.add_argument("fetch_csv")
     t.add_argument("write_csv")
     t.add_argument("--copy-kernel", required=True)
     t.add_argument("--copy-bytes", type=float, required=True)
     t.add_argument("--row", action="append", required=True)
+    t.add_argument("--last", type=int, default=0)
     tl = sub.add_parser("tail")
     tl.add_argument("csv")
     tl.add_argument("--kernel", required=True)
@@ -232,19 +246,21 @@ def main(argv=None):
     m = sub.add_parser("mfma")
     m.add_argument("csv")
     m.add_argument("--kernel", action="append", required=True)
+    m.add_argument("--grid", default="*")
     args = ap.parse_args(argv)
     if args.cmd == "stats":
         print(stats(args.csv, args.top))
     elif args.cmd == "traffic":
-        print(traffic(args.fetch_csv, args.write_csv, args.copy_kernel, args.copy_bytes, args.row))
+        print(traffic(args.fetch_csv, args.write_csv, args.copy_kernel, args.copy_bytes, args.row,
+                      args.last))
     elif args.cmd == "tail":
         print(tail(args.csv, args.kernel, args.count))
     elif args.cmd == "budget":
         print(budget(args.csv, args.after, args.begin, args.frames, args.top))
     elif args.cmd == "mfma":
-        print(mfma(args.csv, args.kernel))
+        print(mfma(args.csv, args.kernel, args.grid))
     else:
-        print(counters(args.csv, args.kernel, args.copy_kernel, args.copy_bytes))
+        print(counters(args.csv, args.kernel, args.copy_kernel, args.copy_bytes, args.last))
 
 
 if __name__ == "__main__":
