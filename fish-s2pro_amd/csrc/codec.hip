@@ -21,14 +21,14 @@
 //   * tiles of one weight tile (m tile) are dealt to the same XCD, so that
 //     XCD's L2 serves its weights to all of its frame tiles.
 // Measured at 2048 latent frames (512 code frames; before: 256-frame tiles of
-// 16-channel stages through registers), us: entry 78 -> 64, transposed convs of
-// blocks 1-4 238 / 448 / 621 / 441 -> 145 / 325 / 385 / 309, k7 convs of blocks
-// 1 and 2 184 / 346 -> 131 / 264, their k1 convs 91 / 232 -> 43 / 150, a residual
-// unit of block 3 (k7 and k1 in one launch now) 856 -> 472, of block 4 548 -> 360;
-// whole decode 10.34 -> 7.20 ms.
-// Small per-frame kernels handle the rest: RVQ lookup, RoPE, the windowed
-// attention of the post-module transformer, depthwise conv + LayerNorm, the
-// output conv + tanh.
+// 16-channel stages through registers), us: entry 78 -> 71, transposed convs of
+// blocks 1-4 238 / 448 / 621 / 441 -> 141 / 313 / 387 / 304, k7 convs of blocks 1
+// and 2 184 / 346 -> 128 / 258, their k1 convs 91 / 232 -> 43 / 152, a residual unit
+// of block 3 (k7 and k1 in one launch now) 856 -> 472, of block 4 548 -> 359;
+// whole decode 10.34 -> 7.02 ms.
+// Small per-frame kernels handle the rest: RVQ lookup, the windowed attention of
+// the post-module transformer (RoPE as it reads q and k), depthwise conv +
+// LayerNorm, the output conv + tanh.
 
 #include <algorithm>
 
@@ -723,9 +723,13 @@ hipError_t conv_gemm_launch(const ConvGemmArgs& a, uint32_t phases, hipStream_t 
 }
 
 // Frames per wave: 64, or 32 where those tiles would leave fewer than two
-// blocks per CU (37 code frames, us: transposed convs 34 / 50 / 43 / 33 -> 30 /
-// 38 / 36 / 26, residual units of blocks 3 and 4 52 / 39 -> 43 / 31; at 512 code
-// frames the 32-frame tiles lose, 376 -> 424 for block 3's transposed conv).
+// blocks per CU (37 code frames, us: transposed convs 34 / 50 / 43 / 33 -> 29 /
+// 38 / 41 / 24, residual units of blocks 3 and 4 52 / 39 -> 42 / 29).  Where the line
+// lies, whole decodes in ms with 64 frames always : from 256 : from 512 : from 1024
+// blocks : never: 37 code frames 1.94 : 1.84 : 1.77 : 1.77 : 1.77, 130 3.31 : 3.25 :
+// 3.26 : 3.11 : 2.93, 180 3.62 : 3.51 : 3.52 : 3.47 : 3.45, 260 4.98 : 4.93 : 4.88 :
+// 4.89 : 4.75, 350 5.75 : 5.68 : 5.67 : 5.69 : 5.72, 512 7.51 : 7.48 : 7.45 : 7.56 :
+// 7.82 (block 3's transposed conv 376 -> 424 us).
 template <int G, int PL, int MC, int WMG, int NB, int NA, bool FU, int OS>
 hipError_t conv_gemm_frames(const ConvGemmArgs& a, uint32_t phases, hipStream_t s) {
   constexpr uint32_t MT = 32 * MC * WMG, FT = 64 * (4 / WMG);

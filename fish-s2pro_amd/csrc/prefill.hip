@@ -1327,9 +1327,17 @@ constexpr int GEMM_DEPTH = 2;
 // other's unpacking: rounds of 768 blocks of 128 x 64 (Q8_0, 389 tokens: wqkv
 // 76 -> 45 us against both tiles over rounds of 256, w2 and wo together 105 ->
 // 96; Q4_0, 150 tokens: w1/w3 82 -> 59, wqkv 43 -> 24).
-// Long rows are split at least so often that no running sum gets longer than
-// it was before these tiles: 2560 wide with the lo products apart (64-token
-// tiles), 1280 where they share the accumulator, at most four.
+// The line between the small and the wide tiles, whole prompts in ms, small : wide:
+// F16 640 tokens 15.7 : 15.9, 768 18.3 : 18.6, 832 20.1 : 20.0, 1024 23.9 : 23.6, 1500
+// 36.3 : 33.7; Q8_0 512 14.5 : 15.8, 768 21.5 : 21.1, 1024 26.7 : 27.6, 1500 40.2 :
+// 39.3, 2048 53.6 : 53.7; Q4_0 512 14.2 : 14.9, 768 21.9 : 21.0, 1024 26.6 : 27.0, 1500
+// 40.5 : 38.0, 2048 53.6 : 51.4.  One line serves the three types: the quantized ones
+// lose up to 6 % between 800 and 1024 tokens and gain 2 to 6 % at 1500.
+// Long rows prefer so many splits that a running sum stays within 2560 k where the lo
+// products are apart (64-token tiles) and within 1280 where they share the
+// accumulator, at most four; fewer where the workspace or the row's stages end.  SwiGLU
+// pairs are never split: 2560-wide rows of w1/w3 are one running sum, as they were
+// before these tiles, and w2's 9728 up to 2432 a sum.
 constexpr uint32_t GEMM_WIDE_N = 768;
 struct GemmPlan {
   uint32_t tile;  // 0: 128 x 64, 1: 256 x 64, 2: 256 x 128
@@ -1533,9 +1541,10 @@ size_t attn_prefill_part_floats(uint32_t n, uint32_t heads, uint32_t hd) {
 }
 
 // Two query groups per block (8 waves sharing each K / V tile, which halves the
-// tile's conversion and staging per wave) past 256 queries: 1500 tokens 191 ->
-// 147 us, 389 30.3 -> 24.9; 256 tokens leave too few blocks for it (19.7 and
-// 20.3 us, the first layers 14.5 and 19.2).
+// tile's conversion and staging per wave) past 256 queries: 1500 tokens 191 -> 147 us,
+// 389 30.3 -> 24.9.  Up to 256 the whole prompt takes the same with either (128 tokens
+// 6.58 and 6.65 ms, 192 7.17 and 7.17, 256 8.57 and 8.57; from 288 on two groups win,
+// 9.38 -> 9.15), and one group needs no more queries than a short prompt has.
 static bool attn_wide(uint32_t n) { return n > 256u; }
 template <int HD>
 static void attn_prefill_launch(const PrefillAttnArgs& a, uint32_t splits, hipStream_t s) {

@@ -374,9 +374,11 @@ void s2hip_codec_snake_host(const float* x, size_t n, const float* alpha, float*
  * `what` over `reps` launches, after one untimed decode of n_frames frames of
  * fixed codes: "decode" (the whole decode_waveform on device buffers) or one
  * convolution of that decode by name ("entry", "b1_convT" .. "b4_convT",
- * "b<1-4>_r<1-3>_conv0" / "_conv1", "up1_convT", "up1_pw1", "up1_pw2",
- * "up2_..."), relaunched with the same arguments.  flops receives 2 x the
- * multiply-adds of one launch (for "decode": of all its convolutions).
+ * "b<1-3>_r<1-3>_conv0" / "_conv1", "b<3-4>_r<1-3>_unit" (a residual unit in
+ * one launch, as blocks 3 and 4 decode it; block 3's two convolutions can also
+ * be timed apart), "up1_convT", "up1_pw1", "up1_pw2", "up2_..."), relaunched
+ * with the same arguments.  flops receives 2 x the multiply-adds of one launch
+ * (for "decode": of all its convolutions).
  * No counterpart in the reference (a measurement hook). */
 int32_t s2hip_codec_time(s2hip_codec* codec, const char* what, uint32_t n_frames, uint32_t reps, double* avg_us,
                          double* flops, char* err, size_t err_cap);
