@@ -1619,7 +1619,11 @@ void Engine::fast_codebooks(const float* hidden, uint32_t sem, const s2hip_sampl
   *st_host_ = init;
   HIPC(hipMemcpyAsync(st_, st_host_, sizeof(DevState), hipMemcpyHostToDevice, stream_));
   HIPC(hipMemcpyAsync(hn_, hidden, s.dim * 4, hipMemcpyHostToDevice, stream_));
+  // the copies that a generation's frames read, so that a code does not hang on
+  // which call came first
+  ensure_repacked();
   ensure_fast_table();
+  ensure_tiled();
   enqueue_fast_frame(SamplerCfg{smp.temperature, smp.top_p, smp.top_k}, 1, nullptr);
   HIPC(hipMemcpyAsync(st_host_, st_, sizeof(DevState), hipMemcpyDeviceToHost, stream_));
   HIPC(hipStreamSynchronize(stream_));

@@ -170,3 +170,19 @@ def test_engines_on_two_devices_of_one_process(model_dir):
         with Engine(path, 128, SHAPE.im_end_id, device=device) as e:
             out.append((e.eval(prompt)[0], e.generate_codes(prompt, 3, min_tokens_before_end=100)["codes"]))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("weights", sorted(TYPES))
+def test_fast_codebooks_of_a_new_engine_equal_those_of_a_used_one(model_dir, weights):
+    """And both the oracle's: the first call builds what a generation would have."""
+    from s2hip import Engine
+
+    path = synth.ensure_gguf(SHAPE.with_(linear_type=TYPES[weights]), model_dir)
+    o = O.OracleModel(path, 64, SHAPE.im_end_id)
+    inputs = [(_inputs(s)[0], s) for s in range(10, 18)]
+    with Engine(path, 64, SHAPE.im_end_id) as e:
+        cold = [e.fast_codebooks(h, s)[0] for h, s in inputs]
+        e.generate_codes(make_prompt(SHAPE, 7, seed=3), 2, min_tokens_before_end=100)
+        for (h, s), want in zip(inputs, cold):
+            assert np.array_equal(e.fast_codebooks(h, s)[0], want), s
+            assert np.array_equal(want, o.fast_codebooks(h, s, 0.0, 1.0, 0, 0)[0]), s
